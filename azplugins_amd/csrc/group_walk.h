@@ -1,0 +1,483 @@
+// Neighbor search of a group of 32 consecutive cell-list slots by one
+// wavefront, on the matrix cores.
+//
+// The squared distances of 32 candidates to the group's 32 particles are a
+// contraction: with candidates and particles as offsets b, a from an anchor,
+//   |a - b|^2 - r^2 = (|a|^2 - r^2) - 2 a.b + |b|^2 . 1,
+// K = 4 in FP32, i.e. two v_mfma_f32_32x32x2_f32 for 1,024 pairs with the
+// particle's |a|^2 - r^2 as the C operand.  The sign of a result is the hit,
+// so a lane collects 32 candidates of one particle into a 32-bit mask with
+// one v_alignbit each (bit o = candidate o), against about eight
+// instructions and a serial append per pair in a lane-per-particle loop.
+// Pairs whose result lies within the FP32 error bound of the list radius are
+// decided by the FP64 predicate of the host oracle, so the pair set is the
+// FP64 one.
+//
+// Candidates are the members of the union of the particles' 27-cell
+// stencils (cells outside a particle's own stencil lie beyond its list
+// radius and only cost tests).  Cells are visited in ascending geometric index
+// and their members in slot order: every list of every walk has this order.
+// A group whose particles lie in cells far apart (a jump of the Morton
+// curve, several replicas) is served in passes over windows of at most
+// 5 x 5 x 5 own cells.
+#pragma once
+
+#include "cells.h"
+
+namespace azp
+{
+
+// Own cells of one pass lie within kGroupReach of the anchor's on every axis,
+// so their stencils span at most kGroupSpan cells per axis.
+constexpr int kGroupReach = 2;
+constexpr uint32_t kGroupSpan = 2 * kGroupReach + 3;
+constexpr uint32_t kGroupCells = kGroupSpan * kGroupSpan * kGroupSpan;
+// Candidates per segment of a pass (the bits of GroupLds::starts).
+constexpr uint32_t kGroupSegment = 8192;
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// The periodic box and cell grid of one pass (wave-uniform).
+struct GroupGeom
+    {
+    int n[3];
+    double L[3], Linv[3];
+    float scale[3]; // L / 2^32
+    uint32_t cell_base;
+    };
+
+struct GroupArgs
+    {
+    const double4* pos;
+    const uint32_t* members;
+    const uint32_t* start;     // slots of cell rank r: start[r] .. start[r + 1]
+    const uint32_t* cell_rank; // storage rank of each cell; null: cells are stored by index
+    const int4* cell_fixed;    // by slot: wrapped fixed-point position, type (>= ntypes: never listed)
+    const double* r_listsq;
+    uint32_t ntypes;
+    float thr;    // largest r_list^2
+    float r_max;  // largest r_list
+    bool direct;  // no matrix tests (several list radii among more types than ONEHOT serves)
+    };
+
+// One wavefront's LDS.
+struct GroupLds
+    {
+    uint64_t starts[kGroupSegment / 64]; // bit p: a cell's first candidate is number p of the segment
+    uint32_t rows[kGroupSpan * kGroupSpan];
+    uint32_t delta[kGroupCells + 1]; // slot - candidate number of each cell's members
+    uint32_t first[kGroupCells + 1]; // candidate number of each cell's first member
+    uint16_t seq[kGroupCells + 1];   // place of a window cell in the pass's sequence
+    };
+
+// Makes one lane's LDS writes visible to the other lanes of its wavefront.
+__device__ __forceinline__ void wave_lds_fence()
+    {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+
+__device__ __forceinline__ int lane_value(int v, int lane)
+    {
+    return __builtin_amdgcn_readlane(v, lane);
+    }
+
+__device__ __forceinline__ uint32_t wave_exclusive_scan(uint32_t v, uint32_t lane, uint32_t& total)
+    {
+    uint32_t x = v;
+    for (uint32_t off = 1; off < 64; off <<= 1)
+        {
+        const uint32_t y = (uint32_t)__shfl_up((int)x, off);
+        if (lane >= off)
+            x += y;
+        }
+    total = (uint32_t)lane_value((int)x, 63);
+    return x - v;
+    }
+
+// One axis of a pass's window: `len` distinct cells from s0 (periodic).
+struct GroupAxis
+    {
+    int n, s0, len;
+    __device__ GroupAxis(int n_, int anchor, int lo, int hi)
+        {
+        n = n_;
+        const int raw = hi - lo + 3;
+        const bool full = raw >= n;
+        len = full ? n : raw;
+        int s = anchor + lo - 1;
+        s = s < 0 ? s + n : (s >= n ? s - n : s);
+        s0 = full ? 0 : s;
+        }
+    // place of cell c in the window
+    __device__ int index(int c) const
+        {
+        const int k = c - s0;
+        return k < 0 ? k + n : k;
+        }
+    // q-th cell of the window in ascending cell index
+    __device__ int cell(int q) const
+        {
+        const int wrapped = max(0, s0 + len - n);
+        return q < wrapped ? q : s0 + (q - wrapped);
+        }
+    __device__ int step(int c, int d) const
+        {
+        const int x = c + d;
+        return x < 0 ? x + n : (x >= n ? x - n : x);
+        }
+    };
+
+// The particle a lane's column stands for (lanes l and l + 32 share column
+// l & 31).
+struct GroupColumn
+    {
+    bool valid;
+    uint32_t slot, i, cell; // cell: global cell index
+    int c[3];               // cell coordinates in the grid
+    int4 fixed;             // position, type
+    };
+
+// The anchor column of a pass over the columns `todo` (not 0): the middle one.
+__device__ __forceinline__ int group_anchor(uint32_t todo)
+    {
+    const uint32_t first = (uint32_t)__builtin_ctz(todo), last = 31u - (uint32_t)__builtin_clz(todo);
+    return __builtin_ctz(todo >> ((first + last) / 2u) << ((first + last) / 2u));
+    }
+
+// Runs one pass: the columns with `todo` bits whose own cells lie in the
+// window around that of the anchor column `al` (and, by `same`, in its
+// system).  Returns
+// the mask of the columns served.  For every 64 candidates, emit(mask, P,
+// off, which) gets the lane's hits among candidates P + 32 (l >> 5) + bit
+// of its column, and candidate P + off, which this lane read: its particle
+// (MEMBERS; any for a number past the last candidate) or its slot (or ~0).
+// begin(cells, total) runs before the first of them.
+//
+// ONEHOT = 0: one list radius for every type pair (or a.direct).  Otherwise
+// 2 * ONEHOT >= ntypes: K grows by one per type, the candidate's type as a
+// unit vector against the particle's radii.
+template<int ONEHOT, bool MEMBERS, class Begin, class Emit>
+__device__ __forceinline__ uint32_t group_pass(const GroupArgs& a,
+                                               const GroupGeom& G,
+                                               GroupLds& s,
+                                               const GroupColumn& me,
+                                               uint32_t todo,
+                                               int al,
+                                               bool same,
+                                               Begin&& begin,
+                                               Emit&& emit)
+    {
+    const uint32_t lane = threadIdx.x & 63u, h = lane >> 5, col = lane & 31u;
+    int o[3], lo[3], hi[3], anchor[3];
+    bool in = me.valid && same && ((todo >> col) & 1u);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+        {
+        anchor[k] = lane_value(me.c[k], al);
+        o[k] = me.c[k] - anchor[k];
+        o[k] += 2 * o[k] > G.n[k] ? -G.n[k] : (2 * o[k] < -G.n[k] ? G.n[k] : 0);
+        in = in && o[k] >= -kGroupReach && o[k] <= kGroupReach;
+        }
+    // Offsets from the anchor column's position: the difference of two is the
+    // minimum image when the column lies within L/2 - r_list of the anchor on
+    // every axis.  Columns farther away wait for another pass; on grids of
+    // three cells or fewer per axis, where that would leave few columns to a
+    // pass, the group takes the direct tests below.
+    const int fx0 = lane_value(me.fixed.x, al), fy0 = lane_value(me.fixed.y, al), fz0 = lane_value(me.fixed.z, al);
+    const float sx = G.scale[0], sy = G.scale[1], sz = G.scale[2];
+    const float ax = (float)fixed_delta(me.fixed.x, fx0) * sx;
+    const float ay = (float)fixed_delta(me.fixed.y, fy0) * sy;
+    const float az = (float)fixed_delta(me.fixed.z, fz0) * sz;
+    const float margin = a.r_max * 1.0001f;
+    const bool far = !(fabsf(ax) + margin < 0.5f * (float)G.L[0] && fabsf(ay) + margin < 0.5f * (float)G.L[1]
+                       && fabsf(az) + margin < 0.5f * (float)G.L[2]);
+    bool direct = a.direct;
+    if (G.n[0] > 3 && G.n[1] > 3 && G.n[2] > 3)
+        in = in && !far;
+    else
+        direct = direct || __ballot(in && far) != 0ull;
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+        {
+        lo[k] = kGroupReach;
+        hi[k] = -kGroupReach;
+#pragma unroll
+        for (int v = -kGroupReach; v <= kGroupReach; ++v)
+            if (__ballot(in && o[k] == v) != 0ull)
+                {
+                lo[k] = min(lo[k], v);
+                hi[k] = max(hi[k], v);
+                }
+        }
+    const uint32_t served = (uint32_t)__ballot(in);
+    const GroupAxis X(G.n[0], anchor[0], lo[0], hi[0]);
+    const GroupAxis Y(G.n[1], anchor[1], lo[1], hi[1]);
+    const GroupAxis Z(G.n[2], anchor[2], lo[2], hi[2]);
+
+    // the cells of the included columns' stencils, as bits of window rows
+    if (lane < kGroupSpan * kGroupSpan)
+        s.rows[lane] = 0u;
+    wave_lds_fence();
+    // once per cell: by the first of its included columns (slots of a cell are
+    // consecutive)
+    const uint32_t prev = (uint32_t)__shfl_up((int)me.cell, 1);
+    if (in && (col == 0u || prev != me.cell || !((served >> (col - 1u)) & 1u)))
+        {
+        const uint32_t bits = (1u << X.index(X.step(me.c[0], X.n > 1 ? -1 : 0))) | (1u << X.index(me.c[0]))
+                              | (1u << X.index(X.step(me.c[0], X.n > 1 ? 1 : 0)));
+        for (uint32_t q = h; q < 9u; q += 2u)
+            {
+            const int dy = (int)(q % 3u) - 1, dz = (int)(q / 3u) - 1;
+            const int y = Y.index(Y.step(me.c[1], Y.n > 1 ? dy : 0));
+            const int z = Z.index(Z.step(me.c[2], Z.n > 1 ? dz : 0));
+            atomicOr(&s.rows[(uint32_t)z * kGroupSpan + (uint32_t)y], bits);
+            }
+        }
+    wave_lds_fence();
+
+    // their candidate ranges in ascending cell index: one lane per row of x
+    uint32_t st[kGroupSpan], ct[kGroupSpan];
+    uint32_t ncell = 0, ncand = 0;
+    const bool row_lane = lane < (uint32_t)(Y.len * Z.len);
+    const int qz = row_lane ? (int)lane / Y.len : 0, qy = row_lane ? (int)lane % Y.len : 0;
+    const int cz = Z.cell(qz), cy = Y.cell(qy);
+    const uint32_t row = (uint32_t)Z.index(cz) * kGroupSpan + (uint32_t)Y.index(cy);
+    const uint32_t bits = row_lane ? s.rows[row] : 0u;
+#pragma unroll
+    for (uint32_t q = 0; q < kGroupSpan; ++q)
+        {
+        st[q] = ct[q] = 0u;
+        if ((int)q < X.len)
+            {
+            const int cx = X.cell((int)q);
+            if ((bits >> X.index(cx)) & 1u)
+                {
+                const uint32_t c = G.cell_base + (uint32_t)((cz * Y.n + cy) * X.n + cx);
+                const uint32_t r = a.cell_rank ? a.cell_rank[c] : c;
+                st[q] = a.start[r];
+                ct[q] = a.start[r + 1] - st[q];
+                }
+            }
+        }
+#pragma unroll
+    for (uint32_t q = 0; q < kGroupSpan; ++q)
+        {
+        ncell += ct[q] != 0u ? 1u : 0u;
+        ncand += ct[q];
+        }
+    uint32_t cells, total;
+    uint32_t k0 = wave_exclusive_scan(ncell, lane, cells);
+    uint32_t p0 = wave_exclusive_scan(ncand, lane, total);
+#pragma unroll
+    for (uint32_t q = 0; q < kGroupSpan; ++q)
+        if (ct[q] != 0u)
+            {
+            s.delta[k0] = st[q] - p0;
+            s.first[k0] = p0;
+            s.seq[row * kGroupSpan + (uint32_t)X.index(X.cell((int)q))] = (uint16_t)k0;
+            ++k0;
+            p0 += ct[q];
+            }
+    wave_lds_fence();
+    begin(cells, total);
+
+    // the column's own candidate number (its particle is not its neighbor)
+    uint32_t self = 0xffffffffu;
+    if (in)
+        {
+        const uint32_t own = ((uint32_t)Z.index(me.c[2]) * kGroupSpan + (uint32_t)Y.index(me.c[1])) * kGroupSpan
+                             + (uint32_t)X.index(me.c[0]);
+        self = me.slot - s.delta[s.seq[own]];
+        }
+
+    // |FP32 error| <= 16 2^-24 ((|a| + |b|)^2 + r^2): at most a dozen
+    // roundings of partial sums no larger than that, and the rounding of the
+    // offsets; |a|, |b| <= the window's diagonal.  The direct tests' own error
+    // is far inside 1e-5 r^2.
+    const float wx = (float)(X.len * G.L[0] / X.n), wy = (float)(Y.len * G.L[1] / Y.n),
+                wz = (float)(Z.len * G.L[2] / Z.n);
+    const float diag2 = wx * wx + wy * wy + wz * wz;
+    const float band = 1e-5f * a.thr + (direct ? 0.0f : 9.5367e-7f * (4.0f * diag2 + a.thr));
+
+    const float asq = ax * ax + ay * ay + az * az;
+    const bool listed = in && (uint32_t)me.fixed.w < a.ntypes;
+    // a result is |a - b|^2 - r^2 - band: negative for every pair that may be
+    // listed, and above -2 band (in the integer order of negative floats:
+    // below `near_bits`) where FP32 does not decide
+    const float c0 = !listed ? 1e30f : (ONEHOT == 0 ? asq - a.thr : asq) - band;
+    const int near_bits = __float_as_int(-2.0f * band);
+    f32x16 C;
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+        C[r] = c0;
+    const float bxy = h ? -2.0f * ay : -2.0f * ax;
+    const float bzw = h ? 1.0f : -2.0f * az;
+    [[maybe_unused]] float bt[ONEHOT > 0 ? ONEHOT : 1];
+    if constexpr (ONEHOT > 0)
+        {
+#pragma unroll
+        for (int t = 0; t < ONEHOT; ++t)
+            {
+            const uint32_t tj = 2u * t + h;
+            const double rl = (listed && tj < a.ntypes) ? a.r_listsq[(uint32_t)me.fixed.w * a.ntypes + tj] : 0.0;
+            bt[t] = rl > 0.0 ? -(float)rl : 1e30f;
+            }
+        }
+
+    // candidate this lane reads of each 64: rows 8 (r / 4) + 4 h + r % 4 of a
+    // 32 x 32 result are registers r of lanes of half h, so half h collects
+    // candidates 32 h .. 32 h + 31 (the direct tests take them in lane order)
+    const uint32_t off = direct ? lane : 32u * ((lane >> 2) & 1u) + 16u * h + 4u * ((lane >> 3) & 3u) + (lane & 3u);
+    const uint64_t upto = (2ull << off) - 1ull;
+
+    for (uint32_t seg = 0; seg < total; seg += kGroupSegment)
+        {
+        for (uint32_t w = lane; w < kGroupSegment / 64; w += 64)
+            s.starts[w] = 0ull;
+        wave_lds_fence();
+        uint32_t before = 0; // cells that start before the current 64 candidates
+        for (uint32_t k = lane; k < ((cells + 63u) & ~63u); k += 64)
+            {
+            const uint32_t p = k < cells ? s.first[k] : 0xffffffffu;
+            if (p >= seg && p - seg < kGroupSegment)
+                atomicOr(reinterpret_cast<unsigned long long*>(&s.starts[(p - seg) >> 6]), 1ull << ((p - seg) & 63u));
+            before += (uint32_t)__popcll(__ballot(p < seg));
+            }
+        wave_lds_fence();
+        const uint32_t end = min(total, seg + kGroupSegment);
+        uint32_t next_before = before, slot_next = 0;
+        uint64_t word_next = 0;
+        uint32_t member_next = 0;
+        int4 cand_next;
+        auto fetch = [&](uint32_t P) {
+            uint64_t w = s.starts[(P - seg) >> 6];
+            w = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(w >> 32)) << 32)
+                | (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)w);
+            const uint32_t run = next_before + (uint32_t)__popcll(w & upto) - 1u;
+            const uint32_t p = P + off;
+            const uint32_t at = s.delta[run] + p; // past the last candidate: not a slot
+            slot_next = p < total ? at : 0xffffffffu;
+            cand_next = a.cell_fixed[p < total ? at : 0u];
+            if constexpr (MEMBERS)
+                member_next = a.members[p < total ? at : 0u];
+            word_next = w;
+            next_before += (uint32_t)__popcll(w);
+        };
+        fetch(seg);
+        for (uint32_t P = seg; P < end; P += 64)
+            {
+            const int4 c = cand_next;
+            const uint32_t slot = slot_next, member = member_next;
+            const uint64_t word = word_next;
+            const uint32_t base = next_before - (uint32_t)__popcll(word);
+            if (P + 64 < end)
+                fetch(P + 64);
+            const bool real = slot != 0xffffffffu && (uint32_t)c.w < a.ntypes;
+            uint32_t mask = 0, near = 0;
+            if (!direct)
+                {
+                const float x = (float)fixed_delta(c.x, fx0) * sx;
+                const float y = (float)fixed_delta(c.y, fy0) * sy;
+                const float z = (float)fixed_delta(c.z, fz0) * sz;
+                const float w = real ? x * x + y * y + z * z : 1e30f;
+                // both halves of 32 candidates as A operands (k = 0 in lanes
+                // 0..31, k = 1 in lanes 32..63)
+                auto pair_up = [](float p, float q, float& first, float& second) {
+                    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(p), __float_as_uint(q), false, false);
+                    first = __uint_as_float(r[0]);
+                    second = __uint_as_float(r[1]);
+                };
+                float xy0, xy1, zw0, zw1;
+                pair_up(x, y, xy0, xy1);
+                pair_up(z, w, zw0, zw1);
+                f32x16 d0 = __builtin_amdgcn_mfma_f32_32x32x2f32(xy0, bxy, C, 0, 0, 0);
+                f32x16 d1 = __builtin_amdgcn_mfma_f32_32x32x2f32(xy1, bxy, C, 0, 0, 0);
+                d0 = __builtin_amdgcn_mfma_f32_32x32x2f32(zw0, bzw, d0, 0, 0, 0);
+                d1 = __builtin_amdgcn_mfma_f32_32x32x2f32(zw1, bzw, d1, 0, 0, 0);
+                if constexpr (ONEHOT > 0)
+                    {
+#pragma unroll
+                    for (int t = 0; t < ONEHOT; ++t)
+                        {
+                        float e0, e1;
+                        pair_up(c.w == 2 * t ? 1.0f : 0.0f, c.w == 2 * t + 1 ? 1.0f : 0.0f, e0, e1);
+                        d0 = __builtin_amdgcn_mfma_f32_32x32x2f32(e0, bt[t], d0, 0, 0, 0);
+                        d1 = __builtin_amdgcn_mfma_f32_32x32x2f32(e1, bt[t], d1, 0, 0, 0);
+                        }
+                    }
+                int least = 0;
+#pragma unroll
+                for (int r = 15; r >= 0; --r)
+                    mask = __builtin_amdgcn_alignbit(mask, __float_as_uint(d1[r]), 31);
+#pragma unroll
+                for (int r = 15; r >= 0; --r)
+                    mask = __builtin_amdgcn_alignbit(mask, __float_as_uint(d0[r]), 31);
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    least = min(least, min(__float_as_int(d0[r]), __float_as_int(d1[r])));
+                if (__ballot(least < near_bits) != 0ull)
+                    {
+                    uint32_t sure = 0;
+#pragma unroll
+                    for (int r = 15; r >= 0; --r)
+                        sure = __builtin_amdgcn_alignbit(sure, __float_as_uint(d1[r] + 2.0f * band), 31);
+#pragma unroll
+                    for (int r = 15; r >= 0; --r)
+                        sure = __builtin_amdgcn_alignbit(sure, __float_as_uint(d0[r] + 2.0f * band), 31);
+                    near = mask & ~sure;
+                    }
+                }
+            else
+                {
+                for (uint32_t m = served; m != 0u; m &= m - 1u)
+                    {
+                    const int q = __builtin_ctz(m);
+                    const uint32_t tq = (uint32_t)lane_value(me.fixed.w, q);
+                    const float x = (float)fixed_delta(c.x, lane_value(me.fixed.x, q)) * sx;
+                    const float y = (float)fixed_delta(c.y, lane_value(me.fixed.y, q)) * sy;
+                    const float z = (float)fixed_delta(c.z, lane_value(me.fixed.z, q)) * sz;
+                    const bool both = real && tq < a.ntypes;
+                    float rl = a.thr;
+                    if (ONEHOT > 0 || a.direct)
+                        rl = both ? (float)a.r_listsq[tq * a.ntypes + (uint32_t)c.w] : 0.0f;
+                    const float d = (both && rl > 0.0f) ? x * x + y * y + z * z - rl - band : 1e30f;
+                    const uint64_t hit = __ballot(d < 0.0f), maybe = __ballot(__float_as_int(d) < near_bits);
+                    if (col == (uint32_t)q)
+                        {
+                        mask = h ? (uint32_t)(hit >> 32) : (uint32_t)hit;
+                        near = h ? (uint32_t)(maybe >> 32) : (uint32_t)maybe;
+                        }
+                    }
+                }
+            near = listed ? near : 0u;
+            if (__ballot(near != 0u) != 0ull)
+                {
+                // FP32 cannot decide these: the FP64 predicate of the host oracle
+                while (near != 0u)
+                    {
+                    const uint32_t bit = (uint32_t)__builtin_ctz(near);
+                    near &= near - 1u;
+                    const uint32_t q = 32u * h + bit;
+                    const uint32_t run = base + (uint32_t)__popcll(word & ((2ull << q) - 1ull)) - 1u;
+                    const uint32_t cs = s.delta[run] + P + q;
+                    const uint32_t j = a.members[cs];
+                    const double4 pi = a.pos[me.i], pj = a.pos[j];
+                    const double rl = a.r_listsq[(uint32_t)me.fixed.w * a.ntypes + (uint32_t)a.cell_fixed[cs].w];
+                    const double ex = min_image_1d(pi.x - pj.x, G.L[0], G.Linv[0]);
+                    const double ey = min_image_1d(pi.y - pj.y, G.L[1], G.Linv[1]);
+                    const double ez = min_image_1d(pi.z - pj.z, G.L[2], G.Linv[2]);
+                    const bool hit = rl > 0.0 && rsq3_nofma(ex, ey, ez) <= rl;
+                    mask = hit ? mask | (1u << bit) : mask & ~(1u << bit);
+                    }
+                }
+            const uint32_t ds = self - (P + 32u * h);
+            mask &= ds < 32u ? ~(1u << ds) : 0xffffffffu;
+            emit(mask, P, off, MEMBERS ? member : slot);
+            }
+        }
+    return served;
+    }
+
+} // namespace azp

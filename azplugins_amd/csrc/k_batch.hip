@@ -8,8 +8,9 @@
 //
 // * One cell list over all replicas: replica r owns a contiguous range of
 //   global cells (its own grid, cells at least r_list wide) and a contiguous
-//   range of particles; the walk lists each particle's neighbors inside its
-//   own replica with the same FP64 predicate as the single-system build.
+//   range of particles; the walk (group_walk.h) lists each particle's neighbors
+//   inside its own replica with the same FP64 predicate as the single-system
+//   build.
 // * One persistent force launch: a grid sized to the chip pulls 64-particle
 //   chunks from a work counter, so replicas of 500 and of 20,000 particles
 //   share the launch without tail effects.  Block size, chunks per fetch and
@@ -28,6 +29,7 @@
 #include <vector>
 
 #include "cells.h"
+#include "group_walk.h"
 #include "tpm.h"
 
 namespace azp
@@ -125,13 +127,25 @@ __global__ void k_b_scatter(uint32_t N,
     members[start[cell_of[i]] + slot_of[i]] = i;
     }
 
-// Each cell's members in increasing particle index (a deterministic order).
-// One wavefront per cell: a member's place is the number of the cell's
-// members with a smaller index (indices are distinct), so after copying the
-// cell to LDS every lane writes its members straight to their places.  A
-// cell with more members than the copy holds is sorted by the wavefront's
-// first lane (insertion sort).  Every exit is uniform over the wavefront and
-// lanes exchange data only through their wavefront's LDS row.
+// The cell-ordered copy of particle j for the walk: wrapped fixed-point
+// position in its replica's box and its type; ntypes in place of a type out of
+// range, ntypes + 1 for a position that is not finite (never listed).
+__device__ __forceinline__ int4 b_cell_entry(const double4& p, const RepInfo& R, uint32_t ntypes)
+    {
+    if (!(isfinite(p.x) && isfinite(p.y) && isfinite(p.z)))
+        return make_int4(0, 0, 0, (int)(ntypes + 1u));
+    return make_int4(to_fixed(p.x, R.Linv[0]), to_fixed(p.y, R.Linv[1]), to_fixed(p.z, R.Linv[2]),
+                     (int)checked_type(p.w, ntypes));
+    }
+
+// Each cell's members in increasing particle index (a deterministic order),
+// and their cell-ordered copies.  One wavefront per cell: a member's place is
+// the number of the cell's members with a smaller index (indices are
+// distinct), so after copying the cell to LDS every lane writes its members
+// straight to their places.  A cell with more members than the copy holds is
+// sorted by the wavefront's first lane (insertion sort).  Every exit is
+// uniform over the wavefront and lanes exchange data only through their
+// wavefront's LDS row.
 constexpr uint32_t kSortWaves = 4;
 constexpr uint32_t kSortCap = 256;
 
@@ -140,6 +154,10 @@ __global__ void __launch_bounds__(256) k_b_sort_cells(uint32_t ncell,
                                                       const uint32_t* __restrict__ rep_flag,
                                                       const uint32_t* __restrict__ start,
                                                       uint32_t* __restrict__ members,
+                                                      const double4* __restrict__ pos,
+                                                      const RepInfo* __restrict__ reps,
+                                                      uint32_t ntypes,
+                                                      int4* __restrict__ cell_fixed,
                                                       const uint32_t* gate)
     {
     __shared__ uint32_t s_m[kSortWaves][kSortCap];
@@ -150,13 +168,13 @@ __global__ void __launch_bounds__(256) k_b_sort_cells(uint32_t ncell,
     const uint32_t c = blockIdx.x * kSortWaves + w;
     if (c >= ncell || !rep_flag[cell_rep[c]])
         return;
+    const RepInfo& R = reps[cell_rep[c]];
     const uint32_t b = start[c];
     const uint32_t n = start[c + 1] - b;
-    if (n < 2)
-        return;
     if (n > kSortCap)
         {
         if (lane == 0)
+            {
             for (uint32_t k = b + 1; k < b + n; ++k)
                 {
                 const uint32_t v = members[k];
@@ -168,14 +186,15 @@ __global__ void __launch_bounds__(256) k_b_sort_cells(uint32_t ncell,
                     }
                 members[m] = v;
                 }
+            for (uint32_t k = b; k < b + n; ++k)
+                cell_fixed[k] = b_cell_entry(pos[members[k]], R, ntypes);
+            }
         return;
         }
     uint32_t* sm = s_m[w];
     for (uint32_t k = lane; k < n; k += 64)
         sm[k] = members[b + k];
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_lds_fence();
     for (uint32_t k = lane; k < n; k += 64)
         {
         const uint32_t v = sm[k];
@@ -183,20 +202,17 @@ __global__ void __launch_bounds__(256) k_b_sort_cells(uint32_t ncell,
         for (uint32_t t = 0; t < n; ++t)
             rank += sm[t] < v ? 1u : 0u;
         members[b + rank] = v;
+        cell_fixed[b + rank] = b_cell_entry(pos[v], R, ntypes);
         }
     }
 
 struct BatchWalkArgs
     {
-    const double4* pos;
+    GroupArgs g;
     uint32_t N;
     const uint32_t* rep_of;
     const RepInfo* reps;
     const uint32_t* cell_of;
-    const uint32_t* start;
-    const uint32_t* members;
-    const double* r_listsq;
-    uint32_t ntypes;
     uint32_t* n_neigh;
     uint32_t* nlist;
     uint32_t pitch;
@@ -206,118 +222,121 @@ struct BatchWalkArgs
     const uint32_t* rep_flag;
     };
 
-// Particle i's neighbors inside its own replica (same cell order, predicate
-// and rounding as the single-system walk).
-__device__ uint32_t b_walk_one(const BatchWalkArgs& a, uint32_t i, const double* __restrict__ r_listsq)
-    {
-    const double4 pi = a.pos[i];
-    const uint32_t ti = checked_type(pi.w, a.ntypes);
-    const bool finite = isfinite(pi.x) && isfinite(pi.y) && isfinite(pi.z);
-    if (ti == a.ntypes || !finite)
-        {
-        atomicOr(a.flags + 2, finite ? 1u : 2u);
-        return 0;
-        }
-    const RepInfo& R = a.reps[a.rep_of[i]];
-    // the box in registers: the list stores below may not be assumed apart
-    // from the replica table, which would otherwise be reloaded per candidate
-    const double L0 = R.L[0], L1 = R.L[1], L2 = R.L[2];
-    const double Li0 = R.Linv[0], Li1 = R.Linv[1], Li2 = R.Linv[2];
-    const uint32_t lc = a.cell_of[i] - R.cell_base;
-    const int cx = (int)(lc % (uint32_t)R.n[0]);
-    const int cy = (int)((lc / (uint32_t)R.n[0]) % (uint32_t)R.n[1]);
-    const int cz = (int)(lc / ((uint32_t)R.n[0] * (uint32_t)R.n[1]));
-    int ox[3], oy[3], oz[3];
-    const int nx = stencil_axis(cx, R.n[0], ox);
-    const int ny = stencil_axis(cy, R.n[1], oy);
-    const int nz = stencil_axis(cz, R.n[2], oz);
-    uint32_t count = 0;
-    auto consider = [&](uint32_t j, const double4& pj) {
-        if (j == i)
-            return;
-        const uint32_t tj = checked_type(pj.w, a.ntypes);
-        if (tj == a.ntypes)
-            return;
-        const double rl = r_listsq[ti * a.ntypes + tj];
-        if (!(rl > 0.0))
-            return;
-        const double dx = min_image_1d(pi.x - pj.x, L0, Li0);
-        const double dy = min_image_1d(pi.y - pj.y, L1, Li1);
-        const double dz = min_image_1d(pi.z - pj.z, L2, Li2);
-        const double rsq = rsq3_nofma(dx, dy, dz);
-        if (rsq <= rl)
-            {
-            if (count < a.max_neighbors)
-                a.nlist[(size_t)count * a.pitch + i] = j;
-            ++count;
-            }
-    };
-    for (int iz = 0; iz < nz; ++iz)
-        for (int iy = 0; iy < ny; ++iy)
-            for (int ix = 0; ix < nx; ++ix)
-                {
-                const uint32_t nb = R.cell_base + (uint32_t)((oz[iz] * R.n[1] + oy[iy]) * R.n[0] + ox[ix]);
-                const uint32_t b = a.start[nb], e = a.start[nb + 1];
-                // four candidates at a time: their member and position
-                // loads are in flight together; they are tested in order
-                uint32_t m = b;
-                for (; m + 4 <= e; m += 4)
-                    {
-                    uint32_t jj[4];
-                    double4 pp[4];
-#pragma unroll
-                    for (int u = 0; u < 4; ++u)
-                        jj[u] = a.members[m + u];
-#pragma unroll
-                    for (int u = 0; u < 4; ++u)
-                        pp[u] = a.pos[jj[u]];
-#pragma unroll
-                    for (int u = 0; u < 4; ++u)
-                        consider(jj[u], pp[u]);
-                    }
-                for (; m < e; ++m)
-                    {
-                    const uint32_t j = a.members[m];
-                    consider(j, a.pos[j]);
-                    }
-                }
-    return count;
-    }
+// The flagged replicas' lists: one wavefront per group of 32 consecutive
+// cell-list slots (group_walk.h).  The hit masks of up to kWalkBuffer x 64
+// candidates are kept in LDS with the candidates' particle indices and then
+// written out together: lane l < 32 takes the first half of its column's
+// candidates and lane l + 32 the second, one entry per step, so a step stores
+// to two rows of 32 consecutive columns instead of 64 scattered words.
+// Bound by VALU issue (0.75 ms of it) and latency: 1.21 ms for the lists of
+// all 512 replicas of the workload (2.6M particles), 4.76 ms with a lane per
+// particle walking its 27 cells through position gathers in FP64, 1.83 ms with
+// the entries stored to scattered words as they were found.
+constexpr uint32_t kWalkWaves = 4;
+constexpr uint32_t kWalkBuffer = 8;
 
-// One lane per particle; each wavefront pads its columns with the lane's own
-// index up to its longest list rounded up to 8 (as the single-system walk).
-__global__ void __launch_bounds__(256) k_b_walk(const BatchWalkArgs a)
+template<int ONEHOT> __global__ void __launch_bounds__(64 * kWalkWaves, 4) k_b_walk(const BatchWalkArgs a)
     {
-    // the list radii (up to 8 types) in LDS
-    __shared__ double s_rl[64];
+    __shared__ GroupLds s_group[kWalkWaves];
+    __shared__ uint32_t s_mask[kWalkWaves][kWalkBuffer * 64];
+    __shared__ uint32_t s_j[kWalkWaves][kWalkBuffer * 64];
     if (gated_off(a.gate))
         return;
-    const uint32_t nt2 = a.ntypes * a.ntypes;
-    const bool staged = nt2 <= 64u;
-    if (staged)
+    const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63u, h = lane >> 5;
+    const uint32_t group = xcd_logical_block() * (blockDim.x >> 6) + w;
+    GroupColumn me;
+    me.slot = group * 32u + (lane & 31u);
+    me.valid = me.slot < a.N;
+    me.i = me.valid ? a.g.members[me.slot] : 0u;
+    const uint32_t rep = a.rep_of[me.i];
+    me.valid = me.valid && a.rep_flag[rep] != 0u;
+    uint32_t todo = (uint32_t)__ballot(me.valid);
+    if (todo == 0u)
+        return; // the whole wavefront (no barrier below spans wavefronts)
+    me.cell = a.cell_of[me.i];
+    const uint32_t lc = me.valid ? me.cell - a.reps[rep].cell_base : 0u;
+    const int nx = a.reps[rep].n[0], ny = a.reps[rep].n[1];
+    me.c[0] = (int)(lc % (uint32_t)nx);
+    me.c[1] = (int)((lc / (uint32_t)nx) % (uint32_t)ny);
+    me.c[2] = (int)(lc / ((uint32_t)nx * (uint32_t)ny));
+    me.fixed = a.g.cell_fixed[me.valid ? me.slot : 0u];
+    if (me.valid && h == 0u && (uint32_t)me.fixed.w >= a.g.ntypes)
+        atomicOr(a.flags + 2, (uint32_t)me.fixed.w == a.g.ntypes ? 1u : 2u);
+    uint32_t count = 0; // entries of the column (in both of its lanes)
+    uint32_t left = 0, held = 0, hold = 0, half = 0; // 64-candidate batches: to come, buffered, to buffer, first half
+    uint32_t first = 0, added = 0; // hits of the buffered batches: of the first half, of all
+    auto next_buffer = [&]() {
+        hold = min(left, kWalkBuffer);
+        half = (hold + 1u) / 2u;
+        held = first = added = 0u;
+    };
+    auto begin = [&](uint32_t, uint32_t total) {
+        left = (total + 63u) / 64u;
+        next_buffer();
+    };
+    auto emit = [&](uint32_t mask, uint32_t, uint32_t off, uint32_t j) {
+        s_mask[w][held * 64u + lane] = mask;
+        s_j[w][held * 64u + off] = j;
+        const uint32_t hits = (uint32_t)__popc(mask), both = hits + (uint32_t)__shfl_xor((int)hits, 32);
+        first += held < half ? both : 0u;
+        added += both;
+        if (++held < hold)
+            return;
+        wave_lds_fence();
+        uint32_t at = count + (h ? first : 0u);
+        uint32_t* dst = a.nlist + (size_t)at * a.pitch + me.i;
+        uint32_t q = h ? 2u * half : 0u, word = 0u, base = 0u;
+        const uint32_t qe = h ? 2u * hold : 2u * half;
+        for (;;)
+            {
+            while (word == 0u && q < qe)
+                {
+                base = q * 32u;
+                word = s_mask[w][base + (lane & 31u)];
+                ++q;
+                }
+            if (__ballot(word != 0u) == 0ull)
+                break;
+            if (word != 0u)
+                {
+                const uint32_t j = s_j[w][base + (uint32_t)__builtin_ctz(word)];
+                word &= word - 1u;
+                if (at < a.max_neighbors)
+                    *dst = j;
+                ++at;
+                dst += a.pitch;
+                }
+            }
+        wave_lds_fence();
+        count += added;
+        left -= hold;
+        next_buffer();
+    };
+    while (todo != 0u)
         {
-        for (uint32_t t = threadIdx.x; t < nt2; t += blockDim.x)
-            s_rl[t] = a.r_listsq[t];
-        __syncthreads();
+        const int al = group_anchor(todo);
+        const uint32_t r0 = (uint32_t)lane_value((int)rep, al);
+        const RepInfo& R = a.reps[r0];
+        GroupGeom G;
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            {
+            G.n[k] = R.n[k];
+            G.L[k] = R.L[k];
+            G.Linv[k] = R.Linv[k];
+            G.scale[k] = R.fx_scale[k];
+            }
+        G.cell_base = R.cell_base;
+        todo &= ~group_pass<ONEHOT, true>(a.g, G, s_group[w], me, todo, al, rep == r0, begin, emit);
         }
-    const uint32_t i = xcd_logical_block() * blockDim.x + threadIdx.x;
-    const bool active = i < a.N && a.rep_flag[a.rep_of[i]] != 0u;
-    const uint32_t count = active ? b_walk_one(a, i, staged ? s_rl : a.r_listsq) : 0u;
-    if (active)
+    if (me.valid && h == 0u)
         {
         // a list longer than the capacity is truncated (and reported), so
         // consumers never read past the allocation
-        a.n_neigh[i] = min(count, a.max_neighbors);
+        a.n_neigh[me.i] = min(count, a.max_neighbors);
         if (count > a.max_neighbors)
             atomicMax(a.flags, count);
         }
-    uint32_t wmax = count;
-    for (int off = 32; off > 0; off >>= 1)
-        wmax = max(wmax, (uint32_t)__shfl_xor((int)wmax, off));
-    const uint32_t padded = (wmax + 7u) & ~7u;
-    if (active && wmax <= a.max_neighbors)
-        for (uint32_t k = count; k < padded; ++k)
-            a.nlist[(size_t)k * a.pitch + i] = i;
     }
 
 // Snapshot of the positions of the last build of each rebuilt replica, and
@@ -740,6 +759,7 @@ struct azp_batch
     DeviceArray<uint32_t> cell_of, slot_of, cell_count, cell_start, members, cell_rep, scan_sums;
     DeviceArray<uint32_t> n_neigh, list, flags, counter, rep_flag;
     DeviceArray<double4> last_pos;
+    DeviceArray<int4> cell_fixed;
     DeviceArray<float4> dirs;
     DeviceArray<unsigned long long> d_timestep, d_builds; // builds: [0] rebuild events, [1] replica rebuilds
     uint32_t* h_flags = nullptr; // pinned
@@ -904,6 +924,7 @@ int batch_upload_tables(azp_batch* b, hipStream_t s)
     AZP_TRY(b->members.reserve(b->N));
     AZP_TRY(b->n_neigh.reserve(b->N));
     AZP_TRY(b->last_pos.reserve(b->N));
+    AZP_TRY(b->cell_fixed.reserve(b->N));
     AZP_TRY(b->dirs.reserve(b->N));
     AZP_TRY(b->cell_count.reserve(b->ncell));
     AZP_TRY(b->cell_start.reserve((size_t)b->ncell + 1));
@@ -957,17 +978,22 @@ void enqueue_rebuild(azp_batch* b, hipStream_t s)
     hipLaunchKernelGGL(k_b_scatter, dim3(grid_for(N, B)), dim3(B), 0, s, N, b->rep_of.ptr, rf, b->cell_of.ptr,
                        b->slot_of.ptr, b->cell_start.ptr, b->members.ptr, gate);
     hipLaunchKernelGGL(k_b_sort_cells, dim3((b->ncell + kSortWaves - 1) / kSortWaves), dim3(64 * kSortWaves), 0, s,
-                       b->ncell, b->cell_rep.ptr, rf, b->cell_start.ptr, b->members.ptr, gate);
+                       b->ncell, b->cell_rep.ptr, rf, b->cell_start.ptr, b->members.ptr, pos, b->d_reps.ptr, b->ntypes,
+                       b->cell_fixed.ptr, gate);
     BatchWalkArgs wa;
-    wa.pos = pos;
+    wa.g.pos = pos;
+    wa.g.members = b->members.ptr;
+    wa.g.start = b->cell_start.ptr;
+    wa.g.cell_rank = nullptr;
+    wa.g.cell_fixed = b->cell_fixed.ptr;
+    wa.g.r_listsq = b->d_rlistsq.ptr;
+    wa.g.ntypes = b->ntypes;
+    wa.g.r_max = (float)b->r_list_max();
+    wa.g.thr = (float)(b->r_list_max() * b->r_list_max());
     wa.N = N;
     wa.rep_of = b->rep_of.ptr;
     wa.reps = b->d_reps.ptr;
     wa.cell_of = b->cell_of.ptr;
-    wa.start = b->cell_start.ptr;
-    wa.members = b->members.ptr;
-    wa.r_listsq = b->d_rlistsq.ptr;
-    wa.ntypes = b->ntypes;
     wa.n_neigh = b->n_neigh.ptr;
     wa.nlist = b->list.ptr;
     wa.pitch = b->pitch;
@@ -976,7 +1002,15 @@ void enqueue_rebuild(azp_batch* b, hipStream_t s)
     wa.gate = gate;
     wa.rep_flag = rf;
     const unsigned wb = b->tune.walk_block ? b->tune.walk_block : 256;
-    hipLaunchKernelGGL(k_b_walk, dim3(grid_for(N, wb)), dim3(wb), 0, s, wa);
+    const dim3 walk_grid(grid_for(((size_t)N + 31) / 32, wb / 64));
+    bool uniform = true;
+    for (double rc : b->r_cut)
+        uniform = uniform && rc == b->r_cut[0];
+    wa.g.direct = !uniform && b->ntypes > 8;
+    if (uniform || wa.g.direct)
+        hipLaunchKernelGGL(k_b_walk<0>, walk_grid, dim3(wb), 0, s, wa);
+    else
+        hipLaunchKernelGGL(k_b_walk<4>, walk_grid, dim3(wb), 0, s, wa);
     hipLaunchKernelGGL(k_b_copy_last, dim3(grid_for(N, B)), dim3(B), 0, s, pos, b->last_pos.ptr, N, b->rep_of.ptr,
                        b->d_reps.ptr, rf, b->d_builds.ptr, gate);
     }

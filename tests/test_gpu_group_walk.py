@@ -1,0 +1,99 @@
+"""Group neighbor walk (32 particles and 64 candidates at a time on the matrix
+cores): the lists it writes hold the oracle's pairs, each once, where its
+windows, passes and remainders can go wrong — grids of 2 to 9 cells per axis,
+boxes of unequal edges, groups that straddle replicas and grid rows, 1 to 33
+particles, more candidates than one segment, several list radii.
+"""
+
+import numpy as np
+import pytest
+
+import oracle
+from azplugins_amd import _azp
+from azplugins_amd.batch import ReplicaBatch
+from gpu_util import say
+
+torch = _azp.torch
+pytestmark = pytest.mark.gpu
+
+RC, BUFF = 1.1, 0.4
+RL = RC + BUFF
+
+
+def _batch_lists(boxes, pos4, r_cut):
+    """Directed pairs (i << 32 | j) of every replica, by replica-local index."""
+    nt = r_cut.shape[0]
+    b = ReplicaBatch([p.shape[0] for p in pos4], boxes, ntypes=nt, r_cut=RC, r_buff=BUFF, precision="fp64")
+    for i in range(nt):
+        for j in range(i, nt):
+            b.set_params(i, j, M_d=1.0, M_r=0.2, r_eq=1.0, omega=20.0, alpha=0.4, repulsion=True)
+            _azp.call("azp_batch_set_r_cut", b._h, i, j, float(r_cut[i, j]))
+    b.load(np.concatenate(pos4))
+    b.compute(force_rebuild=True)
+    nn, lst = b.nlist()
+    out = []
+    for r in range(len(pos4)):
+        lo, hi = int(b.offsets[r]), int(b.offsets[r + 1])
+        n = nn[lo:hi].astype(np.int64)
+        k = np.arange(lst.shape[0])[:, None] < n[None, :]
+        j = lst[:, lo:hi].astype(np.int64) - lo
+        i = np.broadcast_to(np.arange(hi - lo)[None, :], j.shape)
+        assert np.all((j[k] >= 0) & (j[k] < hi - lo)), "neighbor outside its replica"
+        out.append(np.sort((i[k] << 32) | j[k]))
+    return out
+
+
+def _oracle_pairs(box, pos4, r_cut):
+    nt = r_cut.shape[0]
+    a, b = (x.astype(np.int64) for x in oracle.nlist(pos4, np.asarray(box), nt,
+                                                     oracle.r_listsq_matrix(r_cut.ravel(), BUFF), "brute"))
+    return np.sort(np.concatenate([(a << 32) | b, (b << 32) | a]))
+
+
+def _check(boxes, sizes, r_cut, seed):
+    rng = np.random.default_rng(seed)
+    pos4 = []
+    for box, n in zip(boxes, sizes):
+        p = np.zeros((n, 4))
+        p[:, :3] = rng.uniform(-0.5, 0.5, (n, 3)) * np.asarray(box)
+        p[:, 3] = rng.integers(0, r_cut.shape[0], n)
+        pos4.append(p)
+    say(f"[group walk] sizes {sizes} types {r_cut.shape[0]}")
+    got = _batch_lists(boxes, pos4, r_cut)
+    for r, (box, p) in enumerate(zip(boxes, pos4)):
+        assert np.array_equal(got[r], _oracle_pairs(box, p, r_cut)), f"replica {r}"
+
+
+@pytest.mark.parametrize("cells", [2, 3, 4, 5, 6, 9])
+def test_group_walk_grids(cells):
+    """Cubic and unequal boxes of `cells` cells on the shortest axis."""
+    L = cells * RL * (1.0 + 1e-8)
+    boxes = [(L, L, L), (L, 1.7 * L, 1.1 * L), (1.3 * L, L, 2.4 * L), (cells * RL,) * 3, (L, L, L)]
+    _check(boxes, [31, 700, 333, 64, 1], np.array([[RC]]), cells)
+
+
+def test_group_walk_straddling_replicas():
+    """Replicas of a few particles share groups."""
+    rng = np.random.default_rng(3)
+    sizes = [1, 2, 3, 5, 8, 13, 21, 32, 33, 7, 1, 64]
+    boxes = [tuple(rng.uniform(2.0, 7.0, 3) * RL) for _ in sizes]
+    _check(boxes, sizes, np.array([[RC]]), 4)
+
+
+def test_group_walk_more_candidates_than_a_segment():
+    """Three cells per axis hold 8,700 candidates for every particle."""
+    L = 3.1 * RL
+    _check([(L, L, L), (L, L, L)], [8700, 40], np.array([[RC]]), 5)
+
+
+@pytest.mark.parametrize("types", [2, 3, 8, 11])
+def test_group_walk_list_radii(types):
+    """Several list radii, excluded type pairs among them."""
+    rng = np.random.default_rng(types)
+    rc = rng.uniform(0.5 * RC, RC, (types, types))
+    rc = np.minimum(rc, rc.T)
+    rc[0, 0] = RC
+    rc[1, 1] = 0.0
+    rc[0, types - 1] = rc[types - 1, 0] = 0.0
+    L = 4.2 * RL
+    _check([(L, L, L), (2.1 * RL, 1.5 * L, L), (2.5 * L, L, L)], [500, 200, 900], rc, 6)
