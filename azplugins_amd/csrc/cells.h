@@ -88,6 +88,25 @@ __device__ __forceinline__ int cell_coord(double x, double L, double Linv, int n
     return c;
     }
 
+// Slot of each lane's particle within its counter: count[r] grows by one per
+// active lane and the lane gets its place (in no particular order).  One
+// atomic for each run of consecutive lanes with the same r (neighbors in
+// memory usually share a cell), all of the wavefront's runs in one
+// instruction; every lane of the wavefront calls this.
+__device__ __forceinline__ uint32_t count_by_runs(uint32_t r, bool active, uint32_t* __restrict__ count)
+    {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t prev = (uint32_t)__shfl_up((int)(active ? r : 0xffffffffu), 1);
+    const uint64_t heads = __ballot(lane == 0u || !active || prev != r);
+    const uint32_t head = 63u - (uint32_t)__builtin_clzll(heads & ((2ull << lane) - 1ull));
+    const uint64_t after = heads & ~((2ull << head) - 1ull);
+    const uint32_t end = after != 0ull ? (uint32_t)__builtin_ctzll(after) : 64u;
+    uint32_t base = 0;
+    if (active && lane == head)
+        base = atomicAdd(&count[r], end - head);
+    return (uint32_t)__shfl((int)base, (int)head) + (lane - head);
+    }
+
 // Type index of a particle, or ntypes when pos.w is not a valid type index.
 __device__ __forceinline__ uint32_t checked_type(double w, uint32_t ntypes)
     {
@@ -95,21 +114,14 @@ __device__ __forceinline__ uint32_t checked_type(double w, uint32_t ntypes)
     }
 
 // The neighbor cells of cell c along one axis (c-1, c, c+1 with periodic
-// wrap), with duplicates removed when the grid is narrower than 3 cells.
-// Returns how many distinct cells were written to out.
+// wrap) in ascending order, with duplicates removed when the grid is narrower
+// than 3 cells.  Returns how many distinct cells were written to out.
 __device__ __forceinline__ int stencil_axis(int c, int n, int out[3])
     {
-    int m = 0;
-    for (int d = -1; d <= 1; ++d)
-        {
-        const int x = (c + d + n) % n;
-        bool dup = false;
-        for (int k = 0; k < m; ++k)
-            dup |= (out[k] == x);
-        if (!dup)
-            out[m++] = x;
-        }
-    return m;
+    out[0] = c == 0 || c == n - 1 ? 0 : c - 1;
+    out[1] = c == 0 ? 1 : (c == n - 1 ? max(1, n - 2) : c);
+    out[2] = c == 0 || c == n - 1 ? n - 1 : c + 1;
+    return min(n, 3);
     }
 
 // ---------------------------------------------------------------------------

@@ -1,14 +1,17 @@
-// Neighbor search of a group of 32 consecutive cell-list slots by one
+// Neighbor search of a group of 64 consecutive cell-list slots by one
 // wavefront, on the matrix cores.
 //
-// The squared distances of 32 candidates to the group's 32 particles are a
-// contraction: with candidates and particles as offsets b, a from an anchor,
+// The squared distances of 32 candidates to 32 particles are a contraction:
+// with candidates and particles as offsets b, a from an anchor,
 //   |a - b|^2 - r^2 = (|a|^2 - r^2) - 2 a.b + |b|^2 . 1,
 // K = 4 in FP32, i.e. two v_mfma_f32_32x32x2_f32 for 1,024 pairs with the
 // particle's |a|^2 - r^2 as the C operand.  The sign of a result is the hit,
 // so a lane collects 32 candidates of one particle into a 32-bit mask with
 // one v_alignbit each (bit o = candidate o), against about eight
 // instructions and a serial append per pair in a lane-per-particle loop.
+// 64 particles share the candidates' reads and conversions; exchanging the
+// halves of two registers then gives every lane both mask words of its own
+// particle.
 // Pairs whose result lies within the FP32 error bound of the list radius are
 // decided by the FP64 predicate of the host oracle, so the pair set is the
 // FP64 one.
@@ -33,7 +36,7 @@ constexpr int kGroupReach = 2;
 constexpr uint32_t kGroupSpan = 2 * kGroupReach + 3;
 constexpr uint32_t kGroupCells = kGroupSpan * kGroupSpan * kGroupSpan;
 // Candidates per segment of a pass (the bits of GroupLds::starts).
-constexpr uint32_t kGroupSegment = 8192;
+constexpr uint32_t kGroupSegment = 2048;
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -83,15 +86,16 @@ __device__ __forceinline__ int lane_value(int v, int lane)
     return __builtin_amdgcn_readlane(v, lane);
     }
 
-__device__ __forceinline__ uint32_t wave_exclusive_scan(uint32_t v, uint32_t lane, uint32_t& total)
+// Exclusive sum over the wavefront (row shifts and broadcasts, no LDS).
+__device__ __forceinline__ uint32_t wave_exclusive_scan(uint32_t v, uint32_t& total)
     {
     uint32_t x = v;
-    for (uint32_t off = 1; off < 64; off <<= 1)
-        {
-        const uint32_t y = (uint32_t)__shfl_up((int)x, off);
-        if (lane >= off)
-            x += y;
-        }
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false); // row_shr:1
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false); // row_bcast:15
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false); // row_bcast:31
     total = (uint32_t)lane_value((int)x, 63);
     return x - v;
     }
@@ -129,8 +133,7 @@ struct GroupAxis
         }
     };
 
-// The particle a lane's column stands for (lanes l and l + 32 share column
-// l & 31).
+// The particle a lane's column stands for.
 struct GroupColumn
     {
     bool valid;
@@ -140,64 +143,69 @@ struct GroupColumn
     };
 
 // The anchor column of a pass over the columns `todo` (not 0): the middle one.
-__device__ __forceinline__ int group_anchor(uint32_t todo)
+__device__ __forceinline__ int group_anchor(uint64_t todo)
     {
-    const uint32_t first = (uint32_t)__builtin_ctz(todo), last = 31u - (uint32_t)__builtin_clz(todo);
-    return __builtin_ctz(todo >> ((first + last) / 2u) << ((first + last) / 2u));
+    const uint32_t first = (uint32_t)__builtin_ctzll(todo), last = 63u - (uint32_t)__builtin_clzll(todo);
+    return __builtin_ctzll(todo >> ((first + last) / 2u) << ((first + last) / 2u));
+    }
+
+// Exchanges the upper half of p with the lower half of q: low and high
+// candidates (or columns) of two values, k = 0 in lanes 0..31 and k = 1 in
+// lanes 32..63, as the matrix operands take them.
+__device__ __forceinline__ void swap_halves(uint32_t p, uint32_t q, uint32_t& first, uint32_t& second)
+    {
+    const auto r = __builtin_amdgcn_permlane32_swap(p, q, false, false);
+    first = r[0];
+    second = r[1];
+    }
+__device__ __forceinline__ void swap_halves(float p, float q, float& first, float& second)
+    {
+    uint32_t f, g;
+    swap_halves(__float_as_uint(p), __float_as_uint(q), f, g);
+    first = __uint_as_float(f);
+    second = __uint_as_float(g);
     }
 
 // Runs one pass: the columns with `todo` bits whose own cells lie in the
 // window around that of the anchor column `al` (and, by `same`, in its
-// system).  Returns
-// the mask of the columns served.  For every 64 candidates, emit(mask, P,
-// off, which) gets the lane's hits among candidates P + 32 (l >> 5) + bit
-// of its column, and candidate P + off, which this lane read: its particle
-// (MEMBERS; any for a number past the last candidate) or its slot (or ~0).
-// begin(cells, total) runs before the first of them.
+// system).  Returns the mask of the columns served; direct_used is set when
+// it took the direct tests.  For every 64 candidates, emit(low, high, P, off,
+// which) gets the column's hits among candidates P .. P + 63 and candidate
+// P + off, which this lane read: its particle (MEMBERS; any for a number past
+// the last candidate) or its slot (or ~0).  begin(cells, total) runs before
+// the first of them.
 //
 // ONEHOT = 0: one list radius for every type pair (or a.direct).  Otherwise
 // 2 * ONEHOT >= ntypes: K grows by one per type, the candidate's type as a
 // unit vector against the particle's radii.
 template<int ONEHOT, bool MEMBERS, class Begin, class Emit>
-__device__ __forceinline__ uint32_t group_pass(const GroupArgs& a,
+__device__ __forceinline__ uint64_t group_pass(const GroupArgs& a,
                                                const GroupGeom& G,
                                                GroupLds& s,
                                                const GroupColumn& me,
-                                               uint32_t todo,
+                                               uint64_t todo,
                                                int al,
                                                bool same,
+                                               bool& direct_used,
                                                Begin&& begin,
                                                Emit&& emit)
     {
-    const uint32_t lane = threadIdx.x & 63u, h = lane >> 5, col = lane & 31u;
+    const uint32_t lane = threadIdx.x & 63u, h = lane >> 5;
     int o[3], lo[3], hi[3], anchor[3];
-    bool in = me.valid && same && ((todo >> col) & 1u);
+    bool in = me.valid && same && ((todo >> lane) & 1u);
 #pragma unroll
     for (int k = 0; k < 3; ++k)
         {
         anchor[k] = lane_value(me.c[k], al);
         o[k] = me.c[k] - anchor[k];
         o[k] += 2 * o[k] > G.n[k] ? -G.n[k] : (2 * o[k] < -G.n[k] ? G.n[k] : 0);
-        in = in && o[k] >= -kGroupReach && o[k] <= kGroupReach;
+        // own cells of a pass span at most n - 2 cells: from the middle of
+        // the span every one of their particles is then within L/2 - r_list
+        // (grids of one or two cells take the direct tests)
+        const int below = G.n[k] >= 6 || G.n[k] < 3 ? -kGroupReach : (G.n[k] == 3 ? 0 : -1);
+        const int above = G.n[k] >= 7 || G.n[k] < 3 ? kGroupReach : (G.n[k] < 5 ? 0 : 1);
+        in = in && o[k] >= below && o[k] <= above;
         }
-    // Offsets from the anchor column's position: the difference of two is the
-    // minimum image when the column lies within L/2 - r_list of the anchor on
-    // every axis.  Columns farther away wait for another pass; on grids of
-    // three cells or fewer per axis, where that would leave few columns to a
-    // pass, the group takes the direct tests below.
-    const int fx0 = lane_value(me.fixed.x, al), fy0 = lane_value(me.fixed.y, al), fz0 = lane_value(me.fixed.z, al);
-    const float sx = G.scale[0], sy = G.scale[1], sz = G.scale[2];
-    const float ax = (float)fixed_delta(me.fixed.x, fx0) * sx;
-    const float ay = (float)fixed_delta(me.fixed.y, fy0) * sy;
-    const float az = (float)fixed_delta(me.fixed.z, fz0) * sz;
-    const float margin = a.r_max * 1.0001f;
-    const bool far = !(fabsf(ax) + margin < 0.5f * (float)G.L[0] && fabsf(ay) + margin < 0.5f * (float)G.L[1]
-                       && fabsf(az) + margin < 0.5f * (float)G.L[2]);
-    bool direct = a.direct;
-    if (G.n[0] > 3 && G.n[1] > 3 && G.n[2] > 3)
-        in = in && !far;
-    else
-        direct = direct || __ballot(in && far) != 0ull;
 #pragma unroll
     for (int k = 0; k < 3; ++k)
         {
@@ -211,7 +219,24 @@ __device__ __forceinline__ uint32_t group_pass(const GroupArgs& a,
                 hi[k] = max(hi[k], v);
                 }
         }
-    const uint32_t served = (uint32_t)__ballot(in);
+    const uint64_t served = __ballot(in);
+    // Offsets from the middle of the own cells: the difference of two is the
+    // minimum image when the particle lies within L/2 - r_list of it on every
+    // axis.  Otherwise the pass takes the direct tests below.
+    const float sx = G.scale[0], sy = G.scale[1], sz = G.scale[2];
+    auto middle = [&](int k) {
+        const double f = (anchor[k] + 0.5 * (lo[k] + hi[k] + 1)) / G.n[k] - 0.5; // in box lengths
+        return __builtin_amdgcn_readfirstlane((int)(uint32_t)(unsigned long long)(long long)(f * 4294967296.0));
+    };
+    const int fx0 = middle(0), fy0 = middle(1), fz0 = middle(2);
+    const float ax = (float)fixed_delta(me.fixed.x, fx0) * sx;
+    const float ay = (float)fixed_delta(me.fixed.y, fy0) * sy;
+    const float az = (float)fixed_delta(me.fixed.z, fz0) * sz;
+    const bool far = !(fabsf(ax) + a.r_max < 0.500001f * (float)G.L[0] && fabsf(ay) + a.r_max < 0.500001f * (float)G.L[1]
+                       && fabsf(az) + a.r_max < 0.500001f * (float)G.L[2])
+                     || G.n[0] < 3 || G.n[1] < 3 || G.n[2] < 3;
+    const bool direct = a.direct || __ballot(in && far && (uint32_t)me.fixed.w < a.ntypes) != 0ull;
+    direct_used = direct_used || direct;
     const GroupAxis X(G.n[0], anchor[0], lo[0], hi[0]);
     const GroupAxis Y(G.n[1], anchor[1], lo[1], hi[1]);
     const GroupAxis Z(G.n[2], anchor[2], lo[2], hi[2]);
@@ -223,11 +248,11 @@ __device__ __forceinline__ uint32_t group_pass(const GroupArgs& a,
     // once per cell: by the first of its included columns (slots of a cell are
     // consecutive)
     const uint32_t prev = (uint32_t)__shfl_up((int)me.cell, 1);
-    if (in && (col == 0u || prev != me.cell || !((served >> (col - 1u)) & 1u)))
+    if (in && (lane == 0u || prev != me.cell || !((served >> (lane - 1u)) & 1u)))
         {
         const uint32_t bits = (1u << X.index(X.step(me.c[0], X.n > 1 ? -1 : 0))) | (1u << X.index(me.c[0]))
                               | (1u << X.index(X.step(me.c[0], X.n > 1 ? 1 : 0)));
-        for (uint32_t q = h; q < 9u; q += 2u)
+        for (uint32_t q = 0; q < 9u; ++q)
             {
             const int dy = (int)(q % 3u) - 1, dz = (int)(q / 3u) - 1;
             const int y = Y.index(Y.step(me.c[1], Y.n > 1 ? dy : 0));
@@ -237,8 +262,9 @@ __device__ __forceinline__ uint32_t group_pass(const GroupArgs& a,
         }
     wave_lds_fence();
 
-    // their candidate ranges in ascending cell index: one lane per row of x
-    uint32_t st[kGroupSpan], ct[kGroupSpan];
+    // their candidate ranges in ascending cell index: one lane per row of x,
+    // the reads of a row's cells in flight together
+    uint32_t st[kGroupSpan], ct[kGroupSpan], place[kGroupSpan];
     uint32_t ncell = 0, ncand = 0;
     const bool row_lane = lane < (uint32_t)(Y.len * Z.len);
     const int qz = row_lane ? (int)lane / Y.len : 0, qy = row_lane ? (int)lane % Y.len : 0;
@@ -248,35 +274,35 @@ __device__ __forceinline__ uint32_t group_pass(const GroupArgs& a,
 #pragma unroll
     for (uint32_t q = 0; q < kGroupSpan; ++q)
         {
-        st[q] = ct[q] = 0u;
-        if ((int)q < X.len)
-            {
-            const int cx = X.cell((int)q);
-            if ((bits >> X.index(cx)) & 1u)
-                {
-                const uint32_t c = G.cell_base + (uint32_t)((cz * Y.n + cy) * X.n + cx);
-                const uint32_t r = a.cell_rank ? a.cell_rank[c] : c;
-                st[q] = a.start[r];
-                ct[q] = a.start[r + 1] - st[q];
-                }
-            }
+        const int cx = X.cell(min((int)q, X.len - 1));
+        place[q] = (uint32_t)X.index(cx);
+        const uint32_t c = G.cell_base + (uint32_t)((cz * Y.n + cy) * X.n + cx);
+        st[q] = a.cell_rank ? a.cell_rank[c] : c;
         }
 #pragma unroll
     for (uint32_t q = 0; q < kGroupSpan; ++q)
         {
+        const uint32_t r = st[q];
+        st[q] = a.start[r];
+        ct[q] = a.start[r + 1];
+        }
+#pragma unroll
+    for (uint32_t q = 0; q < kGroupSpan; ++q)
+        {
+        ct[q] = ((int)q < X.len && ((bits >> place[q]) & 1u)) ? ct[q] - st[q] : 0u;
         ncell += ct[q] != 0u ? 1u : 0u;
         ncand += ct[q];
         }
     uint32_t cells, total;
-    uint32_t k0 = wave_exclusive_scan(ncell, lane, cells);
-    uint32_t p0 = wave_exclusive_scan(ncand, lane, total);
+    uint32_t k0 = wave_exclusive_scan(ncell, cells);
+    uint32_t p0 = wave_exclusive_scan(ncand, total);
 #pragma unroll
     for (uint32_t q = 0; q < kGroupSpan; ++q)
         if (ct[q] != 0u)
             {
             s.delta[k0] = st[q] - p0;
             s.first[k0] = p0;
-            s.seq[row * kGroupSpan + (uint32_t)X.index(X.cell((int)q))] = (uint16_t)k0;
+            s.seq[row * kGroupSpan + place[q]] = (uint16_t)k0;
             ++k0;
             p0 += ct[q];
             }
@@ -308,27 +334,36 @@ __device__ __forceinline__ uint32_t group_pass(const GroupArgs& a,
     // below `near_bits`) where FP32 does not decide
     const float c0 = !listed ? 1e30f : (ONEHOT == 0 ? asq - a.thr : asq) - band;
     const int near_bits = __float_as_int(-2.0f * band);
-    f32x16 C;
+    // matrix operands of columns 0..31 (lanes' values of half 0) and 32..63
+    float bxy[2], bzw[2], cc[2];
+    swap_halves(-2.0f * ax, -2.0f * ay, bxy[0], bxy[1]);
+    swap_halves(-2.0f * az, 1.0f, bzw[0], bzw[1]);
+    swap_halves(c0, c0, cc[0], cc[1]);
+    f32x16 C0, C1;
 #pragma unroll
     for (int r = 0; r < 16; ++r)
-        C[r] = c0;
-    const float bxy = h ? -2.0f * ay : -2.0f * ax;
-    const float bzw = h ? 1.0f : -2.0f * az;
-    [[maybe_unused]] float bt[ONEHOT > 0 ? ONEHOT : 1];
+        {
+        C0[r] = cc[0];
+        C1[r] = cc[1];
+        }
+    [[maybe_unused]] float bt[2][ONEHOT > 0 ? ONEHOT : 1];
     if constexpr (ONEHOT > 0)
         {
 #pragma unroll
         for (int t = 0; t < ONEHOT; ++t)
             {
-            const uint32_t tj = 2u * t + h;
-            const double rl = (listed && tj < a.ntypes) ? a.r_listsq[(uint32_t)me.fixed.w * a.ntypes + tj] : 0.0;
-            bt[t] = rl > 0.0 ? -(float)rl : 1e30f;
+            auto radius = [&](uint32_t tj) {
+                const double rl = (listed && tj < a.ntypes) ? a.r_listsq[(uint32_t)me.fixed.w * a.ntypes + tj] : 0.0;
+                return rl > 0.0 ? -(float)rl : 1e30f;
+            };
+            swap_halves(radius(2u * t), radius(2u * t + 1u), bt[0][t], bt[1][t]);
             }
         }
 
     // candidate this lane reads of each 64: rows 8 (r / 4) + 4 h + r % 4 of a
     // 32 x 32 result are registers r of lanes of half h, so half h collects
-    // candidates 32 h .. 32 h + 31 (the direct tests take them in lane order)
+    // candidates 32 h .. 32 h + 31 of a column (the direct tests take them in
+    // lane order)
     const uint32_t off = direct ? lane : 32u * ((lane >> 2) & 1u) + 16u * h + 4u * ((lane >> 3) & 3u) + (lane & 3u);
     const uint64_t upto = (2ull << off) - 1ull;
 
@@ -375,65 +410,74 @@ __device__ __forceinline__ uint32_t group_pass(const GroupArgs& a,
             if (P + 64 < end)
                 fetch(P + 64);
             const bool real = slot != 0xffffffffu && (uint32_t)c.w < a.ntypes;
-            uint32_t mask = 0, near = 0;
+            uint32_t low = 0, high = 0, near_low = 0, near_high = 0;
             if (!direct)
                 {
                 const float x = (float)fixed_delta(c.x, fx0) * sx;
                 const float y = (float)fixed_delta(c.y, fy0) * sy;
                 const float z = (float)fixed_delta(c.z, fz0) * sz;
                 const float w = real ? x * x + y * y + z * z : 1e30f;
-                // both halves of 32 candidates as A operands (k = 0 in lanes
-                // 0..31, k = 1 in lanes 32..63)
-                auto pair_up = [](float p, float q, float& first, float& second) {
-                    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(p), __float_as_uint(q), false, false);
-                    first = __uint_as_float(r[0]);
-                    second = __uint_as_float(r[1]);
-                };
-                float xy0, xy1, zw0, zw1;
-                pair_up(x, y, xy0, xy1);
-                pair_up(z, w, zw0, zw1);
-                f32x16 d0 = __builtin_amdgcn_mfma_f32_32x32x2f32(xy0, bxy, C, 0, 0, 0);
-                f32x16 d1 = __builtin_amdgcn_mfma_f32_32x32x2f32(xy1, bxy, C, 0, 0, 0);
-                d0 = __builtin_amdgcn_mfma_f32_32x32x2f32(zw0, bzw, d0, 0, 0, 0);
-                d1 = __builtin_amdgcn_mfma_f32_32x32x2f32(zw1, bzw, d1, 0, 0, 0);
+                float xy[2], zw[2];
+                swap_halves(x, y, xy[0], xy[1]);
+                swap_halves(z, w, zw[0], zw[1]);
+                [[maybe_unused]] float e[ONEHOT > 0 ? ONEHOT : 1][2];
                 if constexpr (ONEHOT > 0)
                     {
 #pragma unroll
                     for (int t = 0; t < ONEHOT; ++t)
+                        swap_halves(c.w == 2 * t ? 1.0f : 0.0f, c.w == 2 * t + 1 ? 1.0f : 0.0f, e[t][0], e[t][1]);
+                    }
+                uint32_t mask[2], near[2] = {0u, 0u};
+#pragma unroll
+                for (int g = 0; g < 2; ++g)
+                    {
+                    const f32x16& C = g == 0 ? C0 : C1;
+                    f32x16 d0 = __builtin_amdgcn_mfma_f32_32x32x2f32(xy[0], bxy[g], C, 0, 0, 0);
+                    f32x16 d1 = __builtin_amdgcn_mfma_f32_32x32x2f32(xy[1], bxy[g], C, 0, 0, 0);
+                    d0 = __builtin_amdgcn_mfma_f32_32x32x2f32(zw[0], bzw[g], d0, 0, 0, 0);
+                    d1 = __builtin_amdgcn_mfma_f32_32x32x2f32(zw[1], bzw[g], d1, 0, 0, 0);
+                    if constexpr (ONEHOT > 0)
                         {
-                        float e0, e1;
-                        pair_up(c.w == 2 * t ? 1.0f : 0.0f, c.w == 2 * t + 1 ? 1.0f : 0.0f, e0, e1);
-                        d0 = __builtin_amdgcn_mfma_f32_32x32x2f32(e0, bt[t], d0, 0, 0, 0);
-                        d1 = __builtin_amdgcn_mfma_f32_32x32x2f32(e1, bt[t], d1, 0, 0, 0);
+#pragma unroll
+                        for (int t = 0; t < ONEHOT; ++t)
+                            {
+                            d0 = __builtin_amdgcn_mfma_f32_32x32x2f32(e[t][0], bt[g][t], d0, 0, 0, 0);
+                            d1 = __builtin_amdgcn_mfma_f32_32x32x2f32(e[t][1], bt[g][t], d1, 0, 0, 0);
+                            }
+                        }
+                    int least = 0;
+                    uint32_t m = 0;
+#pragma unroll
+                    for (int r = 15; r >= 0; --r)
+                        m = __builtin_amdgcn_alignbit(m, __float_as_uint(d1[r]), 31);
+#pragma unroll
+                    for (int r = 15; r >= 0; --r)
+                        m = __builtin_amdgcn_alignbit(m, __float_as_uint(d0[r]), 31);
+                    mask[g] = m;
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        least = min(min(least, __float_as_int(d0[r])), __float_as_int(d1[r]));
+                    if (__ballot(least < near_bits) != 0ull)
+                        {
+                        uint32_t sure = 0;
+#pragma unroll
+                        for (int r = 15; r >= 0; --r)
+                            sure = __builtin_amdgcn_alignbit(sure, __float_as_uint(d1[r] + 2.0f * band), 31);
+#pragma unroll
+                        for (int r = 15; r >= 0; --r)
+                            sure = __builtin_amdgcn_alignbit(sure, __float_as_uint(d0[r] + 2.0f * band), 31);
+                        near[g] = m & ~sure;
                         }
                     }
-                int least = 0;
-#pragma unroll
-                for (int r = 15; r >= 0; --r)
-                    mask = __builtin_amdgcn_alignbit(mask, __float_as_uint(d1[r]), 31);
-#pragma unroll
-                for (int r = 15; r >= 0; --r)
-                    mask = __builtin_amdgcn_alignbit(mask, __float_as_uint(d0[r]), 31);
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    least = min(least, min(__float_as_int(d0[r]), __float_as_int(d1[r])));
-                if (__ballot(least < near_bits) != 0ull)
-                    {
-                    uint32_t sure = 0;
-#pragma unroll
-                    for (int r = 15; r >= 0; --r)
-                        sure = __builtin_amdgcn_alignbit(sure, __float_as_uint(d1[r] + 2.0f * band), 31);
-#pragma unroll
-                    for (int r = 15; r >= 0; --r)
-                        sure = __builtin_amdgcn_alignbit(sure, __float_as_uint(d0[r] + 2.0f * band), 31);
-                    near = mask & ~sure;
-                    }
+                // both words of the lane's own column
+                swap_halves(mask[0], mask[1], low, high);
+                swap_halves(near[0], near[1], near_low, near_high);
                 }
             else
                 {
-                for (uint32_t m = served; m != 0u; m &= m - 1u)
+                for (uint64_t m = served; m != 0ull; m &= m - 1ull)
                     {
-                    const int q = __builtin_ctz(m);
+                    const int q = __builtin_ctzll(m);
                     const uint32_t tq = (uint32_t)lane_value(me.fixed.w, q);
                     const float x = (float)fixed_delta(c.x, lane_value(me.fixed.x, q)) * sx;
                     const float y = (float)fixed_delta(c.y, lane_value(me.fixed.y, q)) * sy;
@@ -444,22 +488,23 @@ __device__ __forceinline__ uint32_t group_pass(const GroupArgs& a,
                         rl = both ? (float)a.r_listsq[tq * a.ntypes + (uint32_t)c.w] : 0.0f;
                     const float d = (both && rl > 0.0f) ? x * x + y * y + z * z - rl - band : 1e30f;
                     const uint64_t hit = __ballot(d < 0.0f), maybe = __ballot(__float_as_int(d) < near_bits);
-                    if (col == (uint32_t)q)
+                    if (lane == (uint32_t)q)
                         {
-                        mask = h ? (uint32_t)(hit >> 32) : (uint32_t)hit;
-                        near = h ? (uint32_t)(maybe >> 32) : (uint32_t)maybe;
+                        low = (uint32_t)hit;
+                        high = (uint32_t)(hit >> 32);
+                        near_low = (uint32_t)maybe;
+                        near_high = (uint32_t)(maybe >> 32);
                         }
                     }
                 }
-            near = listed ? near : 0u;
-            if (__ballot(near != 0u) != 0ull)
+            if (__ballot((near_low | near_high) != 0u) != 0ull)
                 {
                 // FP32 cannot decide these: the FP64 predicate of the host oracle
-                while (near != 0u)
+                uint64_t near = listed ? (uint64_t)near_high << 32 | near_low : 0ull;
+                while (near != 0ull)
                     {
-                    const uint32_t bit = (uint32_t)__builtin_ctz(near);
-                    near &= near - 1u;
-                    const uint32_t q = 32u * h + bit;
+                    const uint32_t q = (uint32_t)__builtin_ctzll(near);
+                    near &= near - 1ull;
                     const uint32_t run = base + (uint32_t)__popcll(word & ((2ull << q) - 1ull)) - 1u;
                     const uint32_t cs = s.delta[run] + P + q;
                     const uint32_t j = a.members[cs];
@@ -469,12 +514,15 @@ __device__ __forceinline__ uint32_t group_pass(const GroupArgs& a,
                     const double ey = min_image_1d(pi.y - pj.y, G.L[1], G.Linv[1]);
                     const double ez = min_image_1d(pi.z - pj.z, G.L[2], G.Linv[2]);
                     const bool hit = rl > 0.0 && rsq3_nofma(ex, ey, ez) <= rl;
-                    mask = hit ? mask | (1u << bit) : mask & ~(1u << bit);
+                    const uint32_t bit = 1u << (q & 31u);
+                    low = q < 32u ? (hit ? low | bit : low & ~bit) : low;
+                    high = q < 32u ? high : (hit ? high | bit : high & ~bit);
                     }
                 }
-            const uint32_t ds = self - (P + 32u * h);
-            mask &= ds < 32u ? ~(1u << ds) : 0xffffffffu;
-            emit(mask, P, off, MEMBERS ? member : slot);
+            const uint32_t ds = self - P;
+            low &= ds < 32u ? ~(1u << ds) : 0xffffffffu;
+            high &= ds - 32u < 32u ? ~(1u << (ds - 32u)) : 0xffffffffu;
+            emit(low, high, P, off, MEMBERS ? member : slot);
             }
         }
     return served;

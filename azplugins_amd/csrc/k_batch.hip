@@ -95,19 +95,24 @@ __global__ void k_b_bin(const double4* __restrict__ pos,
     if (gated_off(gate))
         return;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N)
+    const uint32_t r = i < N ? rep_of[i] : 0u;
+    const bool active = i < N && rep_flag[r] != 0u;
+    if (__ballot(active) == 0ull)
         return;
-    const uint32_t r = rep_of[i];
-    if (!rep_flag[r])
-        return;
-    const double4 p = pos[i];
-    const RepInfo& R = reps[r];
-    const int cx = cell_coord(p.x, R.L[0], R.Linv[0], R.n[0]);
-    const int cy = cell_coord(p.y, R.L[1], R.Linv[1], R.n[1]);
-    const int cz = cell_coord(p.z, R.L[2], R.Linv[2], R.n[2]);
-    const uint32_t c = R.cell_base + (uint32_t)((cz * R.n[1] + cy) * R.n[0] + cx);
-    cell_of[i] = c;
-    slot_of[i] = atomicAdd(&count[c], 1u);
+    uint32_t c = 0xffffffffu;
+    if (active)
+        {
+        const double4 p = pos[i];
+        const RepInfo& R = reps[r];
+        const int cx = cell_coord(p.x, R.L[0], R.Linv[0], R.n[0]);
+        const int cy = cell_coord(p.y, R.L[1], R.Linv[1], R.n[1]);
+        const int cz = cell_coord(p.z, R.L[2], R.Linv[2], R.n[2]);
+        c = R.cell_base + (uint32_t)((cz * R.n[1] + cy) * R.n[0] + cx);
+        cell_of[i] = c;
+        }
+    const uint32_t at = count_by_runs(c, active, count);
+    if (active)
+        slot_of[i] = at;
     }
 
 __global__ void k_b_scatter(uint32_t N,
@@ -222,36 +227,35 @@ struct BatchWalkArgs
     const uint32_t* rep_flag;
     };
 
-// The flagged replicas' lists: one wavefront per group of 32 consecutive
+// The flagged replicas' lists: one wavefront per group of 64 consecutive
 // cell-list slots (group_walk.h).  The hit masks of up to kWalkBuffer x 64
 // candidates are kept in LDS with the candidates' particle indices and then
-// written out together: lane l < 32 takes the first half of its column's
-// candidates and lane l + 32 the second, one entry per step, so a step stores
-// to two rows of 32 consecutive columns instead of 64 scattered words.
-// Bound by VALU issue (0.75 ms of it) and latency: 1.21 ms for the lists of
-// all 512 replicas of the workload (2.6M particles), 4.76 ms with a lane per
-// particle walking its 27 cells through position gathers in FP64, 1.83 ms with
-// the entries stored to scattered words as they were found.
+// written out together, one entry per lane and step: as long as a group's
+// candidates fit the buffer, a step stores one row of 64 consecutive columns
+// instead of 64 scattered words.  Bound by VALU issue (0.65 ms of it) and
+// latency: 1.20 ms for the lists of all 512 replicas of the workload (2.6M
+// particles), 4.76 ms with a lane per particle walking its 27 cells through
+// position gathers in FP64.  A buffer of 16 (two wavefronts per SIMD) took
+// 1.47 ms.
 constexpr uint32_t kWalkWaves = 4;
-constexpr uint32_t kWalkBuffer = 8;
+constexpr uint32_t kWalkBuffer = 12;
 
-template<int ONEHOT> __global__ void __launch_bounds__(64 * kWalkWaves, 4) k_b_walk(const BatchWalkArgs a)
+template<int ONEHOT> __global__ void __launch_bounds__(64 * kWalkWaves, 3) k_b_walk(const BatchWalkArgs a)
     {
     __shared__ GroupLds s_group[kWalkWaves];
-    __shared__ uint32_t s_mask[kWalkWaves][kWalkBuffer * 64];
+    __shared__ uint32_t s_mask[kWalkWaves][kWalkBuffer * 128];
     __shared__ uint32_t s_j[kWalkWaves][kWalkBuffer * 64];
     if (gated_off(a.gate))
         return;
-    const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63u, h = lane >> 5;
-    const uint32_t group = xcd_logical_block() * (blockDim.x >> 6) + w;
+    const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     GroupColumn me;
-    me.slot = group * 32u + (lane & 31u);
+    me.slot = (xcd_logical_block() * (blockDim.x >> 6) + w) * 64u + lane;
     me.valid = me.slot < a.N;
     me.i = me.valid ? a.g.members[me.slot] : 0u;
     const uint32_t rep = a.rep_of[me.i];
     me.valid = me.valid && a.rep_flag[rep] != 0u;
-    uint32_t todo = (uint32_t)__ballot(me.valid);
-    if (todo == 0u)
+    uint64_t todo = __ballot(me.valid);
+    if (todo == 0ull)
         return; // the whole wavefront (no barrier below spans wavefronts)
     me.cell = a.cell_of[me.i];
     const uint32_t lc = me.valid ? me.cell - a.reps[rep].cell_base : 0u;
@@ -260,59 +264,45 @@ template<int ONEHOT> __global__ void __launch_bounds__(64 * kWalkWaves, 4) k_b_w
     me.c[1] = (int)((lc / (uint32_t)nx) % (uint32_t)ny);
     me.c[2] = (int)(lc / ((uint32_t)nx * (uint32_t)ny));
     me.fixed = a.g.cell_fixed[me.valid ? me.slot : 0u];
-    if (me.valid && h == 0u && (uint32_t)me.fixed.w >= a.g.ntypes)
+    if (me.valid && (uint32_t)me.fixed.w >= a.g.ntypes)
         atomicOr(a.flags + 2, (uint32_t)me.fixed.w == a.g.ntypes ? 1u : 2u);
-    uint32_t count = 0; // entries of the column (in both of its lanes)
-    uint32_t left = 0, held = 0, hold = 0, half = 0; // 64-candidate batches: to come, buffered, to buffer, first half
-    uint32_t first = 0, added = 0; // hits of the buffered batches: of the first half, of all
-    auto next_buffer = [&]() {
-        hold = min(left, kWalkBuffer);
-        half = (hold + 1u) / 2u;
-        held = first = added = 0u;
-    };
-    auto begin = [&](uint32_t, uint32_t total) {
-        left = (total + 63u) / 64u;
-        next_buffer();
-    };
-    auto emit = [&](uint32_t mask, uint32_t, uint32_t off, uint32_t j) {
-        s_mask[w][held * 64u + lane] = mask;
+    uint32_t count = 0;            // entries of the column
+    uint32_t batches = 0, held = 0; // 64-candidate batches to come and buffered
+    uint32_t some = 0;             // words of the buffered batches that are not empty
+    uint32_t* const column = a.nlist + me.i;
+    bool direct = false;
+    auto begin = [&](uint32_t, uint32_t total) { batches = (total + 63u) / 64u; };
+    auto emit = [&](uint32_t low, uint32_t high, uint32_t, uint32_t off, uint32_t j) {
+        s_mask[w][held * 128u + lane] = low;
+        s_mask[w][held * 128u + 64u + lane] = high;
         s_j[w][held * 64u + off] = j;
-        const uint32_t hits = (uint32_t)__popc(mask), both = hits + (uint32_t)__shfl_xor((int)hits, 32);
-        first += held < half ? both : 0u;
-        added += both;
-        if (++held < hold)
+        some |= (low != 0u ? 1u : 0u) << (2u * held) | (high != 0u ? 2u : 0u) << (2u * held);
+        ++held;
+        if (--batches != 0u && held < kWalkBuffer)
             return;
         wave_lds_fence();
-        uint32_t at = count + (h ? first : 0u);
-        uint32_t* dst = a.nlist + (size_t)at * a.pitch + me.i;
-        uint32_t q = h ? 2u * half : 0u, word = 0u, base = 0u;
-        const uint32_t qe = h ? 2u * hold : 2u * half;
-        for (;;)
+        uint32_t word = 0u, base = 0u;
+        while (__ballot((word | some) != 0u) != 0ull)
             {
-            while (word == 0u && q < qe)
-                {
-                base = q * 32u;
-                word = s_mask[w][base + (lane & 31u)];
-                ++q;
-                }
-            if (__ballot(word != 0u) == 0ull)
-                break;
+            const uint32_t q = some != 0u ? (uint32_t)__builtin_ctz(some) : 0u;
+            const uint32_t v = s_mask[w][q * 64u + lane];
+            const bool advance = word == 0u && some != 0u;
+            word = advance ? v : word;
+            base = advance ? q * 32u : base;
+            some = advance ? some & (some - 1u) : some;
             if (word != 0u)
                 {
-                const uint32_t j = s_j[w][base + (uint32_t)__builtin_ctz(word)];
+                const uint32_t n = s_j[w][base + (uint32_t)__builtin_ctz(word)];
                 word &= word - 1u;
-                if (at < a.max_neighbors)
-                    *dst = j;
-                ++at;
-                dst += a.pitch;
+                if (count < a.max_neighbors)
+                    column[(size_t)count * a.pitch] = n;
+                ++count;
                 }
             }
         wave_lds_fence();
-        count += added;
-        left -= hold;
-        next_buffer();
+        held = 0u;
     };
-    while (todo != 0u)
+    while (todo != 0ull)
         {
         const int al = group_anchor(todo);
         const uint32_t r0 = (uint32_t)lane_value((int)rep, al);
@@ -327,9 +317,9 @@ template<int ONEHOT> __global__ void __launch_bounds__(64 * kWalkWaves, 4) k_b_w
             G.scale[k] = R.fx_scale[k];
             }
         G.cell_base = R.cell_base;
-        todo &= ~group_pass<ONEHOT, true>(a.g, G, s_group[w], me, todo, al, rep == r0, begin, emit);
+        todo &= ~group_pass<ONEHOT, true>(a.g, G, s_group[w], me, todo, al, rep == r0, direct, begin, emit);
         }
-    if (me.valid && h == 0u)
+    if (me.valid)
         {
         // a list longer than the capacity is truncated (and reported), so
         // consumers never read past the allocation
@@ -1002,7 +992,7 @@ void enqueue_rebuild(azp_batch* b, hipStream_t s)
     wa.gate = gate;
     wa.rep_flag = rf;
     const unsigned wb = b->tune.walk_block ? b->tune.walk_block : 256;
-    const dim3 walk_grid(grid_for(((size_t)N + 31) / 32, wb / 64));
+    const dim3 walk_grid(grid_for(((size_t)N + 63) / 64, wb / 64));
     bool uniform = true;
     for (double rc : b->r_cut)
         uniform = uniform && rc == b->r_cut[0];

@@ -22,7 +22,7 @@
 //               reruns the walk.
 //   5. columns: rows transposed to nlist[k * pitch + i] (coalesced for
 //               one-lane-per-particle consumers), padded per 64 particles.
-// With tiles enabled, steps 4 and 5 are replaced by the fused per-tile walk
+// With tiles enabled, steps 4 and 5 are replaced by the per-tile walk
 // (k_tile_walk.hip), which writes the tiled list directly; the plain list is
 // expanded from it only when a consumer asks for it.
 // Rebuild check: a particle moved farther than r_buff/2 since the last build.
@@ -48,8 +48,9 @@ __global__ void k_fill_u32(uint32_t* p, uint32_t v, size_t n)
 
 // cell_of[i] is the geometric cell index; the cell's members occupy slots
 // start[cell_rank[c]] .. start[cell_rank[c] + 1] (Morton order of cells).
-// The count is aggregated per wavefront: one atomic per distinct cell among
-// its 64 particles (neighbors in memory usually share a cell).
+// One atomic per run of particles in the same cell, all runs of a wavefront
+// together: 4,096 particles at two a cell took 23 us with one atomic per
+// distinct cell after the other, 3.3 us now.
 __global__ void k_bin(const double4* __restrict__ pos,
                       uint32_t N,
                       DevBox box,
@@ -60,7 +61,6 @@ __global__ void k_bin(const double4* __restrict__ pos,
                       uint32_t* __restrict__ count)
     {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t lane = threadIdx.x & 63u;
     const bool active = i < N;
     uint32_t r = 0xffffffffu;
     if (active)
@@ -73,20 +73,9 @@ __global__ void k_bin(const double4* __restrict__ pos,
         cell_of[i] = c;
         r = cell_rank[c];
         }
-    uint64_t pending = __ballot(active);
-    while (pending != 0ull)
-        {
-        const uint32_t leader = (uint32_t)__ffsll((unsigned long long)pending) - 1u;
-        const uint32_t lr = (uint32_t)__shfl((int)r, (int)leader);
-        const uint64_t same = __ballot(active && r == lr);
-        uint32_t base = 0;
-        if (lane == leader)
-            base = atomicAdd(&count[lr], (uint32_t)__popcll(same));
-        base = (uint32_t)__shfl((int)base, (int)leader);
-        if (active && r == lr)
-            slot_of[i] = base + (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
-        pending &= ~same;
-        }
+    const uint32_t at = count_by_runs(r, active, count);
+    if (active)
+        slot_of[i] = at;
     }
 
 __global__ void k_scatter(uint32_t N,
@@ -376,6 +365,8 @@ __global__ void k_copy_d4(const double4* __restrict__ in, double4* __restrict__ 
 
 using namespace azp;
 
+constexpr uint32_t kHostFlags = 16;
+
 struct azp_nlist
     {
     double r_buff = 0.4;
@@ -395,9 +386,10 @@ struct azp_nlist
     DeviceArray<uint32_t> cell_rank; // Morton rank of each cell of the grid below
     DeviceArray<uint32_t> rank_cell; // its inverse
     int rank_grid[3] = {0, 0, 0};
-    DeviceArray<uint32_t> flags; // [0] overflow, [1] rebuild, [2] bad type, [3] tile misfit, [4] largest tile set,
-                                 // [5] tiles walked in FP32 offsets, [6] the step kernel's check
-    uint32_t* h_flags = nullptr;  // pinned, 8 words ([4], [5] tile build flags)
+    DeviceArray<uint32_t> flags; // [1] rebuild, [6] the step kernel's check, the others as in tiles.h
+    uint32_t* h_flags = nullptr;  // pinned, kHostFlags words ([4], [5] tile build flags)
+    uint32_t group_cells = 0, group_batches = 0; // per group of 64 slots: room of the per-tile walk
+    uint32_t tile_table = kTileTable;            // and of a tile's rank tables
 
     bool want_tiles = false;
     uint32_t tile_mode = 0; // 1: 512 else 256; 256 / 512: that size only
@@ -466,7 +458,7 @@ static int nlist_build(azp_nlist* nl, const azp_particles* p, hipStream_t s)
     AZP_TRY(nl->rank_of.reserve(N));
     AZP_TRY(nl->n_neigh.reserve(N));
     AZP_TRY(nl->last_pos.reserve(N));
-    AZP_TRY(nl->flags.reserve(7));
+    AZP_TRY(nl->flags.reserve(kTileFlags));
 
     if (g.n[0] != nl->rank_grid[0] || g.n[1] != nl->rank_grid[1] || g.n[2] != nl->rank_grid[2])
         {
@@ -508,11 +500,22 @@ static int nlist_build(azp_nlist* nl, const azp_particles* p, hipStream_t s)
             nl->max_neighbors = 8;
         }
     nl->pitch = wave_pitch(N);
+    // room for a group's cells and candidates in the per-tile walk: at first
+    // those of about 72 cells at the mean density, afterwards what a build
+    // needed
+    if (nl->group_cells == 0)
+        {
+        const double per_cell = (double)N / (double)ncell;
+        nl->group_cells = (uint32_t)std::min(512.0, 128.0 + 500.0 / (1.0 + per_cell));
+        nl->group_batches = (uint32_t)std::min((double)kGroupBatchesMax, 6.0 + 72.0 * per_cell / 64.0);
+        }
+    bool uniform = true;
+    for (double rc : nl->r_cut)
+        uniform = uniform && rc == nl->r_cut[0];
 
-    for (int attempt = 0; attempt < 4; ++attempt)
+    for (int attempt = 0; attempt < 6; ++attempt)
         {
         AZP_TRY(nl->list.reserve((size_t)nl->max_neighbors * nl->pitch));
-        AZP_TRY(nl->rows.reserve((size_t)nl->max_neighbors * N));
         nl->tiles.valid = false;
         nl->plain_ready = true;
         nl->fused = false;
@@ -532,37 +535,38 @@ static int nlist_build(azp_nlist* nl, const azp_particles* p, hipStream_t s)
                     continue;
                     }
                 hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, nl->flags.ptr, 0u, (size_t)6);
+                hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, nl->flags.ptr + kTileFlagCells, 0u, (size_t)3);
                 TileWalkArgs ta;
-                ta.pos = pos;
+                ta.g.pos = pos;
+                ta.g.members = nl->members.ptr;
+                ta.g.start = nl->start.ptr;
+                ta.g.cell_rank = nl->cell_rank.ptr;
+                ta.g.cell_fixed = nl->cell_fixed.ptr;
+                ta.g.r_listsq = nl->r_listsq.ptr;
+                ta.g.ntypes = nl->ntypes;
+                ta.g.r_max = (float)rmax;
+                ta.g.thr = (float)(rmax * rmax);
+                ta.g.direct = false;
                 ta.N = N;
                 ta.box = box;
                 for (int k = 0; k < 3; ++k)
                     ta.fx_scale[k] = (float)(box.L[k] / 4294967296.0);
-                ta.g = g;
+                ta.grid = g;
                 ta.cell_of = nl->cell_of.ptr;
-                ta.cell_rank = nl->cell_rank.ptr;
-                ta.rank_cell = nl->rank_cell.ptr;
-                ta.start = nl->start.ptr;
-                ta.members = nl->members.ptr;
-                ta.cell_fixed = nl->cell_fixed.ptr;
-                ta.rank_of = nl->rank_of.ptr;
-                ta.r_listsq = nl->r_listsq.ptr;
-                ta.r_listsq_lo = nl->r_listsq_lo.ptr;
-                ta.r_listsq_hi = nl->r_listsq_hi.ptr;
-                ta.r_list_max = rmax;
-                ta.ntypes = nl->ntypes;
                 ta.n_neigh = nl->n_neigh.ptr;
-                ta.rows = reinterpret_cast<uint16_t*>(nl->rows.ptr);
                 ta.max_neighbors = nl->max_neighbors;
                 ta.flags = nl->flags.ptr;
                 ta.pitch = nl->pitch;
-                AZP_TRY(tiles_walk(nl->tiles, ts, ta, s));
+                ta.group_cell_cap = nl->group_cells;
+                ta.group_batch_cap = nl->group_batches;
+                ta.table_cap = nl->tile_table;
+                AZP_TRY(tiles_walk(nl->tiles, ts, ta, uniform, s));
                 // the positions of this build, queued before the flags are
                 // read so that no host round trip separates it from the walk
                 // (a failed attempt copies them again)
                 hipLaunchKernelGGL(k_copy_d4, dim3(grid_for(N, B)), dim3(B), 0, s, pos, nl->last_pos.ptr, N);
                 AZP_LAUNCH_CHECK();
-                AZP_HIP(hipMemcpyAsync(nl->h_flags, nl->flags.ptr, 6 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+                AZP_HIP(hipMemcpyAsync(nl->h_flags, nl->flags.ptr, kTileFlags * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
                 AZP_HIP(hipStreamSynchronize(s));
                 if (nl->h_flags[2] & 2u)
                     return set_error(AZP_ERR_INVALID, "a particle position is not finite (NaN or inf)");
@@ -570,11 +574,25 @@ static int nlist_build(azp_nlist* nl, const azp_particles* p, hipStream_t s)
                     return set_error(AZP_ERR_INVALID,
                                      "a particle type index is outside [0, %u) (pos.w must hold the type)",
                                      nl->ntypes);
-                if (nl->h_flags[0] != 0u)
+                if (nl->h_flags[kTileFlagBatches] > kGroupBatchesMax)
+                    nl->h_flags[kTileFlagMisfit] |= 2u;
+                else if (nl->h_flags[kTileFlagCells] != 0u || nl->h_flags[kTileFlagBatches] != 0u)
                     {
+                    // a group ran out of room (every count above is valid)
+                    nl->group_cells = std::max(nl->group_cells, nl->h_flags[kTileFlagCells] * 5 / 4);
+                    nl->group_batches = std::min(kGroupBatchesMax,
+                                                 std::max(nl->group_batches, nl->h_flags[kTileFlagBatches] * 5 / 4));
                     grown = true;
-                    break;
                     }
+                if (nl->h_flags[kTileFlagTable] != 0u && nl->h_flags[kTileFlagMisfit] == 0u)
+                    {
+                    nl->tile_table = std::min(kTileTableMax, (nl->h_flags[kTileFlagTable] * 9u / 8u + 511u) & ~511u);
+                    grown = true;
+                    }
+                if (nl->h_flags[0] != 0u)
+                    grown = true;
+                if (grown)
+                    break;
                 if (nl->h_flags[3] == 0u)
                     {
                     nl->tiles.size = ts;
@@ -590,7 +608,8 @@ static int nlist_build(azp_nlist* nl, const azp_particles* p, hipStream_t s)
                 }
             if (grown)
                 {
-                nl->max_neighbors = ((uint32_t)(nl->h_flags[0] * 1.1) + 8u) & ~7u;
+                if (nl->h_flags[0] != 0u)
+                    nl->max_neighbors = ((uint32_t)(nl->h_flags[0] * 1.1) + 8u) & ~7u;
                 continue;
                 }
             if (done)
@@ -602,6 +621,7 @@ static int nlist_build(azp_nlist* nl, const azp_particles* p, hipStream_t s)
                 return AZP_OK;
                 }
             }
+        AZP_TRY(nl->rows.reserve((size_t)nl->max_neighbors * N));
         hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, nl->flags.ptr, 0u, (size_t)3);
         WalkArgs wa;
         wa.pos = pos;
@@ -674,7 +694,7 @@ extern "C" int azp_nlist_create(azp_nlist** out)
     if (!out)
         return set_error(AZP_ERR_INVALID, "null out");
     azp_nlist* nl = new azp_nlist();
-    if (hipHostMalloc((void**)&nl->h_flags, 8 * sizeof(uint32_t), hipHostMallocCoherent) != hipSuccess)
+    if (hipHostMalloc((void**)&nl->h_flags, kHostFlags * sizeof(uint32_t), hipHostMallocCoherent) != hipSuccess)
         {
         nl->h_flags = nullptr;
         delete nl;

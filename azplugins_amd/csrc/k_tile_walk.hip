@@ -1,115 +1,49 @@
-// Fused neighbor walk and tile build.  Tiles are runs of T = 512 or 256
+// Tiled list straight from the cell list.  Tiles are runs of T = 512 or 256
 // consecutive slots of the cell list, whose cells are stored in Morton order,
-// so a tile covers a compact block of space whatever order the particles
-// are in; slot s holds particle members[s].  One workgroup per tile writes
-// the tiled list (tiles.h) straight from the cell list:
+// so a tile covers a compact block of space whatever order the particles are
+// in; slot s holds particle members[s].  Two kernels:
 //
-//   1. union:   the distinct cells of the tile's particles and their 27
-//               neighbor cells, collected in an LDS hash and sorted by Morton
-//               rank; their member counts give each cell's offset in LDS,
-//   2. stage:   the members' fixed-point positions (the cell-ordered copy,
-//               16 bytes each, contiguous per cell) are copied into LDS, so
-//               the tile's candidates are read from global memory once,
-//   3. walk:    each lane tests its particle against the candidates of its
-//               27 cells from LDS (the same FP32 test with the FP64 decision
-//               near r_list as the plain walk, so the pair set is the same)
-//               and appends the candidate's LDS index to its own row of
-//               16-bit entries; then every listed candidate is marked from
-//               the finished rows,
-//   4. compact: an exclusive scan of the marks gives each neighbor its rank
-//               in the tile's neighbor set (Morton cell order), whose
-//               particle indices go to jset,
-//   5. columns: each lane rereads its row and writes ranks two per word in
-//               column s of the tiled list, padded with the tile's count.
+//   k_group_rows     one wavefront per group of 64 slots (group_walk.h): each
+//                    particle's neighbors as numbers among the group's
+//                    candidates, the candidates that any of them lists, and
+//                    the group's cells;
+//   k_tile_compact   one workgroup per tile: the union of its groups' cells
+//                    (LDS hash, sorted into Morton order) numbers the tile's
+//                    candidates; those that are listed get their ranks in the
+//                    tile's neighbor set (jset) by a scan of their marks; a
+//                    table per group turns its candidate numbers into ranks,
+//                    and the columns of the tiled list are written through
+//                    it, ordered by list length.
 //
 // A tile whose cells hold more candidates than LDS does, or whose neighbor
 // set exceeds kTileCap - 1, reports it; the host then uses the plain walk.
+//
+// 1M particles, 139 entries each: k_group_rows 0.56 ms, k_tile_compact 0.32 ms,
+// against 1.27 ms for one kernel in which each lane walked its 27 cells from
+// LDS and appended its hits serially (17 instructions per candidate).  The
+// rows take 12,400 VALU instructions per 64 particles: 5,400 in the tests of
+// 27 batches of 64 candidates, 3,500 in taking 139 entries out of the masks.
+// At 60,000 particles (DPD, density 3) 46 + 37 us against 98, at 4,096 37 + 53
+// against 100.
 #include "cells.h"
 #include "device_common.h"
+#include "group_walk.h"
 #include "tiles.h"
 
 namespace azp
 {
 
-template<uint32_t T> struct TileWalkShape;
-// candidates staged per tile: 96 KB (T = 512) or 64 KB (T = 256) of LDS
-template<> struct TileWalkShape<512>
-    {
-    static constexpr uint32_t cand = 6144;
-    };
-template<> struct TileWalkShape<256>
-    {
-    static constexpr uint32_t cand = 4096;
-    };
-
-constexpr uint32_t kUnionCells = 512; // distinct cells around one tile
+// Candidates of one tile (two bytes of LDS each).
+constexpr uint32_t kTileCand = 6144;
+constexpr uint32_t kUnionCells = 512; // distinct non-empty cells around one tile
 constexpr uint32_t kCellHash = 1024;  // open-addressing table of those cells
-// Per-lane ring of 16 list entries (32 bytes) padded to 40 bytes, so that the
-// lanes' 16-bit appends fall in different LDS banks.
-constexpr uint32_t kRingWords = 10;
-// The tile's own cells are the cells of Morton rank first .. last of its
-// slots; each gets a 27-entry table of its neighbor cells' candidate ranges.
+// A tile whose slots span more cells than this (about four particles a cell
+// or fewer) is left to the plain walk: its union outgrows the hash.
 constexpr uint32_t kOwnCells = 128;
-constexpr uint32_t kNoRange = 0xffffffffu; // a repeated stencil cell (grids narrower than 3)
-// Candidates tested per step of the walk (two steps' reads in flight).
-constexpr uint32_t kWalkBatch = 4;
-constexpr uint16_t kUsed = 0x8000u;    // mark bit beside a 15-bit rank
 
 __device__ __forceinline__ uint32_t cell_hash(uint32_t c)
     {
     return (c * 2654435761u) >> 22; // 10 bits
-    }
-
-// Hash entries: cell index in the high word; once the offsets are known the
-// low word holds the cell's candidate range in LDS (first | end << 16).
-constexpr uint64_t kNoEntry = ~0ull;
-
-// Inserts cell c; returns true when this call added it.  *full is set when
-// the table has no free slot left for it.
-__device__ __forceinline__ bool cell_insert(uint64_t* tab, uint32_t c, bool* full)
-    {
-    const uint64_t key = (uint64_t)c << 32;
-    uint32_t h = cell_hash(c);
-    for (uint32_t p = 0; p < kCellHash; ++p)
-        {
-        const uint64_t prev = atomicCAS(reinterpret_cast<unsigned long long*>(&tab[h]), kNoEntry, key);
-        if (prev == kNoEntry)
-            return true;
-        if ((uint32_t)(prev >> 32) == c)
-            return false;
-        h = (h + 1u) & (kCellHash - 1u);
-        }
-    *full = true;
-    return false;
-    }
-
-// Slot of cell c (present in the table).
-__device__ __forceinline__ uint32_t cell_slot(const uint64_t* tab, uint32_t c)
-    {
-    uint32_t h = cell_hash(c);
-    for (uint32_t p = 0; p < kCellHash; ++p)
-        {
-        if ((uint32_t)(tab[h] >> 32) == c)
-            return h;
-        h = (h + 1u) & (kCellHash - 1u);
-        }
-    return 0u; // not reached: every looked-up cell was inserted
-    }
-
-// Index of the union cell whose candidate range holds m (ranges ascending,
-// the cell's own range non-empty): the largest u < U with off[u] <= m.
-__device__ __forceinline__ uint32_t union_cell_of(const uint32_t* off, uint32_t U, uint32_t m)
-    {
-    uint32_t lo = 0, hi = U;
-    while (hi - lo > 1u)
-        {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (off[mid] <= m)
-            lo = mid;
-        else
-            hi = mid;
-        }
-    return lo;
     }
 
 // Largest value over the 64 lanes of the wavefront (every lane gets it).
@@ -146,336 +80,260 @@ template<uint32_t T> __device__ __forceinline__ uint32_t tile_scan(uint32_t v, u
     return base + x - v;
     }
 
-struct TileWalkLds
+// OR over the wavefront.
+__device__ __forceinline__ uint32_t wave_or(uint32_t v)
     {
-    const int4* cand;
-    uint16_t* mark;
-    const uint32_t* stencil; // 27 candidate ranges (first | end << 16) per own cell
-    const uint32_t* off;
-    const uint32_t* gs; // first cell-list slot of each union cell
-    const float2* lohi; // r_list^2 (1 -+ 1e-5) per type pair (several types)
-    uint32_t U;
-    };
-
-// the fused walk's type-pair table lives in LDS
-constexpr uint32_t kTileWalkTypes = kTileWalkMaxTypes;
-
-// How a tile's candidates are staged and tested.
-enum WalkMode
-    {
-    kWalkFixed = 0,      // wrapped fixed-point positions, r^2 in physical units
-    kWalkFixedCubic = 1, // the same, r^2 in fixed-point units (cubic box)
-    kWalkRelative = 2,   // FP32 offsets from a tile anchor in physical units
-    };
-
-// Lists particle i against the staged candidates; returns its neighbor
-// count.  Entries are LDS candidate indices, appended to the lane's 16-entry
-// LDS ring and stored to its row eight at a time (16 bytes).  Candidates are
-// read four at a time (the staging array has room for the three past a
-// cell's end); the per-candidate tests are branch-free, and only the rare
-// candidates near r_list take the FP64 branch.
-//
-// kWalkRelative: every staged position is its minimum-image offset from the
-// tile's anchor in FP32 (physical units), and the lane's own position is its
-// own staged entry, so a displacement is one FP32 subtraction per axis.  The
-// tile uses it only when all its candidate cells lie within L/4 of the
-// anchor on every axis, where the difference of two such offsets is the
-// minimum image, and within 8 r_list, where the FP32 error of r^2 stays
-// inside the 1e-5 band.
-template<bool SINGLE, int MODE>
-__device__ uint32_t tile_walk_one(const TileWalkArgs& a,
-                                  const TileWalkLds& s,
-                                  uint32_t slot,
-                                  uint32_t i,
-                                  uint32_t own,
-                                  uint32_t* ring)
-    {
-    const double4 pi = a.pos[i];
-    const uint32_t ti = checked_type(pi.w, a.ntypes);
-    const bool finite = isfinite(pi.x) && isfinite(pi.y) && isfinite(pi.z);
-    if (ti == a.ntypes || !finite)
-        {
-        atomicOr(a.flags + 2, finite ? 1u : 2u);
-        return 0;
-        }
-    constexpr bool CUBIC = MODE == kWalkFixedCubic;
-    constexpr bool REL = MODE == kWalkRelative;
-    const int32_t fxi = to_fixed(pi.x, a.box.Linv[0]);
-    const int32_t fyi = to_fixed(pi.y, a.box.Linv[1]);
-    const int32_t fzi = to_fixed(pi.z, a.box.Linv[2]);
-    const float sx = a.fx_scale[0], sy = a.fx_scale[1], sz = a.fx_scale[2];
-    const float unit2 = CUBIC ? 1.0f / (sx * sx) : 1.0f; // r^2 -> fixed-point units^2
-    // the lane's 27 neighbor cells in stencil_axis order; the own cell is the
-    // entry with offset 0 on every axis: the middle one, or the first on an
-    // axis one cell wide (a box of exactly 2 r_list), whose other entries
-    // repeat it and are empty
-    const uint32_t* stencil = s.stencil + own * 27u;
-    const uint32_t own_k = (a.g.n[0] > 1 ? 1u : 0u) + (a.g.n[1] > 1 ? 3u : 0u) + (a.g.n[2] > 1 ? 9u : 0u);
-    const uint32_t own_first = stencil[own_k] & 0xffffu;
-    const uint32_t self = own_first + (slot - s.gs[union_cell_of(s.off, s.U, own_first)]);
-    const int4 me = s.cand[self];
-    const float rxi = __int_as_float(me.x), ryi = __int_as_float(me.y), rzi = __int_as_float(me.z);
-    const double rl0 = a.r_listsq[0];
-    // wave-uniform, held in scalar registers: the candidate loop then never
-    // waits on the vector memory counter (which the row stores also use)
-    const float lo0 = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, a.r_listsq_lo[0])))
-                      * unit2;
-    const float hi0 = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, a.r_listsq_hi[0])))
-                      * unit2;
-    uint16_t* ring16 = reinterpret_cast<uint16_t*>(ring);
-    uint16_t* row = a.rows + (size_t)slot * a.max_neighbors;
-    uint32_t count = 0;
-    // a completed group read from the ring, not yet stored to the row
-    bool pend = false;
-    uint4 pend_data = make_uint4(0u, 0u, 0u, 0u);
-    uint32_t pend_at = 0;
-    auto store_pending = [&]() {
-        if (pend)
-            *reinterpret_cast<uint4*>(row + pend_at) = pend_data;
-        pend = false;
-    };
-    // the next cell's range and first candidates are read one step ahead
-    // one batch: four candidates from m0 (entries past the cell's end masked).
-    // The flags are named scalars, not arrays: an array of flags becomes a
-    // packed byte vector in VGPRs, while scalars stay lane masks.
-    static_assert(kWalkBatch == 4, "the batch below is written out for four candidates");
-    // CHECKED false: the wavefront knows that every lane's four candidates lie
-    // inside its cell and that the cell is not the lane's own (no range or
-    // self test per candidate)
-    auto batch = [&](const int4 (&pc)[kWalkBatch], uint32_t m0, uint32_t e, auto checked) {
-        constexpr bool CHECKED = decltype(checked)::value;
-        // offsets from m0: candidate q is in the range when q < rem and is
-        // the lane's own particle when q == dself (which wraps to a large
-        // value when self < m0)
-        const uint32_t rem = e - m0;
-        const uint32_t dself = self - m0;
-        auto test = [&](const int4& c, uint32_t q, bool& hit, bool& band) {
-            const uint32_t tj = (uint32_t)c.w;
-            // with one type, a candidate of an invalid type can only exist
-            // when its own lane reports it, which fails the build
-            const bool valid = (!CHECKED || ((q < rem) & (q != dself))) & (SINGLE || tj < a.ntypes);
-            const uint32_t tp = SINGLE ? 0u : ti * a.ntypes + min(tj, a.ntypes - 1);
-            const float lo = SINGLE ? lo0 : s.lohi[tp].x * unit2;
-            const float hi = SINGLE ? hi0 : s.lohi[tp].y * unit2;
-            float dx, dy, dz;
-            if constexpr (REL)
-                {
-                dx = __int_as_float(c.x) - rxi;
-                dy = __int_as_float(c.y) - ryi;
-                dz = __int_as_float(c.z) - rzi;
-                }
-            else
-                {
-                dx = (float)fixed_delta(fxi, c.x) * (CUBIC ? 1.0f : sx);
-                dy = (float)fixed_delta(fyi, c.y) * (CUBIC ? 1.0f : sy);
-                dz = (float)fixed_delta(fzi, c.z) * (CUBIC ? 1.0f : sz);
-                }
-            // FP32 rounding here is far inside the 1e-5 band
-            const float rsq = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
-            const bool below = rsq < lo;
-            hit = valid & below;
-            band = valid & !below & (rsq <= hi);
-        };
-        // The FP64 predicate of the host oracle for a candidate FP32 cannot
-        // decide; only the loads are lane-divergent.
-        auto retest = [&](const int4& c, uint32_t q, bool band) {
-            double rsq64 = 0.0, rl = 0.0;
-            if (band)
-                {
-                const uint32_t m = m0 + q;
-                const uint32_t u = union_cell_of(s.off, s.U, m);
-                const uint32_t j = a.members[s.gs[u] + (m - s.off[u])];
-                const double4 p64 = a.pos[j];
-                const uint32_t tp = SINGLE ? 0u : ti * a.ntypes + (uint32_t)c.w;
-                rl = SINGLE ? rl0 : a.r_listsq[tp];
-                const double qx = min_image_1d(pi.x - p64.x, a.box.L[0], a.box.Linv[0]);
-                const double qy = min_image_1d(pi.y - p64.y, a.box.L[1], a.box.Linv[1]);
-                const double qz = min_image_1d(pi.z - p64.z, a.box.L[2], a.box.Linv[2]);
-                rsq64 = rsq3_nofma(qx, qy, qz);
-                }
-            return band & (rsq64 <= rl);
-        };
-        bool h0, h1, h2, h3, b0, b1, b2, b3;
-        test(pc[0], 0u, h0, b0);
-        test(pc[1], 1u, h1, b1);
-        test(pc[2], 2u, h2, b2);
-        test(pc[3], 3u, h3, b3);
-        // taken by the whole wavefront when any lane has such a candidate
-        if (__ballot(b0 | b1 | b2 | b3) != 0ull)
-            {
-            h0 = h0 | retest(pc[0], 0u, b0);
-            h1 = h1 | retest(pc[1], 1u, b1);
-            h2 = h2 | retest(pc[2], 2u, b2);
-            h3 = h3 | retest(pc[3], 3u, b3);
-            }
-        // Append the hits in candidate order.  Every candidate is written to
-        // the ring slot after the last hit; a miss is overwritten by the next
-        // candidate, so the ring needs no per-candidate branch.
-        uint32_t pos = count;
-        auto put = [&](uint32_t q, bool h) {
-            ring16[pos & 15u] = (uint16_t)(m0 + q);
-            pos += h ? 1u : 0u;
-        };
-        put(0u, h0);
-        put(1u, h1);
-        put(2u, h2);
-        put(3u, h3);
-        // A completed group of eight leaves as one 16-byte store.  The ring
-        // is read here, the store is issued after the next batch's reads
-        // (store_pending): waiting for this read right away would also wait
-        // for every LDS access issued before it.
-        if (((pos ^ count) & ~7u) != 0u && count < a.max_neighbors)
-            {
-            const uint2* h = reinterpret_cast<const uint2*>(ring + ((count >> 1) & 4u));
-            const uint2 w0 = h[0], w1 = h[1];
-            pend_data = make_uint4(w0.x, w0.y, w1.x, w1.y);
-            pend_at = count & ~7u;
-            pend = true;
-            }
-        count = pos;
-    };
-    auto load_batch = [&](int4 (&pc)[kWalkBatch], uint32_t m0) {
-#pragma unroll
-        for (uint32_t q = 0; q < kWalkBatch; ++q)
-            pc[q] = s.cand[m0 + q];
-    };
-    // Two batches per iteration in two register sets: the reads of the next
-    // batch are issued before the current one is tested (the scheduling
-    // barriers keep them there), so LDS latency overlaps the tests.
-    uint32_t range_next = stencil[0];
-    for (uint32_t k = 0; k < 27u; ++k)
-        {
-        const uint32_t range = range_next;
-        range_next = stencil[min(k + 1u, 26u)];
-        const uint32_t b = range & 0xffffu, e = range >> 16;
-        int4 pa[kWalkBatch], pb[kWalkBatch];
-        load_batch(pa, b);
-        for (uint32_t m0 = b; m0 < e; m0 += 2 * kWalkBatch)
-            {
-            load_batch(pb, m0 + kWalkBatch);
-            __builtin_amdgcn_sched_barrier(0);
-            store_pending();
-            // both batches whole for every lane still in its cell, and not
-            // the own cell: the tests need no masks
-            if (k != own_k && __ballot(m0 + 2 * kWalkBatch > e) == 0ull)
-                {
-                batch(pa, m0, e, std::false_type{});
-                load_batch(pa, m0 + 2 * kWalkBatch);
-                __builtin_amdgcn_sched_barrier(0);
-                store_pending();
-                batch(pb, m0 + kWalkBatch, e, std::false_type{});
-                continue;
-                }
-            batch(pa, m0, e, std::true_type{});
-            if (m0 + kWalkBatch < e)
-                {
-                load_batch(pa, m0 + 2 * kWalkBatch);
-                __builtin_amdgcn_sched_barrier(0);
-                store_pending();
-                batch(pb, m0 + kWalkBatch, e, std::true_type{});
-                }
-            }
-        }
-    store_pending();
-    if ((count & 7u) != 0u && count < a.max_neighbors)
-        {
-        const uint2* h = reinterpret_cast<const uint2*>(ring + ((count >> 1) & 4u));
-        const uint2 w0 = h[0], w1 = h[1];
-        *reinterpret_cast<uint4*>(row + (count & ~7u)) = make_uint4(w0.x, w0.y, w1.x, w1.y);
-        }
-    return count;
+    // rotations within rows of 16 lanes
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, false);
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xf, 0xf, false);
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x122, 0xf, 0xf, false);
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x121, 0xf, 0xf, false);
+    return (uint32_t)(lane_value((int)v, 0) | lane_value((int)v, 16) | lane_value((int)v, 32) | lane_value((int)v, 48));
     }
 
-template<uint32_t T, bool SINGLE> __global__ void __launch_bounds__(T) k_tile_walk(const TileWalkArgs a)
-    {
-    constexpr uint32_t C = TileWalkShape<T>::cand;
-    __shared__ int4 s_cand[C + 3 * kWalkBatch];
-    __shared__ uint16_t s_mark[C];
-    __shared__ uint64_t s_tab[kCellHash];
-    __shared__ uint64_t s_ucell[kUnionCells];
-    __shared__ uint32_t s_off[kUnionCells + 1];
-    __shared__ uint32_t s_gs[kUnionCells];
-    __shared__ uint32_t s_ring[T * kRingWords];
-    __shared__ uint32_t s_stencil[kOwnCells * 27];
-    __shared__ uint32_t s_wave[T / 64];
-    __shared__ float2 s_lohi[SINGLE ? 1 : kTileWalkTypes * kTileWalkTypes];
-    __shared__ uint32_t s_n, s_bad, s_rfirst, s_rlast, s_ext[3];
+// The neighbors of each particle, by groups of 64 cell-list slots.  A column's
+// mask words that are not empty wait in a ring in LDS, with the number of
+// their first candidate; while some lane's ring is full, and at the end, every
+// lane takes one entry per step from its own, and stores four (8 bytes) at a
+// time: entries stored one by one
+// to scattered rows cost a memory transaction each and took 0.4 of 0.63 ms,
+// and draining whole buffers instead of keeping the ring took 0.70 ms.
+constexpr uint32_t kGroupWaves = 4;
+constexpr uint32_t kRowBuffer = 16; // a power of two
 
-    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+template<int ONEHOT> __global__ void __launch_bounds__(64 * kGroupWaves, 4) k_group_rows(const TileWalkArgs a)
+    {
+    __shared__ GroupLds s_group[kGroupWaves];
+    __shared__ uint32_t s_mask[kGroupWaves][kRowBuffer * 64];
+    __shared__ uint16_t s_first[kGroupWaves][kRowBuffer * 64];
+    const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+    const uint32_t group = xcd_logical_block() * kGroupWaves + w;
+    if (group * 64u >= a.N)
+        return; // the whole wavefront (no barrier below spans wavefronts)
+    GroupColumn me;
+    me.slot = group * 64u + lane;
+    me.valid = me.slot < a.N;
+    me.i = me.valid ? a.g.members[me.slot] : 0u;
+    me.cell = me.valid ? a.cell_of[me.i] : 0u;
+    GroupGeom G;
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+        {
+        G.n[k] = a.grid.n[k];
+        G.L[k] = a.box.L[k];
+        G.Linv[k] = a.box.Linv[k];
+        G.scale[k] = a.fx_scale[k];
+        }
+    G.cell_base = 0u;
+    me.c[0] = (int)(me.cell % (uint32_t)G.n[0]);
+    me.c[1] = (int)((me.cell / (uint32_t)G.n[0]) % (uint32_t)G.n[1]);
+    me.c[2] = (int)(me.cell / ((uint32_t)G.n[0] * (uint32_t)G.n[1]));
+    me.fixed = a.g.cell_fixed[me.valid ? me.slot : 0u];
+    if (me.valid && (uint32_t)me.fixed.w >= a.g.ntypes)
+        {
+        const double4 p = a.g.pos[me.i];
+        atomicOr(a.flags + kTileFlagBad, isfinite(p.x) && isfinite(p.y) && isfinite(p.z) ? 1u : 2u);
+        }
+    // cells and 64-candidate batches of the passes so far; a group that needs
+    // more of either than there is room for reports it and stores nothing
+    uint32_t ncell = 0, nbatch = 0, from = 0;
+    uint32_t pushed = 0, taken = 0;   // words of the column put into its ring, taken from it
+    uint32_t word = 0, base = 0;      // the rest of the last one taken
+    uint32_t count = 0;               // entries of the column
+    uint32_t four_low = 0, four_high = 0; // the last of them, the newest in the high bits
+    bool room = true, direct = false;
+    uint2* cells = a.group_cells + (size_t)group * a.group_cell_cap;
+    uint32_t* used = a.group_used + (size_t)group * a.group_batch_cap * 2u;
+    uint16_t* row = a.group_rows + (size_t)me.slot * a.max_neighbors;
+    // one entry per lane and step until no lane's ring holds more than `keep`
+    // words
+    auto drain = [&](uint32_t keep, bool last) {
+        while (__ballot(pushed - taken > keep || (last && word != 0u)) != 0ull)
+            {
+            const uint32_t at = (taken & (kRowBuffer - 1u)) * 64u + lane;
+            const uint32_t v = s_mask[w][at], n = s_first[w][at];
+            const bool advance = word == 0u && taken != pushed;
+            word = advance ? v : word;
+            base = advance ? n : base;
+            taken += advance ? 1u : 0u;
+            if (word != 0u)
+                {
+                const uint32_t entry = base + (uint32_t)__builtin_ctz(word);
+                word &= word - 1u;
+                four_low = __builtin_amdgcn_alignbit(four_high, four_low, 16);
+                four_high = __builtin_amdgcn_alignbit(entry, four_high, 16);
+                ++count;
+                if ((count & 3u) == 0u && count <= a.max_neighbors)
+                    *reinterpret_cast<uint2*>(row + count - 4u) = make_uint2(four_low, four_high);
+                }
+            }
+    };
+    auto begin = [&](uint32_t n, uint32_t total) {
+        const uint32_t batches = (total + 63u) / 64u;
+        room = room && ncell + n <= a.group_cell_cap && nbatch + batches <= a.group_batch_cap;
+        if (room)
+            for (uint32_t k = lane; k < n; k += 64)
+                {
+                const uint32_t first = s_group[w].first[k];
+                const uint32_t next = k + 1 < n ? s_group[w].first[k + 1] : total;
+                cells[ncell + k] = make_uint2(s_group[w].delta[k] + first, (first + nbatch * 64u) | ((next - first) << 16));
+                }
+        used = a.group_used + ((size_t)group * a.group_batch_cap + nbatch) * 2u;
+        from = nbatch * 64u;
+        ncell += n;
+        nbatch += batches;
+    };
+    auto emit = [&](uint32_t low, uint32_t high, uint32_t P, uint32_t, uint32_t) {
+        if (!room)
+            {
+            count += (uint32_t)(__popc(low) + __popc(high));
+            return;
+            }
+        const uint32_t any_low = wave_or(low), any_high = wave_or(high);
+        if (lane < 2u)
+            used[(P >> 5) + lane] = lane == 0u ? any_low : any_high;
+        // room for two words (a lane reads back only what it wrote itself)
+        drain(kRowBuffer - 2u, false);
+        if (low != 0u)
+            {
+            const uint32_t at = (pushed++ & (kRowBuffer - 1u)) * 64u + lane;
+            s_mask[w][at] = low;
+            s_first[w][at] = (uint16_t)(from + P);
+            }
+        if (high != 0u)
+            {
+            const uint32_t at = (pushed++ & (kRowBuffer - 1u)) * 64u + lane;
+            s_mask[w][at] = high;
+            s_first[w][at] = (uint16_t)(from + P + 32u);
+            }
+    };
+    uint64_t todo = __ballot(me.valid);
+    while (todo != 0ull)
+        todo &= ~group_pass<ONEHOT, false>(a.g, G, s_group[w], me, todo, group_anchor(todo), true, direct, begin, emit);
+    drain(0u, true);
+    // the entries after the last whole four
+    if (me.valid && room && (count & 3u) != 0u && count <= a.max_neighbors)
+        {
+        const uint64_t four = ((uint64_t)four_high << 32 | four_low) >> (16u * (4u - (count & 3u)));
+        *reinterpret_cast<uint2*>(row + (count & ~3u)) = make_uint2((uint32_t)four, (uint32_t)(four >> 32));
+        }
+    if (me.valid)
+        {
+        // a list longer than the capacity is truncated (and reported), so
+        // consumers never read past the allocation
+        a.n_neigh[me.i] = min(count, a.max_neighbors);
+        if (count > a.max_neighbors)
+            atomicMax(a.flags + kTileFlagOverflow, count);
+        }
+    if (lane == 0)
+        {
+        a.group_meta[group] = room ? make_uint2(ncell, nbatch | (direct ? 0x80000000u : 0u)) : make_uint2(0u, 0u);
+        if (!room)
+            {
+            atomicMax(a.flags + kTileFlagCells, ncell);
+            atomicMax(a.flags + kTileFlagBatches, nbatch);
+            }
+        }
+    }
+
+// Distinct neighbors, ranks and columns of each tile.
+template<uint32_t T> __global__ void __launch_bounds__(T, T == 512 ? 4 : 2) k_tile_compact(const TileWalkArgs a)
+    {
+    constexpr uint32_t C = kTileCand;
+    constexpr uint32_t G = T / 64u, NW = T / 64u;
+    // hash of the union's cells: first slots, then (u16) candidate numbers;
+    // the column sort's three arrays once the ranks are known
+    __shared__ uint32_t s_hash[kCellHash + kCellHash / 2];
+    __shared__ uint32_t s_gs[kUnionCells];      // first slot of each union cell
+    __shared__ uint16_t s_off[kUnionCells + 2]; // its first candidate number
+    __shared__ uint16_t s_mark[C];
+    extern __shared__ uint64_t s_ucell[]; // union cells until the rank tables take their place
+    __shared__ uint32_t s_wave[NW], s_nc[G], s_nb[G], s_base[G + 1];
+    __shared__ uint32_t s_n, s_bad, s_direct, s_rfirst, s_rlast;
+    uint32_t* s_key = s_hash;
+    uint16_t* s_val = reinterpret_cast<uint16_t*>(s_hash + kCellHash);
+    uint16_t* s_table = reinterpret_cast<uint16_t*>(s_ucell);
+
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t t = xcd_logical_block();
     const uint32_t slot = t * T + tid;
     const bool active = slot < a.N;
-    const uint32_t nx = (uint32_t)a.g.n[0], ny = (uint32_t)a.g.n[1], nz = (uint32_t)a.g.n[2];
+    const uint32_t g0 = t * G, ng = min(G, (a.N + 63u) / 64u - g0);
+    const uint32_t i = active ? a.g.members[slot] : 0u;
 
     for (uint32_t k = tid; k < kCellHash; k += T)
-        s_tab[k] = kNoEntry;
-    if (!SINGLE)
-        for (uint32_t k = tid; k < a.ntypes * a.ntypes; k += T)
-            s_lohi[k] = make_float2(a.r_listsq_lo[k], a.r_listsq_hi[k]);
+        s_key[k] = 0xffffffffu;
+    for (uint32_t k = tid; k < C; k += T)
+        s_mark[k] = 0u;
     if (tid == 0)
         {
-        s_n = 0u;
-        s_bad = 0u;
-        s_ext[0] = s_ext[1] = s_ext[2] = 0u;
+        s_n = s_bad = s_direct = 0u;
+        s_rfirst = a.g.cell_rank[a.cell_of[i]];
         }
-    __syncthreads();
-
-    // 1. the tile's own cells: Morton ranks first .. last of its slots
-    const uint32_t i = active ? a.members[slot] : 0u;
-    const uint32_t c = active ? a.cell_of[i] : 0u;
-    const uint32_t crank = active ? a.cell_rank[c] : 0u;
-    if (tid == 0)
-        s_rfirst = crank;
     if (active && (tid == T - 1 || slot == a.N - 1))
-        s_rlast = crank;
+        s_rlast = a.g.cell_rank[a.cell_of[i]];
     __syncthreads();
-    const uint32_t r_first = s_rfirst;
-    const uint32_t D = s_rlast - r_first + 1u;
-    if (D > kOwnCells)
+    if (tid < ng)
         {
-        if (tid == 0)
-            atomicOr(a.flags + 3, 8u);
-        return; // D is the same for every thread
-        }
-    // 2. their neighbor cells (periodic) make the union; the stencil table
-    // keeps each neighbor's cell index until the ranges are known, and marks
-    // the offsets that repeat a cell on grids narrower than 3
-    for (uint32_t q = tid; q < D * 27u; q += T)
-        {
-        const uint32_t oc = a.rank_cell[r_first + q / 27u];
-        const uint32_t sidx = q % 27u;
-        const uint32_t dx = sidx % 3u, dy = (sidx / 3u) % 3u, dz = sidx / 9u; // offset + 1
-        if (dx > min(nx, 3u) - 1u || dy > min(ny, 3u) - 1u || dz > min(nz, 3u) - 1u)
-            {
-            s_stencil[q] = kNoRange;
-            continue;
-            }
-        const uint32_t ox = oc % nx, oy = (oc / nx) % ny, oz = oc / (nx * ny);
-        const uint32_t x = (ox + nx + dx - 1u) % nx;
-        const uint32_t y = (oy + ny + dy - 1u) % ny;
-        const uint32_t z = (oz + nz + dz - 1u) % nz;
-        const uint32_t nb = (z * ny + y) * nx + x;
-        s_stencil[q] = nb;
-        bool full = false;
-        if (cell_insert(s_tab, nb, &full))
-            {
-            const uint32_t k = atomicAdd(&s_n, 1u);
-            if (k < kUnionCells)
-                s_ucell[k] = ((uint64_t)a.cell_rank[nb] << 32) | nb;
-            }
-        if (full)
-            s_bad = 1u;
+        const uint2 m = a.group_meta[g0 + tid];
+        s_nc[tid] = m.x;
+        s_nb[tid] = m.y & 0x7fffffffu;
+        if (m.y & 0x80000000u)
+            s_direct = 1u;
         }
     __syncthreads();
-    const uint32_t U = s_n;
-    if (s_bad != 0u || U > kUnionCells)
+    if (tid == 0)
+        {
+        uint32_t b = 0;
+        for (uint32_t g = 0; g < ng; ++g)
+            {
+            s_base[g] = b;
+            b += s_nb[g] * 64u;
+            }
+        s_base[ng] = b;
+        }
+    // 1. the distinct cells of the groups
+    for (uint32_t g = wave; g < ng; g += NW)
+        for (uint32_t k = lane; k < s_nc[g]; k += 64)
+            {
+            const uint2 c = a.group_cells[(size_t)(g0 + g) * a.group_cell_cap + k];
+            uint32_t hs = cell_hash(c.x), p = 0;
+            for (; p < kCellHash; ++p)
+                {
+                const uint32_t prev = atomicCAS(&s_key[hs], 0xffffffffu, c.x);
+                if (prev == 0xffffffffu)
+                    {
+                    const uint32_t u = atomicAdd(&s_n, 1u);
+                    if (u < kUnionCells)
+                        s_ucell[u] = ((uint64_t)c.x << 32) | (hs << 16) | (c.y >> 16);
+                    break;
+                    }
+                if (prev == c.x)
+                    break;
+                hs = (hs + 1u) & (kCellHash - 1u);
+                }
+            if (p == kCellHash)
+                s_bad = 1u;
+            }
+    __syncthreads();
+    const uint32_t U = s_n, entries = s_base[ng];
+    // every thread leaves together: the conditions are shared
+    const uint32_t misfit = (s_rlast - s_rfirst + 1u > kOwnCells ? 8u : 0u) | ((s_bad != 0u || U > kUnionCells) ? 1u : 0u)
+                            | (entries > kTileTableMax ? 2u : 0u);
+    if (misfit != 0u || U == 0u || entries > a.table_cap)
         {
         if (tid == 0)
-            atomicOr(a.flags + 3, 1u);
-        return; // the whole workgroup leaves (U and s_bad are shared)
+            {
+            if (misfit == 0u && U != 0u)
+                atomicMax(a.flags + kTileFlagTable, entries);
+            atomicOr(a.flags + kTileFlagMisfit, misfit);
+            a.tile_count[t] = 0u;
+            }
+        return;
         }
 
-    // Morton order: bitonic sort over the next power of two
+    // 2. in Morton order (ascending first slot): bitonic sort over the next
+    // power of two
     uint32_t P2 = 1;
     while (P2 < U)
         P2 <<= 1;
@@ -537,202 +395,147 @@ template<uint32_t T, bool SINGLE> __global__ void __launch_bounds__(T) k_tile_wa
                 }
         }
 
-    // 2. LDS offsets of the union cells' members; the anchor of the FP32
-    // offsets is the tile's middle particle
-    const uint32_t mid = t * T + (min(T, a.N - t * T) >> 1);
-    const uint32_t anchor_cell = a.cell_of[a.members[mid]];
+    // 3. candidate numbers
     constexpr uint32_t QC = kUnionCells / T;
-    uint32_t cnt[QC];
+    uint64_t cell[QC];
     uint32_t sum = 0;
 #pragma unroll
     for (uint32_t q = 0; q < QC; ++q)
         {
         const uint32_t u = tid * QC + q;
-        cnt[q] = 0u;
-        if (u < U)
-            {
-            const uint32_t r = (uint32_t)(s_ucell[u] >> 32);
-            const uint32_t b = a.start[r];
-            s_gs[u] = b;
-            cnt[q] = a.start[r + 1] - b;
-            // periodic distance in cells from the anchor's cell, per axis
-            const uint32_t cu = (uint32_t)s_ucell[u], ca = anchor_cell;
-            const uint32_t d[3] = {cu % nx > ca % nx ? cu % nx - ca % nx : ca % nx - cu % nx,
-                                   (cu / nx) % ny > (ca / nx) % ny ? (cu / nx) % ny - (ca / nx) % ny
-                                                                   : (ca / nx) % ny - (cu / nx) % ny,
-                                   cu / (nx * ny) > ca / (nx * ny) ? cu / (nx * ny) - ca / (nx * ny)
-                                                                   : ca / (nx * ny) - cu / (nx * ny)};
-            atomicMax(&s_ext[0], min(d[0], nx - d[0]));
-            atomicMax(&s_ext[1], min(d[1], ny - d[1]));
-            atomicMax(&s_ext[2], min(d[2], nz - d[2]));
-            }
-        sum += cnt[q];
+        cell[q] = u < U ? s_ucell[u] : 0ull;
+        sum += (uint32_t)cell[q] & 0xffffu;
         }
     uint32_t Mc;
     uint32_t run = tile_scan<T>(sum, s_wave, Mc);
+    if (Mc > C)
+        {
+        if (tid == 0)
+            {
+            atomicOr(a.flags + kTileFlagMisfit, 2u);
+            a.tile_count[t] = 0u;
+            }
+        return; // Mc is the same for every thread
+        }
 #pragma unroll
     for (uint32_t q = 0; q < QC; ++q)
         {
         const uint32_t u = tid * QC + q;
         if (u < U)
             {
-            const uint32_t cu = (uint32_t)s_ucell[u];
-            s_off[u] = run;
-            // candidate range in the hash entry (Mc <= C < 2^16 is checked below
-            // before any lookup)
-            s_tab[cell_slot(s_tab, cu)] = ((uint64_t)cu << 32) | (run & 0xffffu) | ((run + cnt[q]) << 16);
+            s_gs[u] = (uint32_t)(cell[q] >> 32);
+            s_off[u] = (uint16_t)run;
+            s_val[((uint32_t)cell[q] >> 16) & (kCellHash - 1u)] = (uint16_t)run;
+            run += (uint32_t)cell[q] & 0xffffu;
             }
-        run += cnt[q];
         }
     if (tid == 0)
-        s_off[U] = Mc;
-    if (Mc > C)
-        {
-        if (tid == 0)
-            atomicOr(a.flags + 3, 2u);
-        return; // Mc is the same for every thread
-        }
-    __syncthreads();
-    // FP32 offsets from the anchor (the tile's middle particle) when every
-    // candidate cell is within L/4 of the anchor's cell on every axis (so
-    // differences of offsets are minimum images) and within 8 r_list (so the
-    // FP32 error of r^2, below 6e-8 (13.9 R/r + 6.5) r^2 for offsets up to R,
-    // stays under the 1e-5 band)
-    const double reach = 8.0 * a.r_list_max;
-    const bool rel = (s_ext[0] + 1u) * 4u < nx && (s_ext[1] + 1u) * 4u < ny && (s_ext[2] + 1u) * 4u < nz
-                     && (s_ext[0] + 1u) * a.box.L[0] <= reach * nx && (s_ext[1] + 1u) * a.box.L[1] <= reach * ny
-                     && (s_ext[2] + 1u) * a.box.L[2] <= reach * nz;
-    const int4 anchor = a.cell_fixed[mid];
-    const float sx = a.fx_scale[0], sy = a.fx_scale[1], sz = a.fx_scale[2];
-    auto staged = [&](int4 v) {
-        return rel ? make_int4(__float_as_int((float)fixed_delta(v.x, anchor.x) * sx),
-                               __float_as_int((float)fixed_delta(v.y, anchor.y) * sy),
-                               __float_as_int((float)fixed_delta(v.z, anchor.z) * sz), v.w)
-                   : v;
-    };
-    // stage the candidates: one wavefront per cell, four cells' loads in
-    // flight at a time (cells past 64 members finish in a second loop)
-    constexpr uint32_t NW = T / 64;
-    auto stage_load = [&](uint32_t u) {
-        return (u < U && lane < s_off[u + 1] - s_off[u]) ? a.cell_fixed[s_gs[u] + lane] : make_int4(0, 0, 0, 0);
-    };
-    auto stage_store = [&](uint32_t u, int4 v) {
-        if (u >= U)
-            return;
-        const uint32_t o = s_off[u], n = s_off[u + 1] - o;
-        if (lane < n)
-            s_cand[o + lane] = staged(v);
-        for (uint32_t k = lane + 64; k < n; k += 64)
-            s_cand[o + k] = staged(a.cell_fixed[s_gs[u] + k]);
-    };
-    for (uint32_t u0 = tid >> 6; u0 < U; u0 += 4 * NW)
-        {
-        const int4 v0 = stage_load(u0), v1 = stage_load(u0 + NW);
-        const int4 v2 = stage_load(u0 + 2 * NW), v3 = stage_load(u0 + 3 * NW);
-        stage_store(u0, v0);
-        stage_store(u0 + NW, v1);
-        stage_store(u0 + 2 * NW, v2);
-        stage_store(u0 + 3 * NW, v3);
-        }
-    for (uint32_t m = tid; m < Mc; m += T)
-        s_mark[m] = 0u;
-    for (uint32_t q = tid; q < D * 27u; q += T)
-        {
-        const uint32_t nb = s_stencil[q];
-        s_stencil[q] = nb == kNoRange ? 0u : (uint32_t)s_tab[cell_slot(s_tab, nb)];
-        }
+        s_off[U] = (uint16_t)Mc;
     __syncthreads();
 
-    // 3. walk
-    uint32_t count = 0;
-    if (active)
+    // 4. each group's candidates by tile candidate number: a wavefront a
+    // group, 16 lanes a cell, the next cell read ahead
+    {
+    const uint32_t g = min(wave, ng - 1u);
+    const uint32_t n = wave < ng ? s_nc[g] : 0u;
+    const uint2* src = a.group_cells + (size_t)(g0 + g) * a.group_cell_cap;
+    uint32_t k = lane >> 4;
+    uint2 next = k < n ? src[k] : make_uint2(0u, 0u);
+    for (; k < n; k += 4u)
         {
-        const TileWalkLds s = {s_cand, s_mark, s_stencil, s_off, s_gs, s_lohi, U};
-        uint32_t* ring = s_ring + tid * kRingWords;
-        const bool cubic = a.fx_scale[0] == a.fx_scale[1] && a.fx_scale[0] == a.fx_scale[2];
-        const uint32_t own = crank - r_first;
-        count = rel     ? tile_walk_one<SINGLE, kWalkRelative>(a, s, slot, i, own, ring)
-                : cubic ? tile_walk_one<SINGLE, kWalkFixedCubic>(a, s, slot, i, own, ring)
-                        : tile_walk_one<SINGLE, kWalkFixed>(a, s, slot, i, own, ring);
-        a.n_neigh[i] = min(count, a.max_neighbors);
-        if (count > a.max_neighbors)
-            atomicMax(a.flags, count);
-        // mark the listed candidates, reading the row back in 16-byte chunks
-        // (once per entry here instead of once per tested candidate above)
-        const uint32_t nl = min(count, a.max_neighbors);
-        const uint4* row = reinterpret_cast<const uint4*>(a.rows + (size_t)slot * a.max_neighbors);
-        for (uint32_t k0 = 0; k0 < nl; k0 += 8)
+        const uint2 c = next;
+        if (k + 4u < n)
+            next = src[k + 4u];
+        uint32_t hs = cell_hash(c.x);
+        while (s_key[hs] != c.x) // every cell was inserted
+            hs = (hs + 1u) & (kCellHash - 1u);
+        const uint32_t o = s_val[hs], first = s_base[g] + (c.y & 0xffffu), m = c.y >> 16;
+        for (uint32_t q = tid & 15u; q < m; q += 16u)
+            s_table[first + q] = (uint16_t)(o + q);
+        }
+    }
+    __syncthreads();
+    // 5. marks of the listed ones: a wavefront a group, two words (64
+    // candidates) at a time, 64 words read at once
+    {
+    const uint32_t g = min(wave, ng - 1u);
+    const uint32_t n = wave < ng ? 2u * s_nb[g] : 0u;
+    const uint32_t* src = a.group_used + (size_t)(g0 + g) * a.group_batch_cap * 2u;
+    for (uint32_t q0 = 0; q0 < n; q0 += 64u)
+        {
+        const uint32_t mine = q0 + lane < n ? src[q0 + lane] : 0u;
+        const uint32_t m = min(64u, n - q0);
+        for (uint32_t q = 0; q < m; q += 2u)
             {
-            const uint4 ch = row[k0 / 8];
-            const uint32_t w4[4] = {ch.x, ch.y, ch.z, ch.w};
-#pragma unroll
-            for (uint32_t w = 0; w < 4; ++w)
-                {
-                if (k0 + 2 * w < nl)
-                    s_mark[w4[w] & 0xffffu] = 1u;
-                if (k0 + 2 * w + 1 < nl)
-                    s_mark[w4[w] >> 16] = 1u;
-                }
+            const uint32_t word = (uint32_t)__shfl((int)mine, (int)(q + (lane >> 5)));
+            if ((word >> (lane & 31u)) & 1u)
+                s_mark[s_table[s_base[g] + (q0 + q) * 32u + lane]] = 1u;
             }
         }
+    }
     __syncthreads();
-
-    // 4. ranks of the listed candidates: in-place exclusive scan of the marks
+    // 6. ranks: exclusive scan of the marks; the neighbor set
     constexpr uint32_t QM = C / T;
     uint32_t msum = 0;
 #pragma unroll
     for (uint32_t q = 0; q < QM; ++q)
-        {
-        const uint32_t m = tid * QM + q;
-        msum += (m < Mc && s_mark[m] != 0u) ? 1u : 0u;
-        }
+        msum += s_mark[tid * QM + q];
     uint32_t M;
     uint32_t r = tile_scan<T>(msum, s_wave, M);
+    if (M > kTileCap - 1)
+        {
+        if (tid == 0)
+            {
+            atomicOr(a.flags + kTileFlagMisfit, 4u);
+            a.tile_count[t] = 0u;
+            }
+        return; // M is the same for every thread
+        }
+    // the union cell of the thread's first candidate, then onwards
+    uint32_t lo = 0, hi = U;
+    while (hi - lo > 1u)
+        {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (s_off[mid] <= tid * QM)
+            lo = mid;
+        else
+            hi = mid;
+        }
 #pragma unroll
     for (uint32_t q = 0; q < QM; ++q)
         {
         const uint32_t m = tid * QM + q;
-        if (m < Mc)
+        while (lo + 1u < U && s_off[lo + 1u] <= m)
+            ++lo;
+        if (s_mark[m] != 0u)
             {
-            const bool used = s_mark[m] != 0u;
-            s_mark[m] = (uint16_t)(used ? (kUsed | r) : r);
-            r += used ? 1u : 0u;
-            }
-        }
-    if (M > kTileCap - 1)
-        {
-        if (tid == 0)
-            atomicOr(a.flags + 3, 4u);
-        return; // M is the same for every thread
-        }
-    __syncthreads();
-    for (uint32_t m = tid; m < Mc; m += T)
-        {
-        const uint32_t v = s_mark[m];
-        if (v & kUsed)
-            {
-            const uint32_t lo = union_cell_of(s_off, U, m);
-            a.tile_jset[(size_t)t * kTileCap + (v & ~(uint32_t)kUsed)] = a.members[s_gs[lo] + (m - s_off[lo])];
+            a.tile_jset[(size_t)t * kTileCap + r] = a.g.members[s_gs[lo] + (m - s_off[lo])];
+            s_mark[m] = (uint16_t)(r << 4); // entries are 16 x rank
+            ++r;
             }
         }
     if (tid == 0)
         {
         a.tile_count[t] = M;
-        atomicMax(a.flags + 4, M);
-        if (rel)
-            atomicAdd(a.flags + 5, 1u);
+        atomicMax(a.flags + kTileFlagLargest, M);
+        if (s_direct == 0u)
+            atomicAdd(a.flags + kTileFlagRelative, 1u);
         }
+    __syncthreads();
+    // 7. the tables hold ranks from here on (places past a pass's last
+    // candidate are never read: no mask has their bits)
+    for (uint32_t x = tid; x < entries; x += T)
+        s_table[x] = s_mark[min((uint32_t)s_table[x], C - 1u)];
 
-    // 5. columns ordered by list length (longest first, ties by slot), so the
+    // 8. columns ordered by list length (longest first, ties by slot), so the
     // pair kernel's 64-lane wavefronts run lists of nearly equal length: a
     // bitonic sort of (length, slot) keys, one per thread, whose stages with
-    // a stride below 64 exchange keys within the wavefront (no barrier); the
-    // staging space (free now) carries the others and the slots' particles
-    // and lengths
-    const uint32_t nn = active ? min(count, a.max_neighbors) : 0u;
-    uint32_t* s_sort = reinterpret_cast<uint32_t*>(s_cand);
+    // a stride below 64 exchange keys within the wavefront (no barrier)
+    const uint32_t nn = active ? a.n_neigh[i] : 0u;
+    uint32_t* s_sort = s_hash;
     uint32_t* s_who = s_sort + T;
     uint32_t* s_len = s_who + T;
+    static_assert(3 * T <= kCellHash + kCellHash / 2, "the sort's arrays fit the hash's space");
     s_who[tid] = i;
     s_len[tid] = nn;
     uint32_t key = (min(nn, 0xffffu) << 16) | (0xffffu - tid);
@@ -768,12 +571,16 @@ template<uint32_t T, bool SINGLE> __global__ void __launch_bounds__(T) k_tile_wa
     a.tile_nn[col] = cnn;
     a.tile_order[col] = ci;
     a.tile_col[ci] = col;
-    // the row is reread in 16-byte chunks (8 entries), four in flight
-    const uint4* row = reinterpret_cast<const uint4*>(a.rows + (size_t)(t * T + cslot) * a.max_neighbors);
-    auto chunk_load = [&](uint32_t kc) { return kc < cnn ? row[kc / 8] : make_uint4(0u, 0u, 0u, 0u); };
+    // 9. entries, two a word; the row is read in 16-byte chunks (8 entries),
+    // four in flight.  A group without room stored no rows (its build is
+    // repeated).
+    const uint32_t g = cslot >> 6;
+    const uint32_t have = s_nb[g] != 0u ? cnn : 0u;
+    const uint16_t* tab = s_table + s_base[g];
+    const uint4* row = reinterpret_cast<const uint4*>(a.group_rows + (size_t)(t * T + cslot) * a.max_neighbors);
+    auto chunk_load = [&](uint32_t kc) { return kc < have ? row[kc / 8] : make_uint4(0u, 0u, 0u, 0u); };
     auto rank_of_entry = [&](uint32_t k, uint32_t word, uint32_t half) {
-        const uint32_t m = (word >> (16u * half)) & 0xffffu;
-        return (k < cnn ? (uint32_t)(s_mark[m] & ~kUsed) : M) << 4; // stored as 16 x rank
+        return k < have ? (uint32_t)tab[(word >> (16u * half)) & 0xffffu] : M << 4; // 16 x rank
     };
     auto chunk_store = [&](uint32_t kc, uint4 ch) {
         if (kc >= P)
@@ -781,8 +588,8 @@ template<uint32_t T, bool SINGLE> __global__ void __launch_bounds__(T) k_tile_wa
         const uint32_t w4[4] = {ch.x, ch.y, ch.z, ch.w};
 #pragma unroll
         for (uint32_t w = 0; w < 4; ++w)
-            a.tlist[(size_t)((kc >> 1) + w) * a.pitch + col] =
-                rank_of_entry(kc + 2 * w, w4[w], 0u) | (rank_of_entry(kc + 2 * w + 1, w4[w], 1u) << 16);
+            a.tlist[(size_t)((kc >> 1) + w) * a.pitch + col]
+                = rank_of_entry(kc + 2 * w, w4[w], 0u) | (rank_of_entry(kc + 2 * w + 1, w4[w], 1u) << 16);
     };
     for (uint32_t k0 = 0; k0 < P; k0 += 32)
         {
@@ -829,20 +636,25 @@ __global__ void __launch_bounds__(64) k_tiles_to_plain(uint32_t N,
         }
     }
 
-int tiles_walk(TileList& t, uint32_t tile_size, const TileWalkArgs& args, hipStream_t s)
+int tiles_walk(TileList& t, uint32_t tile_size, const TileWalkArgs& args, bool uniform, hipStream_t s)
     {
     if (tile_size != 256 && tile_size != 512)
         return set_error(AZP_ERR_INVALID, "tile size %u must be 256 or 512", tile_size);
-    if (args.ntypes == 0 || args.ntypes > kTileWalkTypes)
-        return set_error(AZP_ERR_UNSUPPORTED, "the per-tile walk serves 1 to %u particle types", kTileWalkTypes);
+    if (args.g.ntypes == 0 || args.g.ntypes > kTileWalkMaxTypes)
+        return set_error(AZP_ERR_UNSUPPORTED, "the per-tile walk serves 1 to %u particle types", kTileWalkMaxTypes);
     const uint32_t ntiles = (args.N + tile_size - 1) / tile_size;
     const uint32_t words = (((args.max_neighbors + 7u) & ~7u) + 1u) / 2u;
+    const size_t groups = ((size_t)args.N + 63) / 64;
     AZP_TRY(t.count.reserve(ntiles));
     AZP_TRY(t.jset.reserve((size_t)ntiles * kTileCap));
     AZP_TRY(t.list.reserve((size_t)words * args.pitch));
     AZP_TRY(t.nn.reserve(args.N));
     AZP_TRY(t.order_buf.reserve(args.N));
     AZP_TRY(t.col.reserve(args.N));
+    AZP_TRY(t.group_cells.reserve(groups * args.group_cell_cap));
+    AZP_TRY(t.group_rows.reserve((size_t)args.N * args.max_neighbors));
+    AZP_TRY(t.group_used.reserve(groups * args.group_batch_cap * 2));
+    AZP_TRY(t.group_meta.reserve(groups));
     TileWalkArgs a = args;
     a.tile_nn = t.nn.ptr;
     a.tile_order = t.order_buf.ptr;
@@ -850,21 +662,30 @@ int tiles_walk(TileList& t, uint32_t tile_size, const TileWalkArgs& args, hipStr
     a.tile_count = t.count.ptr;
     a.tile_jset = t.jset.ptr;
     a.tlist = t.list.ptr;
-    const bool single = a.ntypes == 1;
-    if (tile_size == 512)
-        {
-        if (single)
-            hipLaunchKernelGGL((k_tile_walk<512, true>), dim3(ntiles), dim3(512), 0, s, a);
-        else
-            hipLaunchKernelGGL((k_tile_walk<512, false>), dim3(ntiles), dim3(512), 0, s, a);
-        }
+    a.group_cells = t.group_cells.ptr;
+    a.group_rows = t.group_rows.ptr;
+    a.group_used = t.group_used.ptr;
+    a.group_meta = t.group_meta.ptr;
+    const dim3 grid(grid_for(groups, kGroupWaves)), block(64 * kGroupWaves);
+    if (uniform)
+        hipLaunchKernelGGL(k_group_rows<0>, grid, block, 0, s, a);
+    else if (a.g.ntypes <= 2)
+        hipLaunchKernelGGL(k_group_rows<1>, grid, block, 0, s, a);
     else
-        {
-        if (single)
-            hipLaunchKernelGGL((k_tile_walk<256, true>), dim3(ntiles), dim3(256), 0, s, a);
-        else
-            hipLaunchKernelGGL((k_tile_walk<256, false>), dim3(ntiles), dim3(256), 0, s, a);
-        }
+        hipLaunchKernelGGL(k_group_rows<4>, grid, block, 0, s, a);
+    if (a.table_cap < kTileTable || a.table_cap > kTileTableMax)
+        return set_error(AZP_ERR_INVALID, "rank tables of %u entries", a.table_cap);
+    // gfx950 gives a workgroup 160 KiB of LDS; set on every launch (a host-side
+    // attribute, no device work), so no switch is shared between threads
+    const size_t lds = (size_t)a.table_cap * sizeof(uint16_t);
+    const void* kernel = tile_size == 512 ? reinterpret_cast<const void*>(&k_tile_compact<512>)
+                                          : reinterpret_cast<const void*>(&k_tile_compact<256>);
+    if (lds > 40 * 1024)
+        AZP_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kTileTableMax * sizeof(uint16_t))));
+    if (tile_size == 512)
+        hipLaunchKernelGGL(k_tile_compact<512>, dim3(ntiles), dim3(512), lds, s, a);
+    else
+        hipLaunchKernelGGL(k_tile_compact<256>, dim3(ntiles), dim3(256), lds, s, a);
     AZP_LAUNCH_CHECK();
     t.ntiles = ntiles;
     t.order = t.order_buf.ptr;

@@ -20,6 +20,7 @@
 
 #include "azp_internal.h"
 #include "cells.h"
+#include "group_walk.h"
 
 namespace azp
 {
@@ -38,6 +39,11 @@ struct TileList
     DeviceArray<uint32_t> nn;        // per-tile walk: list length of column s
     DeviceArray<uint32_t> order_buf; // per-tile walk: particle of column s
     DeviceArray<uint32_t> col;       // per-tile walk: column of particle i
+    // per-tile walk, by group of 64 slots: its cells, how many they are, the
+    // candidates that any of its particles lists, the particles' rows
+    DeviceArray<uint2> group_cells, group_meta;
+    DeviceArray<uint32_t> group_used;
+    DeviceArray<uint16_t> group_rows;
     // Tiles of the per-tile walk: a tile's columns are its cell-list slots
     // reordered by list length (longest first); column s belongs to particle
     // order[s] and has nn[s] entries.  Null for tiles of consecutive
@@ -66,51 +72,62 @@ int tiles_build(TileList& t,
                 uint32_t* h_flag,
                 hipStream_t stream);
 
-// Inputs and outputs of the fused walk (k_tile_walk.hip): the cell list
-// (cell_of, cell_rank, start, members, the cell-ordered fixed-point copy and
-// rank_of) and the list radii as in the plain walk; per-particle counts;
-// 16-bit slot-major rows (entry k of slot s at rows[s * max_neighbors + k],
-// LDS candidate indices) as scratch; the slot-ordered tiled list as output.
+// Flag words of the per-tile walk.
+constexpr uint32_t kTileFlagOverflow = 0; // largest count above max_neighbors
+constexpr uint32_t kTileFlagBad = 2;      // bad type (1) / position (2)
+constexpr uint32_t kTileFlagMisfit = 3;   // a tile did not fit (1: cells, 2: candidates, 4: neighbor set, 8: own cells)
+constexpr uint32_t kTileFlagLargest = 4;  // largest neighbor-set size
+constexpr uint32_t kTileFlagRelative = 5; // tiles tested on the matrix cores throughout
+constexpr uint32_t kTileFlagCells = 7;    // most cells of a group beyond group_cell_cap
+constexpr uint32_t kTileFlagBatches = 8;  // most batches of a group beyond group_batch_cap
+constexpr uint32_t kTileFlagTable = 9;    // most rank-table entries of a tile beyond table_cap
+constexpr uint32_t kTileFlags = 10;       // (word 6 belongs to the step kernel's check)
+
+// Inputs and outputs of the per-tile walk (k_tile_walk.hip): the cell list
+// (cell_of, members, the cell-ordered fixed-point copy) and the list radii;
+// per-particle counts; the groups' rows as scratch; the slot-ordered tiled
+// list as output.
 struct TileWalkArgs
     {
-    const double4* pos;
+    GroupArgs g;
     uint32_t N;
     DevBox box;
     float fx_scale[3]; // L / 2^32 per axis
-    CellGrid g;
-    const uint32_t* cell_of;   // geometric cell of each particle
-    const uint32_t* cell_rank; // Morton rank of each geometric cell
-    const uint32_t* rank_cell; // geometric cell of each Morton rank
-    const uint32_t* start;     // slots of rank r: start[r] .. start[r + 1]
-    const uint32_t* members;
-    const int4* cell_fixed;
-    const uint32_t* rank_of;
-    const double* r_listsq;
-    const float* r_listsq_lo;
-    const float* r_listsq_hi;
-    double r_list_max;
-    uint32_t ntypes;
-    uint32_t* n_neigh;    // by particle
-    uint32_t* tile_nn;    // by column (set by tiles_walk)
-    uint32_t* tile_order; // particle of each column (set by tiles_walk)
-    uint32_t* tile_col;   // column of each particle (set by tiles_walk)
-    uint16_t* rows;       // by slot
-    uint32_t max_neighbors; // a multiple of 8
-    // [0] largest count above max_neighbors, [2] bad type (1) / position (2),
-    // [3] a tile did not fit (1: cells, 2: candidates, 4: neighbor set,
-    // 8: own cells), [4] largest neighbor-set size, [5] tiles walked with
-    // FP32 offsets from their anchor
+    CellGrid grid;
+    const uint32_t* cell_of; // geometric cell of each particle
+    uint32_t* n_neigh;       // by particle
+    uint32_t max_neighbors;  // a multiple of 8
     uint32_t* flags;
+    uint32_t pitch;
+    uint32_t group_cell_cap, group_batch_cap, table_cap;
+    // set by tiles_walk
+    uint2* group_cells;    // by group: first slot, first candidate | members << 16 of each cell
+    uint32_t* group_used;  // by group and batch of 64 candidates: two words
+    uint16_t* group_rows;  // by slot: the candidate numbers of its entries
+    uint2* group_meta;     // by group: cells, batches (high bit: direct tests)
+    uint32_t* tile_nn;     // by column
+    uint32_t* tile_order;  // particle of each column
+    uint32_t* tile_col;    // column of each particle
     uint32_t* tile_count;
     uint32_t* tile_jset;
     uint32_t* tlist;
-    uint32_t pitch;
     };
 
-// Enqueues the fused walk with tiles of `tile_size` (256 or 512) particles
+// Rank-table entries (two bytes of LDS each) of a tile: with kTileTable two
+// tiles share a CU (81 KB each); a build whose tiles need more is repeated
+// with room for them, up to one tile per CU.
+constexpr uint32_t kTileTable = 29696;
+constexpr uint32_t kTileTableMax = 69632;
+
+// Most batches of a group the walk makes room for (beyond it a tile's rank
+// tables do not fit anyway).
+constexpr uint32_t kGroupBatchesMax = 64;
+
+// Enqueues the per-tile walk with tiles of `tile_size` (256 or 512) particles
 // into t's arrays (sized here); the caller reads args.flags afterwards and
-// sets t.size / t.slots / t.valid when flags[3] is clear.
-int tiles_walk(TileList& t, uint32_t tile_size, const TileWalkArgs& args, hipStream_t stream);
+// sets t.size / t.slots / t.valid when no misfit is flagged.  `uniform`: one
+// list radius for every type pair.
+int tiles_walk(TileList& t, uint32_t tile_size, const TileWalkArgs& args, bool uniform, hipStream_t stream);
 
 // Most particle types tiles_walk serves.
 constexpr uint32_t kTileWalkMaxTypes = 8;

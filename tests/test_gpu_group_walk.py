@@ -1,7 +1,7 @@
-"""Group neighbor walk (32 particles and 64 candidates at a time on the matrix
+"""Group neighbor walk (64 particles and 64 candidates at a time on the matrix
 cores): the lists it writes hold the oracle's pairs, each once, where its
 windows, passes and remainders can go wrong — grids of 2 to 9 cells per axis,
-boxes of unequal edges, groups that straddle replicas and grid rows, 1 to 33
+boxes of unequal edges, groups that straddle replicas and grid rows, 1 to 64
 particles, more candidates than one segment, several list radii.
 """
 
@@ -64,7 +64,7 @@ def _check(boxes, sizes, r_cut, seed):
         assert np.array_equal(got[r], _oracle_pairs(box, p, r_cut)), f"replica {r}"
 
 
-@pytest.mark.parametrize("cells", [2, 3, 4, 5, 6, 9])
+@pytest.mark.parametrize("cells", [2, 3, 4, 5, 6, 7, 9])
 def test_group_walk_grids(cells):
     """Cubic and unequal boxes of `cells` cells on the shortest axis."""
     L = cells * RL * (1.0 + 1e-8)
