@@ -8,6 +8,7 @@
 // (i, j) exactly in exact arithmetic (both are dU/dgamma_j (r_hat x n_j)).
 #include <type_traits>
 
+#include "lane_split.h"
 #include "tpm.h"
 
 namespace azp
@@ -33,6 +34,7 @@ struct AnisoKernelArgs
     double4* torque;
     double* virial;
     uint32_t vpitch;
+    uint32_t split; // log2 of the lanes per particle (lane_split.h)
     };
 
 template<bool MIXED, bool VIRIAL, bool SINGLE>
@@ -54,10 +56,13 @@ __global__ void __launch_bounds__(512) k_aniso(const AnisoKernelArgs a)
         __syncthreads();
         }
     const uint32_t lb = xcd_logical_block();
-    const uint32_t i = lb * blockDim.x + threadIdx.x;
+    const uint32_t split = a.split;
+    const SplitLane lane = split_lane(split);
+    const uint32_t columns = blockDim.x >> split;
+    const uint32_t i = lb * columns + lane.column;
     // wavefronts entirely past N leave together; lanes past N in the last
     // wavefront walk no entries and store nothing
-    if (lb * blockDim.x + (threadIdx.x & ~63u) >= a.N)
+    if (lb * columns + ((threadIdx.x >> 6) << (6u - split)) >= a.N)
         return;
     const uint32_t ie = min(i, a.N - 1);
     const AnisoSelf<R> me = aniso_self<MIXED>(a.pos, a.pos_fixed, a.orientation, ie);
@@ -73,9 +78,19 @@ __global__ void __launch_bounds__(512) k_aniso(const AnisoKernelArgs a)
     const uint32_t trips = __builtin_amdgcn_readfirstlane((tpm_wave_max(nn) + 3u) & ~3u);
     const uint32_t* row = a.head_list ? a.nlist + a.head_list[ie] : a.nlist + ie;
     const size_t stride = a.head_list ? 1 : a.nlist_pitch;
-    tpm_list<MIXED, VIRIAL, SINGLE, false>(ie, nn, trips, row, stride, a.pos, a.pos_fixed, a.orientation,
-                                           nullptr, me, box, nt, q0, s_q, acc);
-    if (i < a.N)
+    tpm_list<MIXED, VIRIAL, SINGLE, false>(ie, nn, trips, lane.sub, split, row, stride, a.pos, a.pos_fixed,
+                                           a.orientation, nullptr, me, box, nt, q0, s_q, acc);
+    if (split != 0u)
+        {
+        for (double* v : {&acc.fx, &acc.fy, &acc.fz, &acc.tx, &acc.ty, &acc.tz, &acc.pe})
+            *v = split_sum(*v, split);
+        if (VIRIAL)
+            {
+            for (double* v : {&acc.v0, &acc.v1, &acc.v2, &acc.v3, &acc.v4, &acc.v5})
+                *v = split_sum(*v, split);
+            }
+        }
+    if (i < a.N && lane.sub == 0u)
         aniso_store<VIRIAL>(a.force, a.torque, a.virial, a.vpitch, i, acc);
     }
 
@@ -86,7 +101,8 @@ static int launch_aniso_t(const AnisoKernelArgs& ka, unsigned block, hipStream_t
     const size_t shmem = SINGLE ? 0 : (size_t)ka.ntypes * ka.ntypes * sizeof(TPMPrep<R>);
     if (shmem > 64 * 1024)
         return set_error(AZP_ERR_UNSUPPORTED, "too many particle types for LDS staging");
-    hipLaunchKernelGGL((k_aniso<MIXED, VIRIAL, SINGLE>), dim3(grid_for(ka.N, block)), dim3(block), shmem, s, ka);
+    hipLaunchKernelGGL((k_aniso<MIXED, VIRIAL, SINGLE>), dim3(grid_for((size_t)ka.N << ka.split, block)), dim3(block), shmem,
+                       s, ka);
     AZP_LAUNCH_CHECK();
     return AZP_OK;
     }
@@ -154,6 +170,7 @@ extern "C" int azp_gpu_compute_pair_aniso_forces(const azp_pair_args* args, int 
     ka.torque = reinterpret_cast<double4*>(args->out.d_torque);
     ka.virial = args->out.d_virial;
     ka.vpitch = args->out.virial_pitch;
+    ka.split = split_for(p.N, mixed ? SplitTerm::Light : SplitTerm::Fp64);
     const unsigned block = args->block_size ? args->block_size : 256;
     hipStream_t s = (hipStream_t)args->stream;
     if (mixed && !ka.pos_fixed)

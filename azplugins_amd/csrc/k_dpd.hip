@@ -13,6 +13,7 @@
 // counter (min tag, max tag), so both directed evaluations of a pair draw the
 // same alpha and the pair force stays antisymmetric.
 #include "device_common.h"
+#include "lane_split.h"
 #include "portable_math.h"
 #include "tiles.h"
 
@@ -50,6 +51,8 @@ struct DPDKernelArgs
     const uint32_t* tile_order;
     const uint32_t* tile_nn;
     uint32_t tile_slots;
+    uint32_t split;      // log2 of the lanes per particle (lane_split.h)
+    uint32_t part_shift; // tiled: log2 of the workgroups per tile
     };
 
 // One type pair's parameters with the quantities that depend on the pair
@@ -109,13 +112,32 @@ __device__ __forceinline__ DPDPair make_dpd_pair(const DPDKernelArgs& a, uint32_
     return q;
     }
 
+// The entries of one lane: entry m of its own sequence is list entry at(m).
+// With a split (lane_split.h) the particle's lanes take consecutive fours.
+template<bool SPLIT> struct LaneEntries
+    {
+    uint32_t split, first;
+    __device__ __forceinline__ LaneEntries(uint32_t split_, uint32_t sub) : split(split_), first(4u * sub) { }
+    __device__ __forceinline__ uint32_t at(uint32_t m) const
+        {
+        return SPLIT ? ((m & ~3u) << split) + first + (m & 3u) : m;
+        }
+    __device__ __forceinline__ uint32_t count(uint32_t nn) const
+        {
+        if (!SPLIT)
+            return nn;
+        const uint32_t rest = nn & ((4u << split) - 1u);
+        return ((nn >> (2u + split)) << 2) + (rest > first ? min(rest - first, 4u) : 0u);
+        }
+    };
+
 // LDS_TABLE: the type-pair table is staged in LDS (up to 16 KiB, 17 types);
 // otherwise each in-cut pair derives its entry from the global parameter
 // arrays by the same operations (bit-identical, slower).
 // At least four wavefronts per SIMD (at most 128 VGPRs, a few spilled): the
 // kernel waits on its gathers more than it issues, and the fourth wavefront
 // measured 4 % faster than three without the bound.
-template<bool VIRIAL, bool LDS_TABLE>
+template<bool VIRIAL, bool LDS_TABLE, bool SPLIT>
 __global__ void __launch_bounds__(512, 4) k_dpd(const DPDKernelArgs a)
     {
     extern __shared__ double smem[];
@@ -129,7 +151,9 @@ __global__ void __launch_bounds__(512, 4) k_dpd(const DPDKernelArgs a)
             s_p[t] = make_dpd_pair(a, t);
         }
     __syncthreads();
-    const uint32_t i = xcd_logical_block() * blockDim.x + threadIdx.x;
+    const uint32_t split = SPLIT ? a.split : 0u;
+    const SplitLane lane = SPLIT ? split_lane(split) : SplitLane{threadIdx.x, 0u};
+    const uint32_t i = xcd_logical_block() * (blockDim.x >> split) + lane.column;
     if (i >= a.N)
         return;
     const uint32_t bs = blockDim.x;
@@ -145,7 +169,8 @@ __global__ void __launch_bounds__(512, 4) k_dpd(const DPDKernelArgs a)
     const size_t pitch = a.head_list ? 1 : a.nlist_pitch;
     double fx = 0, fy = 0, fz = 0, pe = 0;
     double v0 = 0, v1 = 0, v2 = 0, v3 = 0, v4 = 0, v5 = 0;
-    const uint32_t nn = a.n_neigh[i];
+    const LaneEntries<SPLIT> mine(split, lane.sub);
+    const uint32_t nn = mine.count(a.n_neigh[i]);
     auto in_cut = [&](const double4& pj) {
         const double dx = min_image_fused(pi.x - pj.x, a.box.L[0], a.box.Linv[0]);
         const double dy = min_image_fused(pi.y - pj.y, a.box.L[1], a.box.Linv[1]);
@@ -158,14 +183,26 @@ __global__ void __launch_bounds__(512, 4) k_dpd(const DPDKernelArgs a)
         {
         // scan: fill the queue with the next in-cut neighbors
         uint32_t cnt = 0;
+        if (SPLIT)
+            {
+            // back to a whole four after a queue that filled within one
+            while ((k & 3u) != 0u && k < nn)
+                {
+                const uint32_t j = row[(size_t)mine.at(k) * pitch];
+                ++k;
+                if (in_cut(a.pos[j]))
+                    q_col[(cnt++) * bs] = j;
+                }
+            }
         while (k + 4 <= nn && cnt + 4 <= qlen)
             {
+            const uint32_t e = mine.at(k);
             uint32_t j0, j1, j2, j3;
             if (pitch == 1)
                 {
                 // consecutive entries (HOOMD's head-list rows): one 16-byte load
                 uint4 w;
-                __builtin_memcpy(&w, row + k, sizeof(w));
+                __builtin_memcpy(&w, row + e, sizeof(w));
                 j0 = w.x;
                 j1 = w.y;
                 j2 = w.z;
@@ -173,10 +210,10 @@ __global__ void __launch_bounds__(512, 4) k_dpd(const DPDKernelArgs a)
                 }
             else
                 {
-                j0 = row[(size_t)k * pitch];
-                j1 = row[(size_t)(k + 1) * pitch];
-                j2 = row[(size_t)(k + 2) * pitch];
-                j3 = row[(size_t)(k + 3) * pitch];
+                j0 = row[(size_t)e * pitch];
+                j1 = row[(size_t)(e + 1) * pitch];
+                j2 = row[(size_t)(e + 2) * pitch];
+                j3 = row[(size_t)(e + 3) * pitch];
                 }
             const double4 p0 = a.pos[j0];
             const double4 p1 = a.pos[j1];
@@ -195,7 +232,7 @@ __global__ void __launch_bounds__(512, 4) k_dpd(const DPDKernelArgs a)
             }
         while (k < nn && cnt < qlen)
             {
-            const uint32_t j = row[(size_t)k * pitch];
+            const uint32_t j = row[(size_t)mine.at(k) * pitch];
             ++k;
             if (in_cut(a.pos[j]))
                 q_col[(cnt++) * bs] = j;
@@ -231,6 +268,18 @@ __global__ void __launch_bounds__(512, 4) k_dpd(const DPDKernelArgs a)
                 }
             }
         }
+    if constexpr (SPLIT)
+        {
+        for (double* v : {&fx, &fy, &fz, &pe})
+            *v = split_sum(*v, split);
+        if (VIRIAL)
+            {
+            for (double* v : {&v0, &v1, &v2, &v3, &v4, &v5})
+                *v = split_sum(*v, split);
+            }
+        if (lane.sub != 0u)
+            return;
+        }
     a.force[i] = make_double4(fx, fy, fz, pe);
     if (VIRIAL)
         {
@@ -244,7 +293,8 @@ __global__ void __launch_bounds__(512, 4) k_dpd(const DPDKernelArgs a)
         }
     }
 
-// DPD over the tiled list (tiles.h): one workgroup per tile stages the FP64
+// DPD over the tiled list (tiles.h): one workgroup (several in small
+// systems, lane_split.h) per tile stages the FP64
 // positions of the tile's neighbor set in LDS (32 bytes a neighbor, the
 // fourth word holding the type and the particle index), so the scan over
 // every list entry reads its neighbors from LDS instead of gathering them
@@ -259,7 +309,7 @@ __global__ void __launch_bounds__(512, 4) k_dpd(const DPDKernelArgs a)
 // Four wavefronts per SIMD, i.e. two 512-lane workgroups per CU (their LDS
 // fits twice), so one workgroup's staging overlaps the other's work; with
 // three (the unbounded register count) it ran slower than the plain kernel.
-template<bool VIRIAL>
+template<bool VIRIAL, bool SPLIT>
 __global__ void __launch_bounds__(512, 4) k_dpd_tiled(const DPDKernelArgs a)
     {
     extern __shared__ double smem[];
@@ -270,12 +320,15 @@ __global__ void __launch_bounds__(512, 4) k_dpd_tiled(const DPDKernelArgs a)
     uint16_t* s_q = reinterpret_cast<uint16_t*>(s_p + nt * nt);
     const uint32_t lb = xcd_logical_block();
     const uint32_t bs = blockDim.x;
-    const uint32_t* js = a.tile_jset + (size_t)lb * kTileCap;
+    const uint32_t split = SPLIT ? a.split : 0u;
+    const SplitLane lane = SPLIT ? split_lane(split) : SplitLane{threadIdx.x, 0u};
+    const uint32_t tile = SPLIT ? lb >> a.part_shift : lb;
+    const uint32_t* js = a.tile_jset + (size_t)tile * kTileCap;
     // slot m: the neighbor's x, y, z and, in the fourth word, its type (low
     // half) and particle index (high half), so the evaluation gathers its
     // velocity and tag without reading the neighbor set again
     stage_slots<8>(
-        a.tile_count[lb], js,
+        a.tile_count[tile], js,
         [&](uint32_t j) {
             double4 p = a.pos[j];
             p.w = __hiloint2double((int)j, (int)(uint32_t)p.w);
@@ -285,11 +338,12 @@ __global__ void __launch_bounds__(512, 4) k_dpd_tiled(const DPDKernelArgs a)
     for (uint32_t t = threadIdx.x; t < nt * nt; t += bs)
         s_p[t] = make_dpd_pair(a, t);
     __syncthreads();
-    const uint32_t ie = lb * bs + threadIdx.x;
+    const uint32_t ie = lb * (bs >> split) + lane.column;
     if (ie >= a.N)
         return;
     const uint32_t pe = a.tile_order ? a.tile_order[ie] : ie;
-    const uint32_t nn = a.tile_order ? a.tile_nn[ie] : a.n_neigh[ie];
+    const LaneEntries<SPLIT> mine(split, lane.sub);
+    const uint32_t nn = mine.count(a.tile_order ? a.tile_nn[ie] : a.n_neigh[ie]);
     uint16_t* q_col = s_q + threadIdx.x;
     const uint32_t qlen = a.queue_len;
     const double4 pi = a.pos[pe];
@@ -309,7 +363,8 @@ __global__ void __launch_bounds__(512, 4) k_dpd_tiled(const DPDKernelArgs a)
         const double rsq = dx * dx + dy * dy + dz * dz;
         return rsq < rc_row[(uint32_t)__double2loint(pj.w) * rc_stride];
     };
-    auto rank_at = [&](uint32_t kk) {
+    auto rank_at = [&](uint32_t m) {
+        const uint32_t kk = mine.at(m);
         const uint32_t w = col[(size_t)(kk >> 1) * pitch];
         return ((kk & 1u) ? (w >> 16) : (w & 0xffffu)) >> 4;
     };
@@ -319,9 +374,9 @@ __global__ void __launch_bounds__(512, 4) k_dpd_tiled(const DPDKernelArgs a)
         // scan: fill the queue with the next in-cut neighbors.  A full queue
         // can stop the scan at an odd entry; one single step then realigns k
         // to a word, so the four-entry steps read entries k .. k + 3 as two
-        // whole words.
+        // whole words (with a split, to one of the lane's own fours).
         uint32_t cnt = 0;
-        if (k & 1u)
+        while ((k & (SPLIT ? 3u : 1u)) != 0u && k < nn)
             {
             const uint32_t r = rank_at(k);
             ++k;
@@ -330,8 +385,9 @@ __global__ void __launch_bounds__(512, 4) k_dpd_tiled(const DPDKernelArgs a)
             }
         while (k + 4 <= nn && cnt + 4 <= qlen)
             {
-            const uint32_t w0 = col[(size_t)(k >> 1) * pitch];
-            const uint32_t w1 = col[(size_t)((k >> 1) + 1) * pitch];
+            const uint32_t kw = mine.at(k) >> 1;
+            const uint32_t w0 = col[(size_t)kw * pitch];
+            const uint32_t w1 = col[(size_t)(kw + 1) * pitch];
             const uint32_t r0 = (w0 & 0xffffu) >> 4, r1 = w0 >> 20;
             const uint32_t r2 = (w1 & 0xffffu) >> 4, r3 = w1 >> 20;
             const bool c0 = in_cut(s_pos[r0]), c1 = in_cut(s_pos[r1]);
@@ -385,6 +441,18 @@ __global__ void __launch_bounds__(512, 4) k_dpd_tiled(const DPDKernelArgs a)
                 }
             }
         }
+    if constexpr (SPLIT)
+        {
+        for (double* v : {&fx, &fy, &fz, &pe_sum})
+            *v = split_sum(*v, split);
+        if (VIRIAL)
+            {
+            for (double* v : {&v0, &v1, &v2, &v3, &v4, &v5})
+                *v = split_sum(*v, split);
+            }
+        if (lane.sub != 0u)
+            return;
+        }
     a.force[pe] = make_double4(fx, fy, fz, pe_sum);
     if (VIRIAL)
         {
@@ -431,6 +499,38 @@ __global__ void k_dpd_alpha(uint16_t seed,
 
 int validate_common(const azp_pair_args* args);
 
+template<bool VIRIAL, bool LDS_TABLE>
+static int launch_dpd(const DPDKernelArgs& ka, dim3 grid, unsigned block, size_t shmem, hipStream_t s)
+    {
+    if (ka.split != 0)
+        hipLaunchKernelGGL((k_dpd<VIRIAL, LDS_TABLE, true>), grid, dim3(block), shmem, s, ka);
+    else
+        hipLaunchKernelGGL((k_dpd<VIRIAL, LDS_TABLE, false>), grid, dim3(block), shmem, s, ka);
+    AZP_LAUNCH_CHECK();
+    return AZP_OK;
+    }
+
+template<bool VIRIAL, bool SPLIT>
+static int launch_dpd_tiled(const DPDKernelArgs& ka, dim3 grid, unsigned block, size_t shmem, hipStream_t s)
+    {
+    if (shmem > 64 * 1024)
+        {
+        // more than 64 KiB of dynamic LDS (gfx950 gives a workgroup 160 KiB)
+        static bool raised = false;
+        if (!raised)
+            {
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_dpd_tiled<VIRIAL, SPLIT>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDpdTileLds);
+            if (e != hipSuccess)
+                return set_error(AZP_ERR_HIP, "hipFuncSetAttribute (dynamic LDS) failed: %s", hipGetErrorString(e));
+            raised = true;
+            }
+        }
+    hipLaunchKernelGGL((k_dpd_tiled<VIRIAL, SPLIT>), grid, dim3(block), shmem, s, ka);
+    AZP_LAUNCH_CHECK();
+    return AZP_OK;
+    }
+
 } // namespace azp
 
 using namespace azp;
@@ -465,6 +565,7 @@ extern "C" int azp_gpu_compute_dpd_forces(const azp_pair_args* args, const void*
     ka.force = reinterpret_cast<double4*>(args->out.d_force);
     ka.virial = args->out.d_virial;
     ka.vpitch = args->out.virial_pitch;
+    ka.split = split_for(p.N, SplitTerm::Light);
     hipStream_t s = (hipStream_t)args->stream;
     if (args->d_tile_list && !args->d_head_list && dpd_tile_fits(args->ntypes, args->tile_slots, args->tile_size))
         {
@@ -478,32 +579,20 @@ extern "C" int azp_gpu_compute_dpd_forces(const azp_pair_args* args, const void*
         ka.tile_nn = args->d_tile_nn;
         ka.tile_slots = args->tile_slots;
         ka.queue_len = kDpdTileQueue;
-        const size_t shmem = dpd_tile_lds(args->ntypes, args->tile_slots, args->tile_size, kDpdTileQueue);
-        if (shmem > 64 * 1024)
-            {
-            // more than 64 KiB of dynamic LDS (gfx950 gives a workgroup 160 KiB)
-            static bool raised = false;
-            if (!raised)
-                {
-                for (const void* f : {reinterpret_cast<const void*>(&k_dpd_tiled<true>),
-                                      reinterpret_cast<const void*>(&k_dpd_tiled<false>)})
-                    {
-                    const hipError_t e
-                        = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDpdTileLds);
-                    if (e != hipSuccess)
-                        return set_error(AZP_ERR_HIP, "hipFuncSetAttribute (dynamic LDS) failed: %s",
-                                         hipGetErrorString(e));
-                    }
-                raised = true;
-                }
-            }
-        const dim3 grid(grid_for(p.N, args->tile_size));
+        // a split tile's lanes in workgroups of up to 512, each staging the
+        // tile's neighbors for its own columns
+        unsigned block = std::min(512u, (unsigned)args->tile_size << ka.split);
+        if (dpd_tile_lds(args->ntypes, args->tile_slots, block, kDpdTileQueue) > kDpdTileLds)
+            block = args->tile_size;
+        while ((block << ka.part_shift) < (args->tile_size << ka.split))
+            ++ka.part_shift;
+        const size_t shmem = dpd_tile_lds(args->ntypes, args->tile_slots, block, kDpdTileQueue);
+        const dim3 grid(grid_for(p.N, args->tile_size) << ka.part_shift);
         if (args->compute_virial)
-            hipLaunchKernelGGL((k_dpd_tiled<true>), grid, dim3(args->tile_size), shmem, s, ka);
-        else
-            hipLaunchKernelGGL((k_dpd_tiled<false>), grid, dim3(args->tile_size), shmem, s, ka);
-        AZP_LAUNCH_CHECK();
-        return AZP_OK;
+            return ka.split ? launch_dpd_tiled<true, true>(ka, grid, block, shmem, s)
+                            : launch_dpd_tiled<true, false>(ka, grid, block, shmem, s);
+        return ka.split ? launch_dpd_tiled<false, true>(ka, grid, block, shmem, s)
+                        : launch_dpd_tiled<false, false>(ka, grid, block, shmem, s);
         }
     if (!args->d_nlist)
         return set_error(AZP_ERR_INVALID, "the DPD kernel reads the plain list (d_nlist) when no tiled list fits");
@@ -519,23 +608,11 @@ extern "C" int azp_gpu_compute_dpd_forces(const azp_pair_args* args, const void*
     if (ka.queue_len < 4)
         return set_error(AZP_ERR_INVALID, "DPD block size too large");
     const size_t shmem = table + (size_t)ka.queue_len * block * sizeof(uint32_t);
-    const dim3 grid(grid_for(p.N, block));
-    if (args->compute_virial)
-        {
-        if (lds_table)
-            hipLaunchKernelGGL((k_dpd<true, true>), grid, dim3(block), shmem, s, ka);
-        else
-            hipLaunchKernelGGL((k_dpd<true, false>), grid, dim3(block), shmem, s, ka);
-        }
-    else
-        {
-        if (lds_table)
-            hipLaunchKernelGGL((k_dpd<false, true>), grid, dim3(block), shmem, s, ka);
-        else
-            hipLaunchKernelGGL((k_dpd<false, false>), grid, dim3(block), shmem, s, ka);
-        }
-    AZP_LAUNCH_CHECK();
-    return AZP_OK;
+    const dim3 grid(grid_for((size_t)p.N << ka.split, block));
+    const bool vir = args->compute_virial != 0;
+    if (lds_table)
+        return vir ? launch_dpd<true, true>(ka, grid, block, shmem, s) : launch_dpd<false, true>(ka, grid, block, shmem, s);
+    return vir ? launch_dpd<true, false>(ka, grid, block, shmem, s) : launch_dpd<false, false>(ka, grid, block, shmem, s);
     }
 
 extern "C" int azp_gpu_dpd_alpha(uint16_t seed,

@@ -3,7 +3,7 @@
 // Replaces the launcher instantiated per evaluator at
 // PotentialPairGPUKernel.cu.inc:25-28 (gpu_compute_pair_forces<Eval>).
 //
-// Layout: one lane per particle i, walking its full neighbor list
+// Layout: one lane per particle i (several in small systems), walking its full neighbor list
 // nlist[k * pitch + i] — consecutive lanes read consecutive words, so the
 // list stream is fully coalesced.  Per-type-pair constants (cutoff, hoisted
 // energy shift, parameter products) live in LDS; with one particle type they

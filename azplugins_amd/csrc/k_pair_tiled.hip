@@ -1,6 +1,6 @@
 // Isotropic pair forces over the tiled list (gfx950).
 //
-// One workgroup per tile of 512 (or 256) consecutive cell-list slots: the
+// One workgroup (several in small systems, lane_split.h) per tile of 512 (or 256) consecutive cell-list slots: the
 // tile's distinct neighbors are staged in LDS (fixed-point int4 in the mixed
 // form, the FP64 double4 positions in the plain form) and each lane walks its
 // particle's 16-bit entries (16 x the neighbor's rank in the tile) reading

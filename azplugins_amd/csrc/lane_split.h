@@ -1,0 +1,85 @@
+// Several lanes per particle, for systems too small to fill the chip with one.
+//
+// The pair kernels give a particle one lane when there are enough particles:
+// 256 CUs hold 262,144 lanes at four wavefronts a SIMD.  Below that the time
+// is one lane's walk over its list, a serial chain that idle SIMDs don't
+// shorten, so the list is dealt to 2^split lanes in batches of U entries
+// (lane `sub` of a particle takes batches sub, sub + 2^split, ...), and their
+// FP64 sums are added in a fixed tree at the end.  The lanes of a particle lie
+// 64 >> split apart in one wavefront, so the list words that a wavefront reads
+// for one batch stay consecutive.
+//
+// The split depends on the number of particles and the pair term alone, so
+// every list layout adds a particle's terms in the same order.
+#pragma once
+
+#include "device_common.h"
+
+namespace azp
+{
+
+// Lanes that a split fills the chip up to, by what a list entry costs.  Light
+// terms (the mixed form, DPD's scan) stop at four wavefronts a SIMD, since
+// each further workgroup of a tile stages the tile's neighbors again.  FP64
+// terms, whose registers leave two or three wavefronts a SIMD, take the second
+// lane for up to 229,376 particles: at 262,144 over the plain list it cost a
+// fifth.  Colloid's three divergent branches fill twice as many lanes.
+// Measured with 2^18 / 2^19 lanes (us): mixed PerturbedLJ 60,000 particles
+// 37.4 / 52.2, DPD 60,000 30.2 / 40.3, FP64 Yukawa 60,000 70.2 / 91.4 but
+// 150,000 162 / 142, FP64 TwoPatchMorse 130,000 98 / 105 but 200,000
+// 172 / 155, Colloid 20,000 56 / 51, 73,000 176 / 121 and 200,000 354 / 310
+// (332 with 2^20).  Against one lane per particle: Yukawa 900 particles
+// 85 -> 14.5, Colloid 73,000 200 -> 118, TwoPatchMorse 40,000 66 -> 38 and
+// DPD 60,000 37.5 -> 26.8.
+enum class SplitTerm
+    {
+    Light,
+    Fp64,
+    Colloid,
+    };
+constexpr uint32_t kSplitLanes = 1u << 18;
+constexpr uint32_t kSplitMax = 4;
+
+// log2 of the lanes per particle.
+inline uint32_t split_for(uint32_t N, SplitTerm term)
+    {
+    uint32_t split = 0;
+    while (split < kSplitMax)
+        {
+        const uint32_t lanes = term == SplitTerm::Colloid                ? 2 * kSplitLanes
+                               : term == SplitTerm::Fp64 && split == 0 ? kSplitLanes / 4 * 7
+                                                                       : kSplitLanes;
+        if (((uint64_t)N << (split + 1)) > lanes)
+            break;
+        ++split;
+        }
+    return split;
+    }
+
+// The workgroup-local column and the lane of that column that a lane is: a
+// workgroup covers blockDim.x >> split columns, a wavefront 64 >> split.
+struct SplitLane
+    {
+    uint32_t column;
+    uint32_t sub;
+    };
+
+__device__ __forceinline__ SplitLane split_lane(uint32_t split)
+    {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t shift = 6u - split;
+    SplitLane s;
+    s.column = ((threadIdx.x >> 6) << shift) + (lane & ((1u << shift) - 1u));
+    s.sub = lane >> shift;
+    return s;
+    }
+
+// Sum over a particle's lanes, the same value in each of them.
+__device__ __forceinline__ double split_sum(double v, uint32_t split)
+    {
+    for (uint32_t m = 32; m >= (64u >> split); m >>= 1)
+        v += __shfl_xor(v, (int)m);
+    return v;
+    }
+
+} // namespace azp

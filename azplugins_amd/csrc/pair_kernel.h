@@ -6,9 +6,9 @@
 // Replaces the launcher instantiated per evaluator at
 // PotentialPairGPUKernel.cu.inc:25-28 (gpu_compute_pair_forces<Eval>).
 //
-// Layout: one lane per particle i, walking its full neighbor list
-// nlist[k * pitch + i] — consecutive lanes read consecutive words, so the
-// list stream is fully coalesced.  Per-type-pair constants (cutoff, hoisted
+// Layout: one lane per particle i (several in small systems, lane_split.h),
+// walking its full neighbor list nlist[k * pitch + i] — consecutive lanes read
+// consecutive words, so the list stream is fully coalesced.  Per-type-pair constants (cutoff, hoisted
 // energy shift, parameter products) live in LDS; with one particle type they
 // are held in registers.  Force, energy and the six virial components are
 // accumulated in FP64 registers and written once (no atomics; every lane owns
@@ -28,6 +28,7 @@
 #include <type_traits>
 
 #include "evaluators.h"
+#include "lane_split.h"
 #include "tiles.h"
 
 namespace azp
@@ -67,6 +68,8 @@ struct PairKernelArgs
     const uint32_t* tile_order;
     const uint32_t* tile_nn;
     uint32_t tile_slots; // LDS position slots of the tiled kernel (the tables follow them)
+    uint32_t split;      // log2 of the lanes per particle (lane_split.h)
+    uint32_t part_shift; // tiled: log2 of the workgroups per tile
     // head-list layout: particle i's entries at nlist[head_list[i] + k], k < n_neigh[i]
     const uint64_t* head_list;
     // mixed form: add every entry's terms to the FP64 accumulators
@@ -410,6 +413,23 @@ template<class Eval> static bool tile_fits64(uint32_t ntypes, uint32_t slots)
     }
 
 
+template<bool VIRIAL> __device__ __forceinline__ void split_sum(Acc& acc, uint32_t split)
+    {
+    acc.fx = split_sum(acc.fx, split);
+    acc.fy = split_sum(acc.fy, split);
+    acc.fz = split_sum(acc.fz, split);
+    acc.e = split_sum(acc.e, split);
+    if (VIRIAL)
+        {
+        acc.v0 = split_sum(acc.v0, split);
+        acc.v1 = split_sum(acc.v1, split);
+        acc.v2 = split_sum(acc.v2, split);
+        acc.v3 = split_sum(acc.v3, split);
+        acc.v4 = split_sum(acc.v4, split);
+        acc.v5 = split_sum(acc.v5, split);
+        }
+    }
+
 // Neighbor-list layouts a kernel instance reads.
 constexpr int kLayoutColumn = 0; // nlist[k * pitch + i], padded with i
 constexpr int kLayoutTiled = 1;  // per-tile 16-bit entries (mixed form)
@@ -418,7 +438,7 @@ constexpr int kLayoutHead = 2;   // HOOMD's head list: nlist[head_list[i] + k], 
 // ACC64 (mixed form only): every list entry's FP32 terms are added to the
 // FP64 accumulators as they come, instead of being summed in FP32 over 32
 // entries first.
-template<class Eval, bool MIXED, bool VIRIAL, bool SINGLE, bool XPLOR, bool CUBIC, int LAYOUT, bool ACC64>
+template<class Eval, bool MIXED, bool VIRIAL, bool SINGLE, bool XPLOR, bool CUBIC, int LAYOUT, bool ACC64, bool SPLIT>
 __global__ void __launch_bounds__(512) k_pair(const PairKernelArgs a)
     {
     constexpr bool TILED = LAYOUT == kLayoutTiled;
@@ -453,17 +473,22 @@ __global__ void __launch_bounds__(512) k_pair(const PairKernelArgs a)
         }
 
     const uint32_t lb = xcd_logical_block();
+    const uint32_t split = SPLIT ? a.split : 0u;
+    const SplitLane me = SPLIT ? split_lane(split) : SplitLane{threadIdx.x, 0u};
+    const uint32_t columns = blockDim.x >> split; // of this workgroup
+    const uint32_t i = lb * columns + me.column;
+    [[maybe_unused]] const uint32_t tile = SPLIT ? lb >> a.part_shift : lb;
     int4* s_pos = nullptr;
     const uint32_t* tile_js = nullptr;
     uint32_t tile_m = 0;
     if constexpr (TILED && MIXED)
         {
         // stage the tile's neighbor positions, converted to fixed point here
-        // (block lb is tile lb); every lane of the workgroup takes part before
+        // (2^part_shift workgroups share a tile); every lane of the workgroup takes part before
         // any wavefront may leave.  Slot M is the padding entries' dummy.
         s_pos = reinterpret_cast<int4*>(smem);
-        tile_js = a.tile_jset + (size_t)lb * kTileCap;
-        tile_m = a.tile_count[lb];
+        tile_js = a.tile_jset + (size_t)tile * kTileCap;
+        tile_m = a.tile_count[tile];
         stage_slots<8>(
             tile_m, tile_js, [&](uint32_t j) { return a.pos[j]; },
             [&](uint32_t m, const double4& p) { s_pos[m] = fixed4(p, a.box); });
@@ -474,8 +499,8 @@ __global__ void __launch_bounds__(512) k_pair(const PairKernelArgs a)
         {
         // FP64 form: the FP64 positions themselves (x, y, z in 24-byte slots
         // with one type, x, y, z, type in 32-byte slots otherwise)
-        tile_js = a.tile_jset + (size_t)lb * kTileCap;
-        tile_m = a.tile_count[lb];
+        tile_js = a.tile_jset + (size_t)tile * kTileCap;
+        tile_m = a.tile_count[tile];
         // extent of the staged positions and of the tile's own particles
         TileExtent ext;
         auto track = [&](const double4& p) { ext.add(p.x, p.y, p.z); };
@@ -505,9 +530,8 @@ __global__ void __launch_bounds__(512) k_pair(const PairKernelArgs a)
             if (threadIdx.x == 0)
                 s_pos64[tile_m] = make_double4(0.0, 0.0, 0.0, 0.0);
             }
-        const uint32_t i0 = lb * blockDim.x + threadIdx.x;
-        if (i0 < a.N)
-            track(a.pos[a.tile_order != nullptr ? a.tile_order[i0] : i0]);
+        if (i < a.N)
+            track(a.pos[a.tile_order != nullptr ? a.tile_order[i] : i]);
         ext.store_wave(s_ext);
         }
     if (!SINGLE || TILED)
@@ -519,10 +543,9 @@ __global__ void __launch_bounds__(512) k_pair(const PairKernelArgs a)
     if constexpr (TILED && !MIXED)
         wrap = wrap_axes(s_ext, a.box.L);
 
-    const uint32_t i = lb * blockDim.x + threadIdx.x;
     // wavefronts entirely past N leave together; lanes past N in the last
     // wavefront shadow particle N-1 (same column, results not stored)
-    if (lb * blockDim.x + (threadIdx.x & ~63u) >= a.N)
+    if (lb * columns + ((threadIdx.x >> 6) << (6u - split)) >= a.N)
         return;
     const uint32_t ie = min(i, a.N - 1);
     // slot-ordered tiles: column ie belongs to particle pe
@@ -532,6 +555,11 @@ __global__ void __launch_bounds__(512) k_pair(const PairKernelArgs a)
     // wave-uniform trip count, held in a scalar register
     const uint32_t P = __builtin_amdgcn_readfirstlane((wave_max(nn) + U - 1) & ~(U - 1));
     const size_t stride = a.nlist_pitch;
+    // a particle's 2^split lanes take SU consecutive entries per step; this
+    // lane's are the U from k0 on
+    const uint32_t SU = U << split;
+    const uint32_t k0 = me.sub * U;
+    const bool writes = i < a.N && me.sub == 0u;
 
     Acc acc;
     if constexpr (!MIXED && TILED)
@@ -541,11 +569,11 @@ __global__ void __launch_bounds__(512) k_pair(const PairKernelArgs a)
         // bit-identical to the plain form over the same entries
         const double4 pi = a.pos[pe];
         const uint32_t ti = (uint32_t)pi.w;
-        const uint32_t col_off = ie * 4u;
+        const uint32_t col_off = (ie + (k0 >> 1) * a.nlist_pitch) * 4u;
         const uint32_t tile_m16 = tile_m << 4; // the padding entry
         const char* s_base = reinterpret_cast<const char*>(smem);
         // below F every lane of the wavefront has U real entries per step
-        const uint32_t F = __builtin_amdgcn_readfirstlane(wave_min(nn) & ~(U - 1));
+        const uint32_t F = __builtin_amdgcn_readfirstlane(wave_min(nn) & ~(SU - 1));
         auto step = [&](uint32_t k, auto padded) {
             constexpr bool PADDED = decltype(padded)::value;
             uint32_t w[U / 2];
@@ -612,21 +640,27 @@ __global__ void __launch_bounds__(512) k_pair(const PairKernelArgs a)
                 }
         };
         uint32_t k = 0;
-        for (; k < F; k += U)
+        for (; k < F; k += SU)
             step(k, std::false_type{});
-        for (; k < P; k += U)
-            step(k, std::true_type{});
-        if (i < a.N)
+        for (; k < P; k += SU)
+            {
+            if (!SPLIT || k + k0 < P)
+                step(k, std::true_type{});
+            }
+        if constexpr (SPLIT)
+            split_sum<VIRIAL>(acc, split);
+        if (writes)
             store<VIRIAL>(a, pe, acc);
         }
     else if constexpr (!MIXED)
         {
         const double4 pi = a.pos[ie];
         const uint32_t ti = (uint32_t)pi.w;
-        const uint32_t* hrow = HEAD ? a.nlist + a.head_list[ie] : nullptr;
+        const uint32_t col_off = HEAD ? 0u : (ie + k0 * a.nlist_pitch) * 4u;
+        const uint32_t* hrow = HEAD ? a.nlist + a.head_list[ie] + k0 : nullptr;
         // head list: below F every lane has U entries left in its row, read as
         // 16-byte vectors (one lane's row is contiguous; lanes' rows are not)
-        const uint32_t F = HEAD ? __builtin_amdgcn_readfirstlane(wave_min(nn) & ~(U - 1)) : 0u;
+        const uint32_t F = HEAD ? __builtin_amdgcn_readfirstlane(wave_min(nn) & ~(SU - 1)) : 0u;
         auto step = [&](uint32_t k, auto whole) {
             uint32_t jj[U];
             if constexpr (HEAD && decltype(whole)::value)
@@ -637,9 +671,12 @@ __global__ void __launch_bounds__(512) k_pair(const PairKernelArgs a)
                 for (uint32_t u = 0; u < U; ++u)
                     {
                     if constexpr (HEAD)
-                        jj[u] = k + u < nn ? hrow[k + u] : ie; // rows are not padded
+                        jj[u] = k + k0 + u < nn ? hrow[k + u] : ie; // rows are not padded
                     else
-                        jj[u] = (a.nlist + (size_t)(k + u) * stride)[ie];
+                        {
+                        const char* row = reinterpret_cast<const char*>(a.nlist + (size_t)(k + u) * stride);
+                        jj[u] = *reinterpret_cast<const uint32_t*>(row + col_off);
+                        }
                     }
                 }
             double4 pj[U];
@@ -658,22 +695,27 @@ __global__ void __launch_bounds__(512) k_pair(const PairKernelArgs a)
                 }
         };
         uint32_t k = 0;
-        for (; k < F; k += U)
+        for (; k < F; k += SU)
             step(k, std::true_type{});
-        for (; k < P; k += U)
-            step(k, std::false_type{});
-        if (i < a.N)
+        for (; k < P; k += SU)
+            {
+            if (!SPLIT || k + k0 < P)
+                step(k, std::false_type{});
+            }
+        if constexpr (SPLIT)
+            split_sum<VIRIAL>(acc, split);
+        if (writes)
             store<VIRIAL>(a, i, acc);
         }
     else if constexpr (TILED)
         {
         const int4 pi = fixed4(a.pos[pe], a.box);
         const uint32_t ti = (uint32_t)pi.w;
-        const uint32_t col_off = ie * 4u;
+        const uint32_t col_off = (ie + (k0 >> 1) * a.nlist_pitch) * 4u;
         const uint32_t tile_m16 = tile_m << 4; // the padding entry
         // below F every lane of the wavefront has U real entries per step:
         // those steps skip the padding test
-        const uint32_t F = __builtin_amdgcn_readfirstlane(wave_min(nn) & ~(U - 1));
+        const uint32_t F = __builtin_amdgcn_readfirstlane(wave_min(nn) & ~(SU - 1));
         Acc32 part;
         auto step = [&](uint32_t k, auto padded) {
             constexpr bool PADDED = decltype(padded)::value;
@@ -709,18 +751,30 @@ __global__ void __launch_bounds__(512) k_pair(const PairKernelArgs a)
                     part = Acc32();
                     }
                 }
-            if (!ACC64 && (((k + U) & (kFlushEntries - 1)) == 0 || k + U >= P))
+        };
+        // after a step: the FP32 sums of kFlushEntries entries to FP64
+        auto flush = [&](uint32_t k) {
+            if (!ACC64 && (((k + SU) & ((kFlushEntries << split) - 1u)) == 0 || k + SU >= P))
                 {
                 flush32<VIRIAL>(acc, part);
                 part = Acc32();
                 }
         };
         uint32_t k = 0;
-        for (; k < F; k += U)
+        for (; k < F; k += SU)
+            {
             step(k, std::false_type{});
-        for (; k < P; k += U)
-            step(k, std::true_type{});
-        if (i < a.N)
+            flush(k);
+            }
+        for (; k < P; k += SU)
+            {
+            if (!SPLIT || k + k0 < P)
+                step(k, std::true_type{});
+            flush(k);
+            }
+        if constexpr (SPLIT)
+            split_sum<VIRIAL>(acc, split);
+        if (writes)
             store_scaled<VIRIAL>(a, pe, acc);
         }
     else
@@ -729,12 +783,12 @@ __global__ void __launch_bounds__(512) k_pair(const PairKernelArgs a)
         const uint32_t ti = (uint32_t)pi.w;
         // 32-bit byte offsets from wave-uniform bases (global loads with an
         // SGPR base and a VGPR offset: no per-entry 64-bit address math)
-        const uint32_t col_off = ie * 4u;
+        const uint32_t col_off = HEAD ? 0u : (ie + k0 * a.nlist_pitch) * 4u;
         const char* pf_base = reinterpret_cast<const char*>(a.pos_fixed);
-        const uint32_t* hrow = HEAD ? a.nlist + a.head_list[ie] : nullptr;
+        const uint32_t* hrow = HEAD ? a.nlist + a.head_list[ie] + k0 : nullptr;
         // head list: below F every lane has U entries left in its row, read as
         // 16-byte vectors
-        const uint32_t F = HEAD ? __builtin_amdgcn_readfirstlane(wave_min(nn) & ~(U - 1)) : 0u;
+        const uint32_t F = HEAD ? __builtin_amdgcn_readfirstlane(wave_min(nn) & ~(SU - 1)) : 0u;
         Acc32 part;
         auto step = [&](uint32_t k, auto whole) {
             uint32_t jj[U];
@@ -747,7 +801,7 @@ __global__ void __launch_bounds__(512) k_pair(const PairKernelArgs a)
                     {
                     if constexpr (HEAD)
                         {
-                        jj[u] = k + u < nn ? hrow[k + u] : ie; // rows are not padded
+                        jj[u] = k + k0 + u < nn ? hrow[k + u] : ie; // rows are not padded
                         }
                     else
                         {
@@ -774,22 +828,58 @@ __global__ void __launch_bounds__(512) k_pair(const PairKernelArgs a)
                     part = Acc32();
                     }
                 }
-            if (!ACC64 && (((k + U) & (kFlushEntries - 1)) == 0 || k + U >= P))
+        };
+        // after a step: the FP32 sums of kFlushEntries entries to FP64
+        auto flush = [&](uint32_t k) {
+            if (!ACC64 && (((k + SU) & ((kFlushEntries << split) - 1u)) == 0 || k + SU >= P))
                 {
                 flush32<VIRIAL>(acc, part);
                 part = Acc32();
                 }
         };
         uint32_t k = 0;
-        for (; k < F; k += U)
+        for (; k < F; k += SU)
+            {
             step(k, std::true_type{});
-        for (; k < P; k += U)
-            step(k, std::false_type{});
-        if (i < a.N)
+            flush(k);
+            }
+        for (; k < P; k += SU)
+            {
+            if (!SPLIT || k + k0 < P)
+                step(k, std::false_type{});
+            flush(k);
+            }
+        if constexpr (SPLIT)
+            split_sum<VIRIAL>(acc, split);
+        if (writes)
             store_scaled<VIRIAL>(a, i, acc);
         }
     }
 
+
+template<class Eval, bool MIXED, bool VIRIAL, bool SINGLE, bool XPLOR, bool CUBIC, int LAYOUT, bool ACC64, bool SPLIT>
+static int launch_k(const PairKernelArgs& kb, unsigned grid, unsigned block, size_t shmem, hipStream_t stream)
+    {
+    constexpr auto kernel = &k_pair<Eval, MIXED, VIRIAL, SINGLE, XPLOR, CUBIC, LAYOUT, ACC64, SPLIT>;
+    if (shmem > 64 * 1024)
+        {
+        // more than 64 KiB of dynamic LDS (gfx950 gives a workgroup 160 KiB):
+        // only the FP64 tiled form stages that much
+        static bool raised = false;
+        if (!raised)
+            {
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTileLds64);
+            if (e != hipSuccess)
+                return set_error(AZP_ERR_HIP, "hipFuncSetAttribute (dynamic LDS %zu bytes) failed: %s", kTileLds64,
+                                 hipGetErrorString(e));
+            raised = true;
+            }
+        }
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(block), shmem, stream, kb);
+    AZP_LAUNCH_CHECK();
+    return AZP_OK;
+    }
 
 template<class Eval, bool MIXED, bool VIRIAL, bool SINGLE, bool XPLOR, bool CUBIC, int LAYOUT>
 static int launch_t(const PairKernelArgs& ka, unsigned block, unsigned slots, hipStream_t stream)
@@ -805,31 +895,27 @@ static int launch_t(const PairKernelArgs& ka, unsigned block, unsigned slots, hi
     const size_t cap = (TILED && !MIXED) ? kTileLds64 : kTileLds;
     if (shmem > cap)
         return set_error(AZP_ERR_UNSUPPORTED, "too many particle types (%u) for LDS staging", ka.ntypes);
-    if (shmem > 64 * 1024)
-        {
-        // more than 64 KiB of dynamic LDS (gfx950 gives a workgroup 160 KiB)
-        static bool raised = false;
-        if (!raised)
-            {
-            // only the FP64 tiled form (ACC64 false) stages more than 64 KiB
-            const hipError_t e = hipFuncSetAttribute(
-                reinterpret_cast<const void*>(&k_pair<Eval, MIXED, VIRIAL, SINGLE, XPLOR, CUBIC, LAYOUT, false>),
-                hipFuncAttributeMaxDynamicSharedMemorySize, (int)cap);
-            if (e != hipSuccess)
-                return set_error(AZP_ERR_HIP, "hipFuncSetAttribute (dynamic LDS %zu bytes) failed: %s", cap,
-                                 hipGetErrorString(e));
-            raised = true;
-            }
-        }
-    const unsigned grid = grid_for(ka.N, block);
-    if (MIXED && ka.acc64)
-        hipLaunchKernelGGL((k_pair<Eval, MIXED, VIRIAL, SINGLE, XPLOR, CUBIC, LAYOUT, MIXED>), dim3(grid), dim3(block),
-                           shmem, stream, kb);
-    else
-        hipLaunchKernelGGL((k_pair<Eval, MIXED, VIRIAL, SINGLE, XPLOR, CUBIC, LAYOUT, false>), dim3(grid), dim3(block),
-                           shmem, stream, kb);
-    AZP_LAUNCH_CHECK();
-    return AZP_OK;
+    kb.split = split_for(ka.N, std::is_same_v<Eval, EvalColloid> ? SplitTerm::Colloid
+                               : MIXED                           ? SplitTerm::Light
+                                                                 : SplitTerm::Fp64);
+    // the lanes' 32-bit byte offsets into the list reach over a step's rows
+    while (kb.split != 0 && ((uint64_t)ka.nlist_pitch << (kb.split + 6)) > 0xffffffffull)
+        --kb.split;
+    // tiled: up to 512 lanes a workgroup, and as many workgroups as the tile's
+    // lanes take, each staging the tile's neighbors for its own columns
+    const unsigned tile = block;
+    if (TILED)
+        block = std::min(512u, tile << kb.split);
+    kb.part_shift = 0;
+    while (TILED && (block << kb.part_shift) < (tile << kb.split))
+        ++kb.part_shift;
+    const unsigned grid = TILED ? grid_for(ka.N, tile) << kb.part_shift : grid_for((size_t)ka.N << kb.split, block);
+    const bool acc64 = MIXED && ka.acc64;
+    if (kb.split != 0)
+        return acc64 ? launch_k<Eval, MIXED, VIRIAL, SINGLE, XPLOR, CUBIC, LAYOUT, MIXED, true>(kb, grid, block, shmem, stream)
+                     : launch_k<Eval, MIXED, VIRIAL, SINGLE, XPLOR, CUBIC, LAYOUT, false, true>(kb, grid, block, shmem, stream);
+    return acc64 ? launch_k<Eval, MIXED, VIRIAL, SINGLE, XPLOR, CUBIC, LAYOUT, MIXED, false>(kb, grid, block, shmem, stream)
+                 : launch_k<Eval, MIXED, VIRIAL, SINGLE, XPLOR, CUBIC, LAYOUT, false, false>(kb, grid, block, shmem, stream);
     }
 
 template<class Eval, bool MIXED, bool VIRIAL, bool SINGLE, int LAYOUT>

@@ -240,14 +240,17 @@ __device__ __forceinline__ uint32_t tpm_wave_max(uint32_t v)
     }
 
 // Particle ie's list walked in a wave-uniform loop of `trips` entries (the
-// wavefront's longest list, rounded up to 4), four entries at a time: their
-// list words, positions and orientations (or precomputed directors, `dirs`)
-// are loaded together before the terms are evaluated.  Entries past the
-// lane's own count are padding.
+// wavefront's longest list), four entries at a time: their list words,
+// positions and orientations (or precomputed directors, `dirs`) are loaded
+// together before the terms are evaluated.  Entries past the lane's own count
+// are padding.  A particle's 2^split lanes (lane_split.h) take consecutive
+// fours, this one's starting at entry 4 sub.
 template<bool MIXED, bool VIRIAL, bool SINGLE, bool DIRS>
 __device__ __forceinline__ void tpm_list(uint32_t ie,
                                          uint32_t nn,
                                          uint32_t trips,
+                                         uint32_t sub,
+                                         uint32_t split,
                                          const uint32_t* row,
                                          size_t stride,
                                          const double4* pos,
@@ -267,17 +270,20 @@ __device__ __forceinline__ void tpm_list(uint32_t ie,
     // consecutive entries (HOOMD's head-list rows): below F every lane has
     // U entries left, read as one 16-byte load
     uint32_t F = 0;
+    const uint32_t SU = U << split;
+    const uint32_t k0 = sub * U;
     if (stride == 1)
         {
         uint32_t m = nn;
         for (int off = 32; off > 0; off >>= 1)
             m = min(m, (uint32_t)__shfl_xor((int)m, off));
-        F = __builtin_amdgcn_readfirstlane(m & ~(U - 1));
+        F = __builtin_amdgcn_readfirstlane(m & ~(SU - 1));
         }
-    for (uint32_t k = 0; k < trips; k += U)
+    for (uint32_t kw = 0; kw < trips; kw += SU)
         {
+        const uint32_t k = kw + k0;
         uint32_t jj[U];
-        if (k < F)
+        if (kw < F)
             {
             uint4 w;
             __builtin_memcpy(&w, row + k, sizeof(w));
