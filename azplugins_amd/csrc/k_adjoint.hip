@@ -235,55 +235,77 @@ struct AdjArgs
     double* partial;     // [gridDim.x][ntypes^2 * kAdjNpar]
     };
 
+// One lane per particle, kAdjBatch entries a step: the step's list words are
+// loaded first, then its positions and gradients, then the terms are
+// evaluated, so a lane waits for two loads a step instead of three an entry
+// (the list pads a wavefront's columns to a multiple of 8 with the particle's
+// own index).  FP64 issue (63 %), the gathers' L1 lookups and the fourth of
+// the wavefronts that the registers leave for a second round bound it
+// together: Yukawa FP64, 262,144 particles of 182 entries, 380 -> 344 us (two
+// entries a step, all wavefronts resident: 370).  Parameter gradients are
+// added over a wavefront by a fixed tree and over the workgroup's wavefronts
+// in order.
+constexpr uint32_t kAdjBatch = 4;
+
 template<class Adj, typename R, int NT>
 __global__ void __launch_bounds__(256) k_adjoint(const AdjArgs a)
     {
     using Prep = typename Adj::template Prep<R>;
     __shared__ Prep s_q[NT * NT];
     __shared__ double s_rc[NT * NT];
-    __shared__ double s_acc[256][NT * kAdjNpar];
-    __shared__ uint32_t s_t[256];
+    __shared__ double s_sum[4][NT * NT * kAdjNpar];
     const auto* params = static_cast<const typename Adj::param_type*>(a.params);
     const uint32_t nt = a.ntypes;
     for (uint32_t t = threadIdx.x; t < nt * nt; t += blockDim.x)
         {
         s_q[t] = Adj::template prepare<R>(params[t], a.rcsq[t], a.shift != 0);
-        s_rc[t] = a.rcsq[t];
+        // a pair whose term is switched off has no cutoff either
+        s_rc[t] = Adj::active(s_q[t]) ? a.rcsq[t] : 0.0;
         }
     __syncthreads();
 
     const uint32_t i = xcd_logical_block() * blockDim.x + threadIdx.x;
+    const uint32_t ie = min(i, a.N - 1);
     double acc[NT * kAdjNpar];
 #pragma unroll
     for (int k = 0; k < NT * kAdjNpar; ++k)
         acc[k] = 0.0;
-    uint32_t ti = 0;
-    if (i < a.N)
+    const double4 pi = a.pos[ie];
+    const double4 gi = a.grad[ie];
+    const uint32_t ti = (uint32_t)pi.w;
+    double gx = 0, gy = 0, gz = 0;
+    const uint32_t nn = i < a.N ? a.n_neigh[ie] : 0u;
+    const uint32_t* col = a.nlist + ie;
+    for (uint32_t k = 0; k < nn; k += kAdjBatch)
         {
-        const double4 pi = a.pos[i];
-        const double4 gi = a.grad[i];
-        ti = (uint32_t)pi.w;
-        double gx = 0, gy = 0, gz = 0;
-        const uint32_t nn = a.n_neigh[i];
-        for (uint32_t k = 0; k < nn; ++k)
+        uint32_t jj[kAdjBatch];
+        double4 pj[kAdjBatch], gj[kAdjBatch];
+#pragma unroll
+        for (uint32_t u = 0; u < kAdjBatch; ++u)
+            jj[u] = k + u < nn ? col[(size_t)(k + u) * a.nlist_pitch] : ie;
+#pragma unroll
+        for (uint32_t u = 0; u < kAdjBatch; ++u)
             {
-            const uint32_t j = a.nlist[(size_t)k * a.nlist_pitch + i];
-            const double4 pj = a.pos[j];
-            const double dx = min_image_1d(pi.x - pj.x, a.box.L[0], a.box.Linv[0]);
-            const double dy = min_image_1d(pi.y - pj.y, a.box.L[1], a.box.Linv[1]);
-            const double dz = min_image_1d(pi.z - pj.z, a.box.L[2], a.box.Linv[2]);
+            pj[u] = a.pos[jj[u]];
+            gj[u] = a.grad[jj[u]];
+            }
+#pragma unroll
+        for (uint32_t u = 0; u < kAdjBatch; ++u)
+            {
+            const double dx = min_image_fused(pi.x - pj[u].x, a.box.L[0], a.box.Linv[0]);
+            const double dy = min_image_fused(pi.y - pj[u].y, a.box.L[1], a.box.Linv[1]);
+            const double dz = min_image_fused(pi.z - pj[u].z, a.box.L[2], a.box.Linv[2]);
             const double rsq = dx * dx + dy * dy + dz * dz;
-            const uint32_t tj = (uint32_t)pj.w;
+            const uint32_t tj = (uint32_t)pj[u].w;
             const uint32_t tp = ti * nt + tj;
-            if (!(rsq < s_rc[tp]) || !Adj::active(s_q[tp]))
+            if (k + u >= nn || !(rsq < s_rc[tp]))
                 continue;
             AdjOut<R> o;
             Adj::eval(s_q[tp], (R)rsq, o);
-            const double4 gj = a.grad[j];
             const double f = o.f, fp = o.fp;
-            const double dGx = gi.x - gj.x, dGy = gi.y - gj.y, dGz = gi.z - gj.z;
+            const double dGx = gi.x - gj[u].x, dGy = gi.y - gj[u].y, dGz = gi.z - gj[u].z;
             const double dxdG = dx * dGx + dy * dGy + dz * dGz;
-            const double hw = 0.5 * (gi.w + gj.w);
+            const double hw = 0.5 * (gi.w + gj[u].w);
             gx += f * dGx + fp * dxdG * dx - hw * f * dx;
             gy += f * dGy + fp * dxdG * dy - hw * f * dy;
             gz += f * dGz + fp * dxdG * dz - hw * f * dz;
@@ -297,24 +319,31 @@ __global__ void __launch_bounds__(256) k_adjoint(const AdjArgs a)
                     acc[t * kAdjNpar + p] += sel * (gdx * (double)o.df[p] + 0.5 * gi.w * (double)o.du[p]);
                 }
             }
-        a.grad_pos[i] = make_double4(gx, gy, gz, 0.0);
         }
-    // workgroup reduction of the parameter gradients, binned by (t_i, t_j)
+    if (i < a.N)
+        a.grad_pos[i] = make_double4(gx, gy, gz, 0.0);
+    // the parameter gradients binned by (t_i, t_j): over the wavefront, then
+    // over the workgroup's four
 #pragma unroll
-    for (int k = 0; k < NT * kAdjNpar; ++k)
-        s_acc[threadIdx.x][k] = acc[k];
-    s_t[threadIdx.x] = (i < a.N) ? ti : 0xffffffffu;
+    for (int t = 0; t < NT; ++t)
+        {
+#pragma unroll
+        for (int k = 0; k < NT * kAdjNpar; ++k)
+            {
+            double v = ti == (uint32_t)t ? acc[k] : 0.0;
+            for (int m = 32; m > 0; m >>= 1)
+                v += __shfl_xor(v, m);
+            if ((threadIdx.x & 63u) == 0u)
+                s_sum[threadIdx.x >> 6][t * NT * kAdjNpar + k] = v;
+            }
+        }
     __syncthreads();
     const uint32_t nq = nt * nt * kAdjNpar;
     for (uint32_t q = threadIdx.x; q < nq; q += blockDim.x)
         {
         const uint32_t t = q / (nt * kAdjNpar);
-        const uint32_t rem = q % (nt * kAdjNpar);
-        double s = 0.0;
-        for (uint32_t l = 0; l < blockDim.x; ++l)
-            if (s_t[l] == t)
-                s += s_acc[l][rem];
-        a.partial[(size_t)blockIdx.x * nq + q] = s;
+        const uint32_t src = t * NT * kAdjNpar + q % (nt * kAdjNpar);
+        a.partial[(size_t)blockIdx.x * nq + q] = ((s_sum[0][src] + s_sum[1][src]) + s_sum[2][src]) + s_sum[3][src];
         }
     }
 
