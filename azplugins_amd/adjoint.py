@@ -73,6 +73,10 @@ class PairForceField:
         self._rcut = rc
         dev = torch.device("cuda")
         self._rcutsq = torch.tensor(rc * rc, dtype=torch.float64, device=dev)
+        # the pairs' rows of an (a, b) table, and 1/2 where a = b
+        self._rows = torch.tensor([a * self.ntypes + b for a, b in self.pair_keys], device=dev)
+        self._share = torch.tensor([[0.5 if k // self.ntypes == k % self.ntypes else 1.0]
+                                    for k in range(self.ntypes * self.ntypes)], dtype=torch.float64, device=dev)
         self._nl = _azplugins.NeighborListGPU(r_buff)
         self._nl.set_r_cut(self.ntypes, rc.tolist())
         self._psize = _azp.lib().azp_param_size(self.evaluator)
@@ -132,7 +136,7 @@ class _PairForceFunction(torch.autograd.Function):
         parts = _azp.Particles(N, ff.box, pos4.data_ptr(), None, None, None, None)
         ff._nl.update(parts)
         d_params = ff._pack(theta)
-        force = torch.zeros((N, 4), dtype=torch.float64, device=pos.device)
+        force = torch.empty((N, 4), dtype=torch.float64, device=pos.device)
         args = ff._args(pos4, force, ff.precision)
         if ff.precision != "fp64":
             pos_fixed = torch.empty((N, 4), dtype=torch.int32, device=pos.device)
@@ -154,23 +158,20 @@ class _PairForceFunction(torch.autograd.Function):
         ff = ctx.ff
         N = pos4.shape[0]
         dev = pos4.device
-        grad = torch.zeros((N, 4), dtype=torch.float64, device=dev)
-        if gF is not None:
-            grad[:, :3] = gF
-        if gE is not None:
-            grad[:, 3] = gE
-        grad = grad.contiguous()
-        gpos = torch.zeros((N, 4), dtype=torch.float64, device=dev)
+        # the launches write every element of what is allocated uninitialised
+        grad = torch.empty((N, 4), dtype=torch.float64, device=dev)
+        grad[:, :3] = gF if gF is not None else 0.0
+        grad[:, 3] = gE if gE is not None else 0.0
+        gpos = torch.empty((N, 4), dtype=torch.float64, device=dev)
         nt = ff.ntypes
-        gpar = torch.zeros(nt * nt * NPAR, dtype=torch.float64, device=dev)
+        gpar = (torch.empty if N else torch.zeros)(nt * nt * NPAR, dtype=torch.float64, device=dev)
         wlen = _azp.lib().azp_adjoint_workspace_size(N, nt)
-        work = torch.zeros(wlen, dtype=torch.float64, device=dev)
+        work = torch.empty(wlen, dtype=torch.float64, device=dev)
         args = ff._args(pos4, None, ff.adjoint_precision)
         _azp.call("azp_gpu_pair_adjoint", ctypes.byref(args), ff.evaluator, _azp.dptr(d_params),
                   _azp.dptr(grad), _azp.dptr(gpos), _azp.dptr(gpar), _azp.dptr(work), wlen)
         g = gpar.view(nt, nt, NPAR)
-        rows = []
-        for a, b in ff.pair_keys:
-            rows.append(g[a, b] + g[b, a] if a != b else g[a, a])
-        gtheta = torch.stack(rows).to(device=ctx.theta_device, dtype=ctx.theta_dtype)
+        # rows (a, b) and (b, a) of a pair of unlike types add up
+        both = (g + g.transpose(0, 1)).view(nt * nt, NPAR)
+        gtheta = (both * ff._share).index_select(0, ff._rows).to(device=ctx.theta_device, dtype=ctx.theta_dtype)
         return gpos[:, :3].clone(), gtheta, None, None
