@@ -8,7 +8,6 @@
 // (i, j) exactly in exact arithmetic (both are dU/dgamma_j (r_hat x n_j)).
 #include <type_traits>
 
-#include "lane_split.h"
 #include "tpm.h"
 
 namespace azp
@@ -75,11 +74,20 @@ __global__ void __launch_bounds__(512) k_aniso(const AnisoKernelArgs a)
         }
     AnisoAcc acc;
     const uint32_t nn = i < a.N ? a.n_neigh[i] : 0u;
-    const uint32_t trips = __builtin_amdgcn_readfirstlane((tpm_wave_max(nn) + 3u) & ~3u);
     const uint32_t* row = a.head_list ? a.nlist + a.head_list[ie] : a.nlist + ie;
     const size_t stride = a.head_list ? 1 : a.nlist_pitch;
-    tpm_list<MIXED, VIRIAL, SINGLE, false>(ie, nn, trips, lane.sub, split, row, stride, a.pos, a.pos_fixed,
-                                           a.orientation, nullptr, me, box, nt, q0, s_q, acc);
+    [[maybe_unused]] uint32_t* queue = reinterpret_cast<uint32_t*>(SINGLE ? s_q : s_q + nt * nt);
+    if constexpr (MIXED)
+        {
+        const uint32_t trips = __builtin_amdgcn_readfirstlane((tpm_wave_max(nn) + 3u) & ~3u);
+        tpm_list<MIXED, VIRIAL, SINGLE, false>(ie, nn, trips, lane.sub, split, row, stride, a.pos, a.pos_fixed,
+                                               a.orientation, nullptr, me, box, nt, q0, s_q, acc);
+        }
+    else
+        {
+        tpm_list_queued<VIRIAL, SINGLE>(nn, lane.sub, split, row, stride, queue, a.pos, a.orientation, me, box, nt, q0,
+                                        s_q, acc);
+        }
     if (split != 0u)
         {
         for (double* v : {&acc.fx, &acc.fy, &acc.fz, &acc.tx, &acc.ty, &acc.tz, &acc.pe})
@@ -98,9 +106,11 @@ template<bool MIXED, bool VIRIAL, bool SINGLE>
 static int launch_aniso_t(const AnisoKernelArgs& ka, unsigned block, hipStream_t s)
     {
     using R = std::conditional_t<MIXED, float, double>;
-    const size_t shmem = SINGLE ? 0 : (size_t)ka.ntypes * ka.ntypes * sizeof(TPMPrep<R>);
-    if (shmem > 64 * 1024)
+    const size_t table = SINGLE ? 0 : (size_t)ka.ntypes * ka.ntypes * sizeof(TPMPrep<R>);
+    if (table > 64 * 1024)
         return set_error(AZP_ERR_UNSUPPORTED, "too many particle types for LDS staging");
+    const size_t shmem = table + tpm_queue_bytes<MIXED>(block);
+    AZP_TRY(tpm_raise_lds(reinterpret_cast<const void*>(&k_aniso<MIXED, VIRIAL, SINGLE>), shmem));
     hipLaunchKernelGGL((k_aniso<MIXED, VIRIAL, SINGLE>), dim3(grid_for((size_t)ka.N << ka.split, block)), dim3(block), shmem,
                        s, ka);
     AZP_LAUNCH_CHECK();

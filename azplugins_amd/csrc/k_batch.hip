@@ -460,6 +460,7 @@ __global__ void __launch_bounds__(512) k_b_forces(const BatchForceArgs a)
         __syncthreads();
         }
     const uint32_t lane = threadIdx.x & 63u;
+    [[maybe_unused]] uint32_t* queue = reinterpret_cast<uint32_t*>(SINGLE ? s_q : s_q + nt * nt);
     for (;;)
         {
         uint32_t c0 = 0;
@@ -486,9 +487,17 @@ __global__ void __launch_bounds__(512) k_b_forces(const BatchForceArgs a)
             const AnisoSelf<R> me = aniso_self<MIXED>(a.pos, a.pos_fixed, a.orientation, ie);
             AnisoAcc acc;
             const uint32_t nn = active ? a.n_neigh[i] : 0u;
-            const uint32_t trips = __builtin_amdgcn_readfirstlane((tpm_wave_max(nn) + 3u) & ~3u);
-            tpm_list<MIXED, VIRIAL, SINGLE, MIXED>(ie, nn, trips, 0u, 0u, a.nlist + ie, a.pitch, a.pos, a.pos_fixed, a.orientation,
-                                                   a.dirs, me, box, nt, q0, s_q, acc);
+            if constexpr (MIXED)
+                {
+                const uint32_t trips = __builtin_amdgcn_readfirstlane((tpm_wave_max(nn) + 3u) & ~3u);
+                tpm_list<MIXED, VIRIAL, SINGLE, MIXED>(ie, nn, trips, 0u, 0u, a.nlist + ie, a.pitch, a.pos, a.pos_fixed,
+                                                       a.orientation, a.dirs, me, box, nt, q0, s_q, acc);
+                }
+            else
+                {
+                tpm_list_queued<VIRIAL, SINGLE>(nn, 0u, 0u, a.nlist + ie, a.pitch, queue, a.pos, a.orientation, me, box,
+                                                nt, q0, s_q, acc);
+                }
             if (active)
                 aniso_store<VIRIAL>(a.force, a.torque, a.virial, a.vpitch, i, acc);
             }
@@ -1054,7 +1063,9 @@ int launch_forces_t(azp_batch* b, const azp_batch_tuning& t, hipStream_t s)
     if (t.workgroups_per_cu > 0)
         grid = std::min<unsigned>(grid, (unsigned)b->num_cu * t.workgroups_per_cu);
     grid = std::max(grid, 1u);
-    const size_t shmem = SINGLE ? 0 : (size_t)b->ntypes * b->ntypes * sizeof(TPMPrep<R>);
+    const size_t table = SINGLE ? 0 : (size_t)b->ntypes * b->ntypes * sizeof(TPMPrep<R>);
+    const size_t shmem = table + tpm_queue_bytes<MIXED>(block);
+    AZP_TRY(tpm_raise_lds(reinterpret_cast<const void*>(&k_b_forces<MIXED, VIRIAL, SINGLE>), shmem));
     hipLaunchKernelGGL(k_b_fill, dim3(1), dim3(64), 0, s, b->counter.ptr, 0u, 1u, nullptr);
     hipLaunchKernelGGL((k_b_forces<MIXED, VIRIAL, SINGLE>), dim3(grid), dim3(block), shmem, s, fa);
     return AZP_OK;

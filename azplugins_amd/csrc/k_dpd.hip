@@ -112,25 +112,6 @@ __device__ __forceinline__ DPDPair make_dpd_pair(const DPDKernelArgs& a, uint32_
     return q;
     }
 
-// The entries of one lane: entry m of its own sequence is list entry at(m).
-// With a split (lane_split.h) the particle's lanes take consecutive fours.
-template<bool SPLIT> struct LaneEntries
-    {
-    uint32_t split, first;
-    __device__ __forceinline__ LaneEntries(uint32_t split_, uint32_t sub) : split(split_), first(4u * sub) { }
-    __device__ __forceinline__ uint32_t at(uint32_t m) const
-        {
-        return SPLIT ? ((m & ~3u) << split) + first + (m & 3u) : m;
-        }
-    __device__ __forceinline__ uint32_t count(uint32_t nn) const
-        {
-        if (!SPLIT)
-            return nn;
-        const uint32_t rest = nn & ((4u << split) - 1u);
-        return ((nn >> (2u + split)) << 2) + (rest > first ? min(rest - first, 4u) : 0u);
-        }
-    };
-
 // LDS_TABLE: the type-pair table is staged in LDS (up to 16 KiB, 17 types);
 // otherwise each in-cut pair derives its entry from the global parameter
 // arrays by the same operations (bit-identical, slower).

@@ -74,6 +74,25 @@ __device__ __forceinline__ SplitLane split_lane(uint32_t split)
     return s;
     }
 
+// The entries of one lane: entry m of its own sequence is list entry at(m).
+// With a split the particle's lanes take consecutive fours.
+template<bool SPLIT> struct LaneEntries
+    {
+    uint32_t split, first;
+    __device__ __forceinline__ LaneEntries(uint32_t split_, uint32_t sub) : split(split_), first(4u * sub) { }
+    __device__ __forceinline__ uint32_t at(uint32_t m) const
+        {
+        return SPLIT ? ((m & ~3u) << split) + first + (m & 3u) : m;
+        }
+    __device__ __forceinline__ uint32_t count(uint32_t nn) const
+        {
+        if (!SPLIT)
+            return nn;
+        const uint32_t rest = nn & ((4u << split) - 1u);
+        return ((nn >> (2u + split)) << 2) + (rest > first ? min(rest - first, 4u) : 0u);
+        }
+    };
+
 // Sum over a particle's lanes, the same value in each of them.
 __device__ __forceinline__ double split_sum(double v, uint32_t split)
     {

@@ -8,6 +8,7 @@
 #include <type_traits>
 
 #include "device_common.h"
+#include "lane_split.h"
 
 namespace azp
 {
@@ -239,7 +240,7 @@ __device__ __forceinline__ uint32_t tpm_wave_max(uint32_t v)
     return v;
     }
 
-// Particle ie's list walked in a wave-uniform loop of `trips` entries (the
+// Particle ie's list (the mixed form's) walked in a wave-uniform loop of `trips` entries (the
 // wavefront's longest list), four entries at a time: their list words,
 // positions and orientations (or precomputed directors, `dirs`) are loaded
 // together before the terms are evaluated.  Entries past the lane's own count
@@ -315,6 +316,121 @@ __device__ __forceinline__ void tpm_list(uint32_t ie,
 #pragma unroll
         for (uint32_t u = 0; u < U; ++u)
             tpm_term<MIXED, VIRIAL, SINGLE>(k + u < nn, jj[u], pj[u], oj[u], pos, me, box, nt, q0, s_q, acc);
+        }
+    }
+
+// In-cut neighbors that a lane holds in LDS between the scan and the
+// evaluation of the plain form (column threadIdx.x of a
+// [kTpmQueue][blockDim.x] array).
+constexpr uint32_t kTpmQueue = 16;
+
+template<bool MIXED> inline size_t tpm_queue_bytes(unsigned block)
+    {
+    return MIXED ? 0 : (size_t)kTpmQueue * block * sizeof(uint32_t);
+    }
+
+// Lets a kernel use more than 64 KiB of dynamic LDS (gfx950 gives a workgroup
+// 160 KiB; the largest table and the queue of 512 lanes take 96).
+inline int tpm_raise_lds(const void* kernel, size_t shmem)
+    {
+    if (shmem > 64 * 1024)
+        AZP_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem));
+    return AZP_OK;
+    }
+
+// Displacement of neighbor j and its square (the plain form).
+__device__ __forceinline__ double tpm_delta(const double4& pj, const AnisoSelf<double>& me, const LaneBox& box, double dr[3])
+    {
+    dr[0] = min_image_1d(me.pos.x - pj.x, box.L[0], box.Linv[0]);
+    dr[1] = min_image_1d(me.pos.y - pj.y, box.L[1], box.Linv[1]);
+    dr[2] = min_image_1d(me.pos.z - pj.z, box.L[2], box.Linv[2]);
+    return dr[0] * dr[0] + dr[1] * dr[1] + dr[2] * dr[2];
+    }
+
+// One particle's list in the plain form: a scan collects the next in-cut
+// neighbors, each lane at its own place in its list, until its queue is full
+// or the list ends; an evaluation pass then takes the queued pairs in list
+// order, two gathers at a time.  A wavefront evaluates as many pairs as its
+// lane with the most in-cut entries has, not as many as its longest list:
+// about a third of the entries lie in the buffer shell, and FP64 issue bounds
+// the walk.  40,009 particles 38.0 -> 33.3 us, 130,000 98 -> 89, 200,000
+// 154 -> 139.  The mixed form stays with tpm_list: its terms are light enough
+// that the gathers weigh as much (2.7 million particles 984 us; with a queue
+// of indices 1133, of displacements 1132).
+template<bool VIRIAL, bool SINGLE>
+__device__ __forceinline__ void tpm_list_queued(uint32_t nn,
+                                                uint32_t sub,
+                                                uint32_t split,
+                                                const uint32_t* row,
+                                                size_t stride,
+                                                uint32_t* queue,
+                                                const double4* pos,
+                                                const double4* orientation,
+                                                const AnisoSelf<double>& me,
+                                                const LaneBox& box,
+                                                uint32_t nt,
+                                                const TPMPrep<double>& q0,
+                                                const TPMPrep<double>* s_q,
+                                                AnisoAcc& acc)
+    {
+    const uint32_t bs = blockDim.x;
+    uint32_t* q_col = queue + threadIdx.x;
+    const LaneEntries<true> mine(split, sub);
+    const uint32_t count = mine.count(nn);
+    uint32_t k = 0;
+    while (k < count)
+        {
+        uint32_t cnt = 0;
+        while (k < count && cnt + 4u <= kTpmQueue)
+            {
+            const uint32_t e = mine.at(k);
+            const uint32_t m = min(count - k, 4u);
+            uint32_t jj[4];
+            if (stride == 1 && m == 4u)
+                {
+                // consecutive entries (HOOMD's head-list rows): one 16-byte load
+                uint4 w;
+                __builtin_memcpy(&w, row + e, sizeof(w));
+                jj[0] = w.x;
+                jj[1] = w.y;
+                jj[2] = w.z;
+                jj[3] = w.w;
+                }
+            else
+                {
+                // past the end: the last entry again, not queued
+#pragma unroll
+                for (uint32_t u = 0; u < 4; ++u)
+                    jj[u] = row[(size_t)(e + min(u, m - 1u)) * stride];
+                }
+            double4 pj[4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u)
+                pj[u] = pos[jj[u]];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u)
+                {
+                double dr[3];
+                const double rsq = tpm_delta(pj[u], me, box, dr);
+                const double rcsq = SINGLE ? q0.rcsq : s_q[me.type * nt + (uint32_t)pj[u].w].rcsq;
+                if (u < m && !(rsq > rcsq)) // AnisoPairEvaluatorTwoPatchMorse.h:135
+                    q_col[(cnt++) * bs] = jj[u];
+                }
+            k += 4u;
+            }
+        for (uint32_t c = 0; c < cnt; c += 2u)
+            {
+            const bool two = c + 1u < cnt;
+            const uint32_t j0 = q_col[c * bs];
+            const uint32_t j1 = two ? q_col[(c + 1u) * bs] : j0;
+            const double4 p0 = pos[j0];
+            const double4 o0 = orientation[j0];
+            const double4 p1 = pos[j1];
+            const double4 o1 = orientation[j1];
+            tpm_term<false, VIRIAL, SINGLE>(true, j0, p0, o0, pos, me, box, nt, q0, s_q, acc);
+            if (two)
+                tpm_term<false, VIRIAL, SINGLE>(true, j1, p1, o1, pos, me, box, nt, q0, s_q, acc);
+            }
         }
     }
 
