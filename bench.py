@@ -47,14 +47,16 @@ HEADLINE_KERNEL = ("void azp::k_pair<azp::EvalPerturbedLJ, true, true, true, fal
 KERNEL_SOURCES = {
     "pmc_plj_1m.json": ("azplugins_amd/csrc/pair_kernel.h", "azplugins_amd/csrc/evaluators.h",
                         "azplugins_amd/csrc/device_common.h", "azplugins_amd/csrc/tiles.h",
-                        "azplugins_amd/csrc/k_pair_tiled.hip", "include/azp.h"),
+                        "azplugins_amd/csrc/lane_split.h", "azplugins_amd/csrc/k_pair_tiled.hip", "include/azp.h"),
     "pmc_dpd_2m.json": ("azplugins_amd/csrc/k_dpd.hip", "azplugins_amd/csrc/device_common.h",
-                        "azplugins_amd/csrc/portable_math.h", "azplugins_amd/csrc/tiles.h", "include/azp.h"),
+                        "azplugins_amd/csrc/portable_math.h", "azplugins_amd/csrc/tiles.h",
+                        "azplugins_amd/csrc/lane_split.h", "include/azp.h"),
     "pmc_tpm_batch.json": ("azplugins_amd/csrc/k_batch.hip", "azplugins_amd/csrc/tpm.h",
+                           "azplugins_amd/csrc/lane_split.h", "azplugins_amd/csrc/group_walk.h",
                            "azplugins_amd/csrc/device_common.h", "include/azp.h"),
     "pmc_yukawa_262k.json": ("azplugins_amd/csrc/k_adjoint.hip", "azplugins_amd/csrc/pair_kernel.h",
                              "azplugins_amd/csrc/evaluators.h", "azplugins_amd/csrc/device_common.h",
-                             "include/azp.h"),
+                             "azplugins_amd/csrc/lane_split.h", "include/azp.h"),
 }
 
 
