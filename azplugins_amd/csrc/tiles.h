@@ -119,9 +119,9 @@ struct TileWalkArgs
 constexpr uint32_t kTileTable = 29696;
 constexpr uint32_t kTileTableMax = 69632;
 
-// Most batches of a group the walk makes room for (beyond it a tile's rank
-// tables do not fit anyway).
-constexpr uint32_t kGroupBatchesMax = 64;
+// Most batches of a group the walk makes room for: a 256-column tile of four
+// such groups fills the largest rank tables.
+constexpr uint32_t kGroupBatchesMax = kTileTableMax / 64 / 4;
 
 // Enqueues the per-tile walk with tiles of `tile_size` (256 or 512) particles
 // into t's arrays (sized here); the caller reads args.flags afterwards and
