@@ -209,6 +209,7 @@ SIGNATURES = [
     ("azp_nlist_get_tile_order", _i, [_vp, ctypes.POINTER(_vp), ctypes.POINTER(_vp)]),
     ("azp_nlist_walk_kind", _i, [_vp, ctypes.POINTER(_i)]),
     ("azp_nlist_tile_stats", _i, [_vp, ctypes.POINTER(_u32), ctypes.POINTER(_u32)]),
+    ("azp_nlist_walk_runs", _i, [_vp, ctypes.POINTER(ctypes.c_uint64), ctypes.POINTER(ctypes.c_uint64)]),
     ("azp_sorter_create", _i, [ctypes.POINTER(_vp)]),
     ("azp_sorter_destroy", _i, [_vp]),
     ("azp_sorter_order", _i, [_vp, ctypes.POINTER(Particles), _u32, _vp, _vp]),

@@ -270,6 +270,13 @@ class NeighborListGPU:
         _azp.call("azp_nlist_tile_stats", self._h, ctypes.byref(n), ctypes.byref(r))
         return n.value, r.value
 
+    def walk_runs(self):
+        """(runs of the per-block walk, runs of its compaction) since the list was created."""
+        rows = ctypes.c_uint64()
+        compactions = ctypes.c_uint64()
+        _azp.call("azp_nlist_walk_runs", self._h, ctypes.byref(rows), ctypes.byref(compactions))
+        return rows.value, compactions.value
+
     def download(self, N):
         """(n_neigh[N], list[max_neighbors, pitch]) as numpy arrays.  They view
         pinned host memory, so each array arrives in one DMA copy."""

@@ -390,6 +390,7 @@ struct azp_nlist
     uint32_t* h_flags = nullptr;  // pinned, kHostFlags words ([4], [5] tile build flags)
     uint32_t group_cells = 0, group_batches = 0; // per group of 64 slots: room of the per-tile walk
     uint32_t tile_table = kTileTable;            // and of a tile's rank tables
+    uint64_t row_runs = 0, compactions = 0;      // of the per-tile walk's kernels
 
     bool want_tiles = false;
     uint32_t tile_mode = 0; // 1: 512 else 256; 256 / 512: that size only
@@ -500,14 +501,19 @@ static int nlist_build(azp_nlist* nl, const azp_particles* p, hipStream_t s)
             nl->max_neighbors = 8;
         }
     nl->pitch = wave_pitch(N);
-    // room for a group's cells and candidates in the per-tile walk: at first
-    // those of about 72 cells at the mean density, afterwards what a build
-    // needed
+    // room for a group's cells and candidates in the per-tile walk, afterwards
+    // what a build needed.  At first, by the mean occupancy m of a cell, about
+    // twice what lattices and random fluids of 900 to 600,000 particles need:
+    // three passes over the whole of a 3 x 3 x 3 grid are 1.3 m batches, two
+    // passes of a larger one the same, and the sparser the cells the more of
+    // them and the more passes a group takes (m = 2: up to 744 cells and 34
+    // batches; 9: 153, 23; 34: 82, 43; 56: 81, 73; 96: 54, 84).  A first build
+    // that runs out of room takes twice as long.
     if (nl->group_cells == 0)
         {
-        const double per_cell = (double)N / (double)ncell;
-        nl->group_cells = (uint32_t)std::min(512.0, 128.0 + 500.0 / (1.0 + per_cell));
-        nl->group_batches = (uint32_t)std::min((double)kGroupBatchesMax, 6.0 + 72.0 * per_cell / 64.0);
+        const double m = (double)N / (double)ncell;
+        nl->group_cells = (uint32_t)std::min((double)kGroupCellsMax, 192.0 + 2500.0 / (1.0 + m));
+        nl->group_batches = (uint32_t)std::min((double)kGroupBatchesMax, 40.0 + 1.5 * m);
         }
     bool uniform = true;
     for (double rc : nl->r_cut)
@@ -561,6 +567,8 @@ static int nlist_build(azp_nlist* nl, const azp_particles* p, hipStream_t s)
                 ta.group_batch_cap = nl->group_batches;
                 ta.table_cap = nl->tile_table;
                 AZP_TRY(tiles_walk(nl->tiles, ts, ta, uniform, s));
+                ++nl->row_runs;
+                ++nl->compactions;
                 // the positions of this build, queued before the flags are
                 // read so that no host round trip separates it from the walk
                 // (a failed attempt copies them again)
@@ -579,7 +587,8 @@ static int nlist_build(azp_nlist* nl, const azp_particles* p, hipStream_t s)
                 else if (nl->h_flags[kTileFlagCells] != 0u || nl->h_flags[kTileFlagBatches] != 0u)
                     {
                     // a group ran out of room (every count above is valid)
-                    nl->group_cells = std::max(nl->group_cells, nl->h_flags[kTileFlagCells] * 5 / 4);
+                    nl->group_cells = std::min(kGroupCellsMax,
+                                               std::max(nl->group_cells, nl->h_flags[kTileFlagCells] * 5 / 4));
                     nl->group_batches = std::min(kGroupBatchesMax,
                                                  std::max(nl->group_batches, nl->h_flags[kTileFlagBatches] * 5 / 4));
                     grown = true;
@@ -1028,6 +1037,15 @@ extern "C" int azp_nlist_tile_stats(const azp_nlist* nl, uint32_t* ntiles, uint3
     const bool ok = nl->fused && nl->tiles.valid;
     *ntiles = ok ? nl->tiles.ntiles : 0u;
     *relative_tiles = ok ? nl->relative_tiles : 0u;
+    return AZP_OK;
+    }
+
+extern "C" int azp_nlist_walk_runs(const azp_nlist* nl, uint64_t* rows, uint64_t* compactions)
+    {
+    if (!nl || !rows || !compactions)
+        return set_error(AZP_ERR_INVALID, "null argument");
+    *rows = nl->row_runs;
+    *compactions = nl->compactions;
     return AZP_OK;
     }
 

@@ -122,6 +122,8 @@ constexpr uint32_t kTileTableMax = 69632;
 // Most batches of a group the walk makes room for: a 256-column tile of four
 // such groups fills the largest rank tables.
 constexpr uint32_t kGroupBatchesMax = kTileTableMax / 64 / 4;
+// Most cells it lists: a pass visits at most 27 for each column that it serves.
+constexpr uint32_t kGroupCellsMax = 64 * 27;
 
 // Enqueues the per-tile walk with tiles of `tile_size` (256 or 512) particles
 // into t's arrays (sized here); the caller reads args.flags afterwards and

@@ -418,6 +418,10 @@ int azp_nlist_walk_kind(const azp_nlist* nl, int* kind);
  * an anchor, rather than some as fixed-point differences (grids of one or two
  * cells on an axis); both 0 after a plain walk. */
 int azp_nlist_tile_stats(const azp_nlist* nl, uint32_t* ntiles, uint32_t* relative_tiles);
+/* How often the two kernels of the per-block walk ran since the list was
+ * created: one of each per build that it serves; more where a build was
+ * repeated with more room, or tried other block sizes. */
+int azp_nlist_walk_runs(const azp_nlist* nl, uint64_t* rows, uint64_t* compactions);
 /* Copy n_neigh[N] and the list (max_neighbors * pitch entries) to host memory
  * (synchronizes the device). */
 int azp_nlist_download(const azp_nlist* nl,
