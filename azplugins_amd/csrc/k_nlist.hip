@@ -132,18 +132,33 @@ __global__ void __launch_bounds__(256) k_sort_cells(uint32_t ncell,
 // Cell-ordered copy of the positions for the walk: slot m (the m-th member in
 // cell order) holds the member's position as wrapped 32-bit fixed point and,
 // in .w, its checked type (ntypes for an invalid type or a non-finite
-// position, which is then never listed); rank_of[j] = m.
+// position, which is then never listed); rank_of[j] = m.  With span_flag (a
+// build that tries the per-tile walk) the tile sizes with a tile of more than
+// kOwnCells cells are flagged there.
 __global__ void k_cell_fixed(uint32_t N,
                              const uint32_t* __restrict__ members,
                              const double4* __restrict__ pos,
                              DevBox box,
                              uint32_t ntypes,
                              int4* __restrict__ cell_fixed,
-                             uint32_t* __restrict__ rank_of)
+                             uint32_t* __restrict__ rank_of,
+                             const uint32_t* __restrict__ cell_of,
+                             const uint32_t* __restrict__ cell_rank,
+                             uint32_t* __restrict__ span_flag)
     {
     const uint32_t m = blockIdx.x * blockDim.x + threadIdx.x;
     if (m >= N)
         return;
+    if (span_flag != nullptr && m % 256u == 0u)
+        {
+        const uint32_t first = cell_rank[cell_of[members[m]]];
+        const uint32_t last256 = cell_rank[cell_of[members[min(m + 256u, N) - 1u]]];
+        const uint32_t last512 = cell_rank[cell_of[members[min(m + 512u, N) - 1u]]];
+        const uint32_t bits = (last256 - first >= kOwnCells ? kTileSpan256 : 0u)
+                              | (m % 512u == 0u && last512 - first >= kOwnCells ? kTileSpan512 : 0u);
+        if (bits != 0u)
+            atomicOr(span_flag, bits);
+        }
     const uint32_t j = members[m];
     const double4 p = pos[j];
     const bool finite = isfinite(p.x) && isfinite(p.y) && isfinite(p.z);
@@ -386,7 +401,7 @@ struct azp_nlist
     DeviceArray<uint32_t> cell_rank; // Morton rank of each cell of the grid below
     DeviceArray<uint32_t> rank_cell; // its inverse
     int rank_grid[3] = {0, 0, 0};
-    DeviceArray<uint32_t> flags; // [1] rebuild, [6] the step kernel's check, the others as in tiles.h
+    DeviceArray<uint32_t> flags; // [1] rebuild, [kFlagStep] the step kernel's check, the others as in tiles.h
     uint32_t* h_flags = nullptr;  // pinned, kHostFlags words ([4], [5] tile build flags)
     uint32_t group_cells = 0, group_batches = 0; // per group of 64 slots: room of the per-tile walk
     uint32_t tile_table = kTileTable;            // and of a tile's rank tables
@@ -402,6 +417,7 @@ struct azp_nlist
     uint32_t relative_tiles = 0; // of which tiles were walked in FP32 offsets
     hipStream_t last_stream = nullptr;
     uint32_t walk_skip[2] = {0, 0}; // builds to skip the fused walk of 512 / 256 after a tile did not fit
+    uint32_t span = 0;              // the last tiled build's span flags: sizes that it ruled out
 
     uint32_t pitch = 0;
     uint32_t max_neighbors = 0;
@@ -409,7 +425,7 @@ struct azp_nlist
     azp_box built_box = {0, 0, 0};
     bool have_list = false;
     uint64_t n_builds = 0;
-    // flags[6] holds the rebuild check of these positions, made by the step
+    // flags[kFlagStep] holds the rebuild check of these positions, made by the step
     // after the last force (k_step) as (checked_seq << 2) | bits; the next
     // update_compute_step reads it.  Each step check takes a new number, so
     // the word is cleared only on first use and when the numbers wrap.
@@ -433,8 +449,26 @@ struct azp_nlist
         }
     };
 
+static uint32_t span_bit(uint32_t tile_size)
+    {
+    return tile_size == 512u ? kTileSpan512 : kTileSpan256;
+    }
+
+// The error of a build's bad-particle flag.
+static int bad_particle(uint32_t bits, uint32_t ntypes)
+    {
+    if (bits & 2u)
+        return set_error(AZP_ERR_INVALID, "a particle position is not finite (NaN or inf)");
+    if (bits & 1u)
+        return set_error(AZP_ERR_INVALID, "a particle type index is outside [0, %u) (pos.w must hold the type)", ntypes);
+    return AZP_OK;
+    }
+
 static int nlist_build(azp_nlist* nl, const azp_particles* p, hipStream_t s)
     {
+    const uint32_t N = p->N;
+    if (N != nl->built_N)
+        nl->span = 0; // another system (so does another grid, below)
     // until this build succeeds there is no list: an error return leaves the
     // list invalid, so the next update rebuilds it instead of comparing the
     // displacement against the failed build's positions
@@ -442,7 +476,6 @@ static int nlist_build(azp_nlist* nl, const azp_particles* p, hipStream_t s)
     nl->built_N = 0;
     nl->tiles.valid = false;
     nl->checked_pos = nullptr;
-    const uint32_t N = p->N;
     const DevBox box = make_box(p->box);
     const double rmax = nl->r_list_max();
     const double L[3] = {p->box.Lx, p->box.Ly, p->box.Lz};
@@ -459,7 +492,7 @@ static int nlist_build(azp_nlist* nl, const azp_particles* p, hipStream_t s)
     AZP_TRY(nl->rank_of.reserve(N));
     AZP_TRY(nl->n_neigh.reserve(N));
     AZP_TRY(nl->last_pos.reserve(N));
-    AZP_TRY(nl->flags.reserve(kTileFlags));
+    AZP_TRY(nl->flags.reserve(kTileFlags + 1));
 
     if (g.n[0] != nl->rank_grid[0] || g.n[1] != nl->rank_grid[1] || g.n[2] != nl->rank_grid[2])
         {
@@ -474,6 +507,7 @@ static int nlist_build(azp_nlist* nl, const azp_particles* p, hipStream_t s)
         AZP_HIP(hipStreamSynchronize(s)); // the host vectors go out of scope
         for (int k = 0; k < 3; ++k)
             nl->rank_grid[k] = g.n[k];
+        nl->span = 0;
         }
 
     const unsigned B = 256;
@@ -486,8 +520,31 @@ static int nlist_build(azp_nlist* nl, const azp_particles* p, hipStream_t s)
                        nl->slot_of.ptr, nl->start.ptr, nl->members.ptr);
     hipLaunchKernelGGL(k_sort_cells, dim3(grid_for(ncell, 4)), dim3(256), 0, s, (uint32_t)ncell,
                        nl->start.ptr, nl->members.ptr);
+    // tile sizes that the per-tile walk tries: 512 particles, else 256.  A size
+    // that did not fit is left out for the next builds, and for as long as the
+    // last build's own cells ruled it out.
+    uint32_t sizes[2], nsizes = 0, size_bits = 0;
+    if (nl->want_tiles && nl->ntypes <= kTileWalkMaxTypes)
+        for (uint32_t k = 0; k < 2; ++k)
+            {
+            const uint32_t ts = k == 0 ? 512u : 256u;
+            if (nl->tile_mode != 1 && nl->tile_mode != ts)
+                continue;
+            if (nl->walk_skip[k] > 0)
+                {
+                --nl->walk_skip[k];
+                continue;
+                }
+            if (nl->span & span_bit(ts))
+                continue;
+            sizes[nsizes++] = ts;
+            size_bits |= span_bit(ts);
+            }
+    if (nl->want_tiles)
+        hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, nl->flags.ptr, 0u, (size_t)kTileFlags);
     hipLaunchKernelGGL(k_cell_fixed, dim3(grid_for(N, B)), dim3(B), 0, s, N, nl->members.ptr, pos, box, nl->ntypes,
-                       nl->cell_fixed.ptr, nl->rank_of.ptr);
+                       nl->cell_fixed.ptr, nl->rank_of.ptr, nl->cell_of.ptr, nl->cell_rank.ptr,
+                       nl->want_tiles ? nl->flags.ptr + kTileFlagSpan : nullptr);
     AZP_LAUNCH_CHECK();
 
     // initial capacity from the density
@@ -525,49 +582,47 @@ static int nlist_build(azp_nlist* nl, const azp_particles* p, hipStream_t s)
         nl->tiles.valid = false;
         nl->plain_ready = true;
         nl->fused = false;
-        if (nl->want_tiles && nl->ntypes <= kTileWalkMaxTypes)
+        if (nsizes != 0)
             {
-            // fused walk: the tiled list straight from the cell list, 512-
-            // particle tiles, else 256
-            bool grown = false, done = false;
-            for (uint32_t ts : {512u, 256u})
+            // fused walk: the tiled list straight from the cell list
+            if (attempt > 0)
+                hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, nl->flags.ptr, 0u, (size_t)kTileFlagSpan);
+            TileWalkArgs ta;
+            ta.g.pos = pos;
+            ta.g.members = nl->members.ptr;
+            ta.g.start = nl->start.ptr;
+            ta.g.cell_rank = nl->cell_rank.ptr;
+            ta.g.cell_fixed = nl->cell_fixed.ptr;
+            ta.g.r_listsq = nl->r_listsq.ptr;
+            ta.g.ntypes = nl->ntypes;
+            ta.g.r_max = (float)rmax;
+            ta.g.thr = (float)(rmax * rmax);
+            ta.g.direct = false;
+            ta.N = N;
+            ta.box = box;
+            for (int k = 0; k < 3; ++k)
+                ta.fx_scale[k] = (float)(box.L[k] / 4294967296.0);
+            ta.grid = g;
+            ta.cell_of = nl->cell_of.ptr;
+            ta.n_neigh = nl->n_neigh.ptr;
+            ta.max_neighbors = nl->max_neighbors;
+            ta.flags = nl->flags.ptr;
+            ta.pitch = nl->pitch;
+            ta.group_cell_cap = nl->group_cells;
+            ta.group_batch_cap = nl->group_batches;
+            ta.sizes = size_bits;
+            AZP_TRY(tiles_rows(nl->tiles, ta, uniform, s));
+            ++nl->row_runs;
+            bool grown = false, fresh = true;
+            for (uint32_t q = 0; q < nsizes;)
                 {
-                if (nl->tile_mode != 1 && nl->tile_mode != ts)
-                    continue;
-                uint32_t& skip = nl->walk_skip[ts == 512u ? 0 : 1];
-                if (skip > 0)
-                    {
-                    --skip;
-                    continue;
-                    }
-                hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, nl->flags.ptr, 0u, (size_t)6);
-                hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, nl->flags.ptr + kTileFlagCells, 0u, (size_t)3);
-                TileWalkArgs ta;
-                ta.g.pos = pos;
-                ta.g.members = nl->members.ptr;
-                ta.g.start = nl->start.ptr;
-                ta.g.cell_rank = nl->cell_rank.ptr;
-                ta.g.cell_fixed = nl->cell_fixed.ptr;
-                ta.g.r_listsq = nl->r_listsq.ptr;
-                ta.g.ntypes = nl->ntypes;
-                ta.g.r_max = (float)rmax;
-                ta.g.thr = (float)(rmax * rmax);
-                ta.g.direct = false;
-                ta.N = N;
-                ta.box = box;
-                for (int k = 0; k < 3; ++k)
-                    ta.fx_scale[k] = (float)(box.L[k] / 4294967296.0);
-                ta.grid = g;
-                ta.cell_of = nl->cell_of.ptr;
-                ta.n_neigh = nl->n_neigh.ptr;
-                ta.max_neighbors = nl->max_neighbors;
-                ta.flags = nl->flags.ptr;
-                ta.pitch = nl->pitch;
-                ta.group_cell_cap = nl->group_cells;
-                ta.group_batch_cap = nl->group_batches;
+                const uint32_t ts = sizes[q];
+                if (!fresh)
+                    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, nl->flags.ptr + kTileFlagMisfit, 0u,
+                                       (size_t)4);
+                fresh = false;
                 ta.table_cap = nl->tile_table;
-                AZP_TRY(tiles_walk(nl->tiles, ts, ta, uniform, s));
-                ++nl->row_runs;
+                AZP_TRY(tiles_compact(nl->tiles, ts, ta, s));
                 ++nl->compactions;
                 // the positions of this build, queued before the flags are
                 // read so that no host round trip separates it from the walk
@@ -576,59 +631,63 @@ static int nlist_build(azp_nlist* nl, const azp_particles* p, hipStream_t s)
                 AZP_LAUNCH_CHECK();
                 AZP_HIP(hipMemcpyAsync(nl->h_flags, nl->flags.ptr, kTileFlags * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
                 AZP_HIP(hipStreamSynchronize(s));
-                if (nl->h_flags[2] & 2u)
-                    return set_error(AZP_ERR_INVALID, "a particle position is not finite (NaN or inf)");
-                if (nl->h_flags[2] & 1u)
-                    return set_error(AZP_ERR_INVALID,
-                                     "a particle type index is outside [0, %u) (pos.w must hold the type)",
-                                     nl->ntypes);
-                if (nl->h_flags[kTileFlagBatches] > kGroupBatchesMax)
-                    nl->h_flags[kTileFlagMisfit] |= 2u;
-                else if (nl->h_flags[kTileFlagCells] != 0u || nl->h_flags[kTileFlagBatches] != 0u)
+                const uint32_t* f = nl->h_flags;
+                AZP_TRY(bad_particle(f[kTileFlagBad], nl->ntypes));
+                nl->span = f[kTileFlagSpan];
+                if (f[kTileFlagBatches] > kGroupBatchesMax)
                     {
-                    // a group ran out of room (every count above is valid)
-                    nl->group_cells = std::min(kGroupCellsMax,
-                                               std::max(nl->group_cells, nl->h_flags[kTileFlagCells] * 5 / 4));
-                    nl->group_batches = std::min(kGroupBatchesMax,
-                                                 std::max(nl->group_batches, nl->h_flags[kTileFlagBatches] * 5 / 4));
-                    grown = true;
-                    }
-                if (nl->h_flags[kTileFlagTable] != 0u && nl->h_flags[kTileFlagMisfit] == 0u)
-                    {
-                    nl->tile_table = std::min(kTileTableMax, (nl->h_flags[kTileFlagTable] * 9u / 8u + 511u) & ~511u);
-                    grown = true;
-                    }
-                if (nl->h_flags[0] != 0u)
-                    grown = true;
-                if (grown)
+                    // no tile holds such a group
+                    for (uint32_t r = q; r < nsizes; ++r)
+                        nl->walk_skip[sizes[r] == 512u ? 0 : 1] = 8;
                     break;
-                if (nl->h_flags[3] == 0u)
+                    }
+                const bool misfit = f[kTileFlagMisfit] != 0u || (nl->span & span_bit(ts)) != 0u;
+                uint32_t next = q + 1;
+                while (next < nsizes && (nl->span & span_bit(sizes[next])))
+                    ++next;
+                if (!misfit || next < nsizes)
+                    {
+                    // a group that ran out of room left its rows out (every
+                    // count above is valid): the rows again with more
+                    grown = f[kTileFlagOverflow] != 0u || f[kTileFlagCells] != 0u || f[kTileFlagBatches] != 0u;
+                    if (grown)
+                        break;
+                    }
+                if (!misfit && f[kTileFlagTable] != 0u)
+                    {
+                    nl->tile_table = std::min(kTileTableMax, (f[kTileFlagTable] * 9u / 8u + 511u) & ~511u);
+                    continue; // this size again with larger tables
+                    }
+                if (!misfit)
                     {
                     nl->tiles.size = ts;
-                    nl->tiles.slots = nl->h_flags[4] + 1u;
+                    nl->tiles.slots = f[kTileFlagLargest] + 1u;
                     nl->tiles.valid = true;
                     nl->plain_ready = false;
                     nl->fused = true;
-                    nl->relative_tiles = nl->h_flags[5];
-                    done = true;
-                    break;
+                    nl->relative_tiles = f[kTileFlagRelative];
+                    nl->built_N = N;
+                    nl->built_box = p->box;
+                    nl->have_list = true;
+                    nl->n_builds++;
+                    return AZP_OK;
                     }
-                skip = 8; // a tile did not fit: plain walk for the next builds
+                nl->walk_skip[ts == 512u ? 0 : 1] = 8;
+                q = next; // from the same rows
                 }
             if (grown)
                 {
-                if (nl->h_flags[0] != 0u)
-                    nl->max_neighbors = ((uint32_t)(nl->h_flags[0] * 1.1) + 8u) & ~7u;
+                const uint32_t* f = nl->h_flags;
+                if (f[kTileFlagCells] != 0u || f[kTileFlagBatches] != 0u)
+                    {
+                    nl->group_cells = std::min(kGroupCellsMax, std::max(nl->group_cells, f[kTileFlagCells] * 5 / 4));
+                    nl->group_batches = std::min(kGroupBatchesMax, std::max(nl->group_batches, f[kTileFlagBatches] * 5 / 4));
+                    }
+                if (f[kTileFlagOverflow] != 0u)
+                    nl->max_neighbors = ((uint32_t)(f[kTileFlagOverflow] * 1.1) + 8u) & ~7u;
                 continue;
                 }
-            if (done)
-                {
-                nl->built_N = N;
-                nl->built_box = p->box;
-                nl->have_list = true;
-                nl->n_builds++;
-                return AZP_OK;
-                }
+            nsizes = 0; // no size fits: this build's list comes from the plain walk
             }
         AZP_TRY(nl->rows.reserve((size_t)nl->max_neighbors * N));
         hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, nl->flags.ptr, 0u, (size_t)3);
@@ -660,14 +719,11 @@ static int nlist_build(azp_nlist* nl, const azp_particles* p, hipStream_t s)
         hipLaunchKernelGGL(k_list_columns, dim3(grid_for(N, 64)), dim3(64), 0, s, N, nl->n_neigh.ptr, nl->rows.ptr,
                            nl->max_neighbors, nl->list.ptr, nl->pitch);
         AZP_LAUNCH_CHECK();
-        AZP_HIP(hipMemcpyAsync(nl->h_flags, nl->flags.ptr, 3 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+        AZP_HIP(hipMemcpyAsync(nl->h_flags, nl->flags.ptr, kTileFlags * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
         AZP_HIP(hipStreamSynchronize(s));
-        if (nl->h_flags[2] & 2u)
-            return set_error(AZP_ERR_INVALID, "a particle position is not finite (NaN or inf)");
-        if (nl->h_flags[2] & 1u)
-            return set_error(AZP_ERR_INVALID,
-                             "a particle type index is outside [0, %u) (pos.w must hold the type)",
-                             nl->ntypes);
+        AZP_TRY(bad_particle(nl->h_flags[kTileFlagBad], nl->ntypes));
+        if (nl->want_tiles)
+            nl->span = nl->h_flags[kTileFlagSpan];
         const uint32_t need = nl->h_flags[0];
         if (need == 0)
             {
@@ -822,7 +878,7 @@ static int nlist_update(azp_nlist* nl, const azp_particles* p, int force_rebuild
         // it lands) instead of waiting for the stream: the step's critical
         // path then skips the wake-up of a blocking synchronization.  After
         // 2 ms it falls back to synchronizing the stream.
-        const uint32_t w = prechecked ? 6u : 1u;
+        const uint32_t w = prechecked ? kFlagStep : 1u;
         volatile uint32_t* hflag = nl->h_flags + w;
         *hflag = kFlagPending;
         std::atomic_thread_fence(std::memory_order_seq_cst);
@@ -895,13 +951,13 @@ int nlist_step_check(azp_nlist* nl, hipStream_t s, StepKernelArgs* k)
     // before the numbers would pass 2^30 (the flag holds seq << 2)
     if (nl->step_seq == 0 || nl->step_seq >= (1u << 30) - 1u)
         {
-        hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, nl->flags.ptr + 6, 0u, (size_t)1);
+        hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, nl->flags.ptr + kFlagStep, 0u, (size_t)1);
         AZP_LAUNCH_CHECK();
         nl->step_seq = 0;
         }
     ++nl->step_seq;
     k->last = nl->last_pos.ptr;
-    k->flag = nl->flags.ptr + 6;
+    k->flag = nl->flags.ptr + kFlagStep;
     k->seq = nl->step_seq;
     const double half = 0.5 * nl->r_buff;
     k->thresh_sq = half * half;

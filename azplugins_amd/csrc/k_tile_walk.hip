@@ -37,9 +37,6 @@ namespace azp
 constexpr uint32_t kTileCand = 6144;
 constexpr uint32_t kUnionCells = 512; // distinct non-empty cells around one tile
 constexpr uint32_t kCellHash = 1024;  // open-addressing table of those cells
-// A tile whose slots span more cells than this (about four particles a cell
-// or fewer) is left to the plain walk: its union outgrows the hash.
-constexpr uint32_t kOwnCells = 128;
 
 __device__ __forceinline__ uint32_t cell_hash(uint32_t c)
     {
@@ -108,8 +105,9 @@ template<int ONEHOT> __global__ void __launch_bounds__(64 * kGroupWaves, 4) k_gr
     __shared__ uint16_t s_first[kGroupWaves][kRowBuffer * 64];
     const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     const uint32_t group = xcd_logical_block() * kGroupWaves + w;
-    if (group * 64u >= a.N)
-        return; // the whole wavefront (no barrier below spans wavefronts)
+    // the whole wavefront leaves (no barrier below spans wavefronts)
+    if (group * 64u >= a.N || (a.flags[kTileFlagSpan] & a.sizes) == a.sizes)
+        return;
     GroupColumn me;
     me.slot = group * 64u + lane;
     me.valid = me.slot < a.N;
@@ -249,11 +247,13 @@ template<uint32_t T> __global__ void __launch_bounds__(T, T == 512 ? 4 : 2) k_ti
     __shared__ uint16_t s_mark[C];
     extern __shared__ uint64_t s_ucell[]; // union cells until the rank tables take their place
     __shared__ uint32_t s_wave[NW], s_nc[G], s_nb[G], s_base[G + 1];
-    __shared__ uint32_t s_n, s_bad, s_direct, s_rfirst, s_rlast;
+    __shared__ uint32_t s_n, s_bad, s_direct;
     uint32_t* s_key = s_hash;
     uint16_t* s_val = reinterpret_cast<uint16_t*>(s_hash + kCellHash);
     uint16_t* s_table = reinterpret_cast<uint16_t*>(s_ucell);
 
+    if (a.flags[kTileFlagSpan] & (T == 512u ? kTileSpan512 : kTileSpan256))
+        return; // a tile of this size spans too many cells: the host sees the flag
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t t = xcd_logical_block();
     const uint32_t slot = t * T + tid;
@@ -266,12 +266,7 @@ template<uint32_t T> __global__ void __launch_bounds__(T, T == 512 ? 4 : 2) k_ti
     for (uint32_t k = tid; k < C; k += T)
         s_mark[k] = 0u;
     if (tid == 0)
-        {
         s_n = s_bad = s_direct = 0u;
-        s_rfirst = a.g.cell_rank[a.cell_of[i]];
-        }
-    if (active && (tid == T - 1 || slot == a.N - 1))
-        s_rlast = a.g.cell_rank[a.cell_of[i]];
     __syncthreads();
     if (tid < ng)
         {
@@ -318,8 +313,7 @@ template<uint32_t T> __global__ void __launch_bounds__(T, T == 512 ? 4 : 2) k_ti
     __syncthreads();
     const uint32_t U = s_n, entries = s_base[ng];
     // every thread leaves together: the conditions are shared
-    const uint32_t misfit = (s_rlast - s_rfirst + 1u > kOwnCells ? 8u : 0u) | ((s_bad != 0u || U > kUnionCells) ? 1u : 0u)
-                            | (entries > kTileTableMax ? 2u : 0u);
+    const uint32_t misfit = ((s_bad != 0u || U > kUnionCells) ? 1u : 0u) | (entries > kTileTableMax ? 2u : 0u);
     if (misfit != 0u || U == 0u || entries > a.table_cap)
         {
         if (tid == 0)
@@ -636,25 +630,9 @@ __global__ void __launch_bounds__(64) k_tiles_to_plain(uint32_t N,
         }
     }
 
-int tiles_walk(TileList& t, uint32_t tile_size, const TileWalkArgs& args, bool uniform, hipStream_t s)
+// The launch arguments with t's arrays.
+static TileWalkArgs tile_args(const TileList& t, const TileWalkArgs& args)
     {
-    if (tile_size != 256 && tile_size != 512)
-        return set_error(AZP_ERR_INVALID, "tile size %u must be 256 or 512", tile_size);
-    if (args.g.ntypes == 0 || args.g.ntypes > kTileWalkMaxTypes)
-        return set_error(AZP_ERR_UNSUPPORTED, "the per-tile walk serves 1 to %u particle types", kTileWalkMaxTypes);
-    const uint32_t ntiles = (args.N + tile_size - 1) / tile_size;
-    const uint32_t words = (((args.max_neighbors + 7u) & ~7u) + 1u) / 2u;
-    const size_t groups = ((size_t)args.N + 63) / 64;
-    AZP_TRY(t.count.reserve(ntiles));
-    AZP_TRY(t.jset.reserve((size_t)ntiles * kTileCap));
-    AZP_TRY(t.list.reserve((size_t)words * args.pitch));
-    AZP_TRY(t.nn.reserve(args.N));
-    AZP_TRY(t.order_buf.reserve(args.N));
-    AZP_TRY(t.col.reserve(args.N));
-    AZP_TRY(t.group_cells.reserve(groups * args.group_cell_cap));
-    AZP_TRY(t.group_rows.reserve((size_t)args.N * args.max_neighbors));
-    AZP_TRY(t.group_used.reserve(groups * args.group_batch_cap * 2));
-    AZP_TRY(t.group_meta.reserve(groups));
     TileWalkArgs a = args;
     a.tile_nn = t.nn.ptr;
     a.tile_order = t.order_buf.ptr;
@@ -666,6 +644,19 @@ int tiles_walk(TileList& t, uint32_t tile_size, const TileWalkArgs& args, bool u
     a.group_rows = t.group_rows.ptr;
     a.group_used = t.group_used.ptr;
     a.group_meta = t.group_meta.ptr;
+    return a;
+    }
+
+int tiles_rows(TileList& t, const TileWalkArgs& args, bool uniform, hipStream_t s)
+    {
+    if (args.g.ntypes == 0 || args.g.ntypes > kTileWalkMaxTypes)
+        return set_error(AZP_ERR_UNSUPPORTED, "the per-tile walk serves 1 to %u particle types", kTileWalkMaxTypes);
+    const size_t groups = ((size_t)args.N + 63) / 64;
+    AZP_TRY(t.group_cells.reserve(groups * args.group_cell_cap));
+    AZP_TRY(t.group_rows.reserve((size_t)args.N * args.max_neighbors));
+    AZP_TRY(t.group_used.reserve(groups * args.group_batch_cap * 2));
+    AZP_TRY(t.group_meta.reserve(groups));
+    const TileWalkArgs a = tile_args(t, args);
     const dim3 grid(grid_for(groups, kGroupWaves)), block(64 * kGroupWaves);
     if (uniform)
         hipLaunchKernelGGL(k_group_rows<0>, grid, block, 0, s, a);
@@ -673,15 +664,31 @@ int tiles_walk(TileList& t, uint32_t tile_size, const TileWalkArgs& args, bool u
         hipLaunchKernelGGL(k_group_rows<1>, grid, block, 0, s, a);
     else
         hipLaunchKernelGGL(k_group_rows<4>, grid, block, 0, s, a);
-    if (a.table_cap < kTileTable || a.table_cap > kTileTableMax)
-        return set_error(AZP_ERR_INVALID, "rank tables of %u entries", a.table_cap);
-    // gfx950 gives a workgroup 160 KiB of LDS; set on every launch (a host-side
-    // attribute, no device work), so no switch is shared between threads
+    AZP_LAUNCH_CHECK();
+    return AZP_OK;
+    }
+
+int tiles_compact(TileList& t, uint32_t tile_size, const TileWalkArgs& args, hipStream_t s)
+    {
+    if (tile_size != 256 && tile_size != 512)
+        return set_error(AZP_ERR_INVALID, "tile size %u must be 256 or 512", tile_size);
+    if (args.table_cap < kTileTable || args.table_cap > kTileTableMax)
+        return set_error(AZP_ERR_INVALID, "rank tables of %u entries", args.table_cap);
+    const uint32_t ntiles = (args.N + tile_size - 1) / tile_size;
+    const uint32_t words = (((args.max_neighbors + 7u) & ~7u) + 1u) / 2u;
+    AZP_TRY(t.count.reserve(ntiles));
+    AZP_TRY(t.jset.reserve((size_t)ntiles * kTileCap));
+    AZP_TRY(t.list.reserve((size_t)words * args.pitch));
+    AZP_TRY(t.nn.reserve(args.N));
+    AZP_TRY(t.order_buf.reserve(args.N));
+    AZP_TRY(t.col.reserve(args.N));
+    const TileWalkArgs a = tile_args(t, args);
+    // gfx950 gives a workgroup 160 KiB of LDS; the largest size on every launch
+    // (a host-side attribute, no device work), so threads agree on it
     const size_t lds = (size_t)a.table_cap * sizeof(uint16_t);
     const void* kernel = tile_size == 512 ? reinterpret_cast<const void*>(&k_tile_compact<512>)
                                           : reinterpret_cast<const void*>(&k_tile_compact<256>);
-    if (lds > 40 * 1024)
-        AZP_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kTileTableMax * sizeof(uint16_t))));
+    AZP_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kTileTableMax * sizeof(uint16_t))));
     if (tile_size == 512)
         hipLaunchKernelGGL(k_tile_compact<512>, dim3(ntiles), dim3(512), lds, s, a);
     else

@@ -72,16 +72,25 @@ int tiles_build(TileList& t,
                 uint32_t* h_flag,
                 hipStream_t stream);
 
-// Flag words of the per-tile walk.
+// Flag words of a neighbor list's builds ([1] is the rebuild check, the last
+// one the step kernel's).  Words 3 to 6 are the compaction's.
 constexpr uint32_t kTileFlagOverflow = 0; // largest count above max_neighbors
 constexpr uint32_t kTileFlagBad = 2;      // bad type (1) / position (2)
-constexpr uint32_t kTileFlagMisfit = 3;   // a tile did not fit (1: cells, 2: candidates, 4: neighbor set, 8: own cells)
+constexpr uint32_t kTileFlagMisfit = 3;   // a tile did not fit (1: cells, 2: candidates, 4: neighbor set)
 constexpr uint32_t kTileFlagLargest = 4;  // largest neighbor-set size
 constexpr uint32_t kTileFlagRelative = 5; // tiles tested on the matrix cores throughout
+constexpr uint32_t kTileFlagTable = 6;    // most rank-table entries of a tile beyond table_cap
 constexpr uint32_t kTileFlagCells = 7;    // most cells of a group beyond group_cell_cap
 constexpr uint32_t kTileFlagBatches = 8;  // most batches of a group beyond group_batch_cap
-constexpr uint32_t kTileFlagTable = 9;    // most rank-table entries of a tile beyond table_cap
-constexpr uint32_t kTileFlags = 10;       // (word 6 belongs to the step kernel's check)
+constexpr uint32_t kTileFlagSpan = 9;     // sizes with a tile of more than kOwnCells cells (kTileSpan512, kTileSpan256)
+constexpr uint32_t kTileFlags = 10;
+constexpr uint32_t kFlagStep = kTileFlags; // the step kernel's rebuild check
+constexpr uint32_t kTileSpan512 = 1, kTileSpan256 = 2;
+
+// A tile whose slots span more cells than this (about four particles a cell
+// or fewer at 512 slots) is left to the plain walk: its union outgrows the
+// compaction's hash.
+constexpr uint32_t kOwnCells = 128;
 
 // Inputs and outputs of the per-tile walk (k_tile_walk.hip): the cell list
 // (cell_of, members, the cell-ordered fixed-point copy) and the list radii;
@@ -100,7 +109,8 @@ struct TileWalkArgs
     uint32_t* flags;
     uint32_t pitch;
     uint32_t group_cell_cap, group_batch_cap, table_cap;
-    // set by tiles_walk
+    uint32_t sizes; // kTileSpan512 | kTileSpan256: the tile sizes that this build may use
+    // set by tiles_rows / tiles_compact
     uint2* group_cells;    // by group: first slot, first candidate | members << 16 of each cell
     uint32_t* group_used;  // by group and batch of 64 candidates: two words
     uint16_t* group_rows;  // by slot: the candidate numbers of its entries
@@ -125,13 +135,17 @@ constexpr uint32_t kGroupBatchesMax = kTileTableMax / 64 / 4;
 // Most cells it lists: a pass visits at most 27 for each column that it serves.
 constexpr uint32_t kGroupCellsMax = 64 * 27;
 
-// Enqueues the per-tile walk with tiles of `tile_size` (256 or 512) particles
-// into t's arrays (sized here); the caller reads args.flags afterwards and
-// sets t.size / t.slots / t.valid when no misfit is flagged.  `uniform`: one
-// list radius for every type pair.
-int tiles_walk(TileList& t, uint32_t tile_size, const TileWalkArgs& args, bool uniform, hipStream_t stream);
+// Enqueues the groups' rows (which no tile size enters) into t's arrays, sized
+// here; nothing is done if the span flags rule out every size of args.sizes.
+// `uniform`: one list radius for every type pair.
+int tiles_rows(TileList& t, const TileWalkArgs& args, bool uniform, hipStream_t stream);
 
-// Most particle types tiles_walk serves.
+// Enqueues the tiled list with tiles of `tile_size` (256 or 512) particles from
+// the rows; the caller reads args.flags afterwards and sets t.size / t.slots /
+// t.valid when no misfit is flagged.
+int tiles_compact(TileList& t, uint32_t tile_size, const TileWalkArgs& args, hipStream_t stream);
+
+// Most particle types the per-tile walk serves.
 constexpr uint32_t kTileWalkMaxTypes = 8;
 
 // Enqueues the expansion of a valid tiled list of the per-tile walk into the

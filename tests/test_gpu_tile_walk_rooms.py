@@ -76,3 +76,37 @@ def test_rooms_grow():
     nl.update(sysm.particles(), force_rebuild=True)
     torch.cuda.synchronize()
     assert nl.walk_runs() == (rows + 1, compactions + 1)
+
+
+def test_rows_serve_both_tile_sizes():
+    """At less than three particles a cell 512 slots span more than 128 cells: the rows are
+    made once and the second size compacts them; later builds go to it at once.
+    A list that served a dense system before has fewer rooms for cells and
+    grows them."""
+    dense, sparse = _fluid(6000, 0.416, 1), _fluid(12000, 1.0, 2)
+    nl = _new(1.0, True)
+    _update(nl, sparse)
+    assert nl.walk_kind() == 1 and nl.get_tiles()[3] == 256
+    assert nl.walk_runs() == (1, 2)
+    _same_as_plain(nl, sparse, 1.0)
+    for n in range(1, 12):
+        nl.update(sparse.particles(), force_rebuild=True)
+        assert nl.walk_kind() == 1 and nl.walk_runs() == (1 + n, 2 + n)
+    nl = _new(5.5, True)
+    _update(nl, dense)
+    assert nl.walk_kind() == 1
+    rows = nl.walk_runs()[0]
+    nl.set_r_cut(1, [1.0])
+    _update(nl, sparse)
+    assert nl.walk_kind() == 1 and nl.walk_runs()[0] == rows + 2
+    _same_as_plain(nl, sparse, 1.0)
+
+
+def test_sparse_cells_leave_the_walk_alone():
+    """Below two particles a cell no tile size fits: found before the rows, once."""
+    sysm = _fluid(20000, 0.5, 3)
+    nl = _new(1.0, True)
+    for n in range(12):
+        nl.update(sysm.particles(), force_rebuild=True)
+        assert nl.walk_kind() == 0 and nl.walk_runs() == (1, 1)
+    _same_as_plain(nl, sysm, 1.0)
