@@ -88,16 +88,11 @@ __global__ void __launch_bounds__(512) k_aniso(const AnisoKernelArgs a)
         tpm_list_queued<VIRIAL, SINGLE>(nn, lane.sub, split, row, stride, queue, a.pos, a.orientation, me, box, nt, q0,
                                         s_q, acc);
         }
-    if (split != 0u)
-        {
-        for (double* v : {&acc.fx, &acc.fy, &acc.fz, &acc.tx, &acc.ty, &acc.tz, &acc.pe})
-            *v = split_sum(*v, split);
-        if (VIRIAL)
-            {
-            for (double* v : {&acc.v0, &acc.v1, &acc.v2, &acc.v3, &acc.v4, &acc.v5})
-                *v = split_sum(*v, split);
-            }
-        }
+    if (VIRIAL)
+        split_sum(split, acc.fx, acc.fy, acc.fz, acc.tx, acc.ty, acc.tz, acc.pe, acc.v0, acc.v1, acc.v2, acc.v3, acc.v4,
+                  acc.v5);
+    else
+        split_sum(split, acc.fx, acc.fy, acc.fz, acc.tx, acc.ty, acc.tz, acc.pe);
     if (i < a.N && lane.sub == 0u)
         aniso_store<VIRIAL>(a.force, a.torque, a.virial, a.vpitch, i, acc);
     }

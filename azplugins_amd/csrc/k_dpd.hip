@@ -251,13 +251,10 @@ __global__ void __launch_bounds__(512, 4) k_dpd(const DPDKernelArgs a)
         }
     if constexpr (SPLIT)
         {
-        for (double* v : {&fx, &fy, &fz, &pe})
-            *v = split_sum(*v, split);
         if (VIRIAL)
-            {
-            for (double* v : {&v0, &v1, &v2, &v3, &v4, &v5})
-                *v = split_sum(*v, split);
-            }
+            split_sum(split, fx, fy, fz, pe, v0, v1, v2, v3, v4, v5);
+        else
+            split_sum(split, fx, fy, fz, pe);
         if (lane.sub != 0u)
             return;
         }
@@ -424,13 +421,10 @@ __global__ void __launch_bounds__(512, 4) k_dpd_tiled(const DPDKernelArgs a)
         }
     if constexpr (SPLIT)
         {
-        for (double* v : {&fx, &fy, &fz, &pe_sum})
-            *v = split_sum(*v, split);
         if (VIRIAL)
-            {
-            for (double* v : {&v0, &v1, &v2, &v3, &v4, &v5})
-                *v = split_sum(*v, split);
-            }
+            split_sum(split, fx, fy, fz, pe_sum, v0, v1, v2, v3, v4, v5);
+        else
+            split_sum(split, fx, fy, fz, pe_sum);
         if (lane.sub != 0u)
             return;
         }

@@ -93,12 +93,52 @@ template<bool SPLIT> struct LaneEntries
         }
     };
 
-// Sum over a particle's lanes, the same value in each of them.
-__device__ __forceinline__ double split_sum(double v, uint32_t split)
+// v plus its value in the lane `across` away (32, 16, 8 or 4).  Register swaps
+// and row operations: only the two lanes of a pair read each other, so the
+// lanes of a column without a particle may have left.
+template<int across> __device__ __forceinline__ double add_across(double v)
     {
-    for (uint32_t m = 32; m >= (64u >> split); m >>= 1)
-        v += __shfl_xor(v, (int)m);
-    return v;
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    if constexpr (across == 32 || across == 16)
+        {
+        const auto swap = [](int x) {
+            if constexpr (across == 32)
+                return __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)x, false, false);
+            else
+                return __builtin_amdgcn_permlane16_swap((uint32_t)x, (uint32_t)x, false, false);
+        };
+        const auto l = swap(lo), h = swap(hi);
+        return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
+        }
+    else
+        {
+        const auto other = [](int x) {
+            if constexpr (across == 8)
+                return __builtin_amdgcn_update_dpp(0, x, 0x128, 0xf, 0xf, false); // row_ror:8
+            else
+                {
+                const int up = __builtin_amdgcn_update_dpp(0, x, 0x104, 0xf, 0x5, false);  // row_shl:4, lanes with bit 2 clear
+                return __builtin_amdgcn_update_dpp(up, x, 0x114, 0xf, 0xa, false);         // row_shr:4, the others
+                }
+        };
+        return v + __hiloint2double(other(hi), other(lo));
+        }
+    }
+
+// Sums over a particle's lanes, the same values in each of them.  All values
+// take a stage before the next: one after the other, the exchanges' latencies
+// added up to 2 us.
+template<class... D> __device__ __forceinline__ void split_sum(uint32_t split, D&... v)
+    {
+    static_assert(kSplitMax == 4, "stages of the sum");
+    if (split > 0u)
+        ((v = add_across<32>(v)), ...);
+    if (split > 1u)
+        ((v = add_across<16>(v)), ...);
+    if (split > 2u)
+        ((v = add_across<8>(v)), ...);
+    if (split > 3u)
+        ((v = add_across<4>(v)), ...);
     }
 
 } // namespace azp

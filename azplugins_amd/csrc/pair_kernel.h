@@ -415,19 +415,10 @@ template<class Eval> static bool tile_fits64(uint32_t ntypes, uint32_t slots)
 
 template<bool VIRIAL> __device__ __forceinline__ void split_sum(Acc& acc, uint32_t split)
     {
-    acc.fx = split_sum(acc.fx, split);
-    acc.fy = split_sum(acc.fy, split);
-    acc.fz = split_sum(acc.fz, split);
-    acc.e = split_sum(acc.e, split);
     if (VIRIAL)
-        {
-        acc.v0 = split_sum(acc.v0, split);
-        acc.v1 = split_sum(acc.v1, split);
-        acc.v2 = split_sum(acc.v2, split);
-        acc.v3 = split_sum(acc.v3, split);
-        acc.v4 = split_sum(acc.v4, split);
-        acc.v5 = split_sum(acc.v5, split);
-        }
+        split_sum(split, acc.fx, acc.fy, acc.fz, acc.e, acc.v0, acc.v1, acc.v2, acc.v3, acc.v4, acc.v5);
+    else
+        split_sum(split, acc.fx, acc.fy, acc.fz, acc.e);
     }
 
 // Neighbor-list layouts a kernel instance reads.
