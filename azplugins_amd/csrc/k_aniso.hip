@@ -175,7 +175,7 @@ extern "C" int azp_gpu_compute_pair_aniso_forces(const azp_pair_args* args, int 
     ka.torque = reinterpret_cast<double4*>(args->out.d_torque);
     ka.virial = args->out.d_virial;
     ka.vpitch = args->out.virial_pitch;
-    ka.split = split_for(p.N, mixed ? SplitTerm::Light : SplitTerm::Fp64);
+    ka.split = split_for(p.N, mixed ? SplitTerm::Aniso : SplitTerm::AnisoFp64, args->ntypes);
     const unsigned block = args->block_size ? args->block_size : 256;
     hipStream_t s = (hipStream_t)args->stream;
     if (mixed && !ka.pos_fixed)

@@ -540,7 +540,7 @@ extern "C" int azp_gpu_compute_dpd_forces(const azp_pair_args* args, const void*
     ka.force = reinterpret_cast<double4*>(args->out.d_force);
     ka.virial = args->out.d_virial;
     ka.vpitch = args->out.virial_pitch;
-    ka.split = split_for(p.N, SplitTerm::Light);
+    ka.split = split_for(p.N, SplitTerm::Dpd, args->ntypes);
     hipStream_t s = (hipStream_t)args->stream;
     if (args->d_tile_list && !args->d_head_list && dpd_tile_fits(args->ntypes, args->tile_slots, args->tile_size))
         {
@@ -561,7 +561,18 @@ extern "C" int azp_gpu_compute_dpd_forces(const azp_pair_args* args, const void*
             block = args->tile_size;
         while ((block << ka.part_shift) < (args->tile_size << ka.split))
             ++ka.part_shift;
-        const size_t shmem = dpd_tile_lds(args->ntypes, args->tile_slots, block, kDpdTileQueue);
+        // a lane of a split holds half as many in-cut ranks or fewer: a shorter
+        // queue where that lets a CU take two workgroups (129,000 to 131,000
+        // particles, 2,040 to 2,145 slots: 49 to 52 us with one, 42 to 47 with
+        // two, 46 to 49 unsplit)
+        if (ka.split != 0)
+            for (uint32_t q = kDpdTileQueue; q >= kDpdTileQueue / 2; q -= 4)
+                if (dpd_tile_lds(args->ntypes, args->tile_slots, block, q) <= kDpdTileLds / 2)
+                    {
+                    ka.queue_len = q;
+                    break;
+                    }
+        const size_t shmem = dpd_tile_lds(args->ntypes, args->tile_slots, block, ka.queue_len);
         const dim3 grid(grid_for(p.N, args->tile_size) << ka.part_shift);
         if (args->compute_virial)
             return ka.split ? launch_dpd_tiled<true, true>(ka, grid, block, shmem, s)

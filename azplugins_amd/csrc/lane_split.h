@@ -9,8 +9,9 @@
 // 64 >> split apart in one wavefront, so the list words that a wavefront reads
 // for one batch stay consecutive.
 //
-// The split depends on the number of particles and the pair term alone, so
-// every list layout adds a particle's terms in the same order.
+// The split depends on the number of particles, the pair term and (the mixed
+// pair form) the number of types alone, so every list layout adds a particle's
+// terms in the same order.
 #pragma once
 
 #include "device_common.h"
@@ -18,41 +19,62 @@
 namespace azp
 {
 
-// Lanes that a split fills the chip up to, by what a list entry costs.  Light
-// terms (the mixed form, DPD's scan) stop at four wavefronts a SIMD, since
-// each further workgroup of a tile stages the tile's neighbors again.  FP64
-// terms, whose registers leave two or three wavefronts a SIMD, take the second
-// lane for up to 229,376 particles: at 262,144 over the plain list it cost a
-// fifth.  Colloid's three divergent branches fill twice as many lanes.
-// Measured with 2^18 / 2^19 lanes (us): mixed PerturbedLJ 60,000 particles
-// 37.4 / 52.2, DPD 60,000 30.2 / 40.3, FP64 Yukawa 60,000 70.2 / 91.4 but
-// 150,000 162 / 142, FP64 TwoPatchMorse 130,000 98 / 105 but 200,000
-// 172 / 155, Colloid 20,000 56 / 51, 73,000 176 / 121 and 200,000 354 / 310
-// (332 with 2^20).  Against one lane per particle: Yukawa 900 particles
-// 85 -> 14.5, Colloid 73,000 200 -> 118, TwoPatchMorse 40,000 66 -> 38 and
-// DPD 60,000 37.5 -> 26.8.
+// Up to 65,536 particles a split fills 2^18 lanes (four wavefronts a SIMD):
+// Yukawa 900 particles 85 -> 12.4 us, DPD 60,000 37.5 -> 26.8, TwoPatchMorse
+// 40,000 66 -> 33.  Above, a second lane has to pay for itself by the kernel's
+// limits (us with one / two lanes):
+//   Pair      the mixed form of one type: PerturbedLJ 90,000 31.2 / 29.4.  With
+//             several types the table reads make it issue-bound: PerturbedLJ
+//             90,000 48.2 / 53.8, Yukawa 67 / 72.
+//   Short     Hertz, lists of about ten entries: four lanes hold them all, and
+//             the chip is full at 2^17 lanes (FP64 900 particles 9.1, two lanes
+//             8.3, four 8.3, sixteen 12.1; mixed 130,000 9.2 / 10.2).
+//   PairFp64  one 512-lane workgroup a CU (LDS, registers), so the chip runs
+//             rounds of 2^17 lanes, and two lanes gain where the rounds round
+//             down: 160,000 PerturbedLJ 103 / 91, Yukawa 165 / 145; 195,000
+//             92 / 75, 228 / 184; but PerturbedLJ of two types 90,000 62 / 71
+//             and 228,000 130 / 147.
+//   Dpd       70,000 45 / 38, 122,000 51 / 42.
+//   Aniso     mixed 100,000 57 / 47, 131,000 59 / 50.
+//   AnisoFp64 rounds of 2^16 lanes (one wavefront a SIMD at a time bound by
+//             FP64 issue): 90,000 80 / 66, 100,000 81 / 85, 140,000 113 / 104,
+//             180,000 115 / 122, 228,000 149 / 139.
+//   Colloid   three divergent branches fill twice as many lanes: 73,000
+//             200 -> 118, 20,000 56 / 51 with 2^18 / 2^19 lanes.
 enum class SplitTerm
     {
-    Light,
-    Fp64,
+    Pair,
+    Short,
+    PairFp64,
+    Dpd,
+    Aniso,
+    AnisoFp64,
     Colloid,
     };
 constexpr uint32_t kSplitLanes = 1u << 18;
 constexpr uint32_t kSplitMax = 4;
 
 // log2 of the lanes per particle.
-inline uint32_t split_for(uint32_t N, SplitTerm term)
+inline uint32_t split_for(uint32_t N, SplitTerm term, uint32_t ntypes)
     {
-    uint32_t split = 0;
-    while (split < kSplitMax)
+    const uint32_t lanes = term == SplitTerm::Colloid ? 2 * kSplitLanes
+                           : term == SplitTerm::Short ? kSplitLanes / 2
+                                                      : kSplitLanes;
+    const uint32_t most = term == SplitTerm::Short ? 2u : kSplitMax;
+    if (N > kSplitLanes / 4 && N <= kSplitLanes)
         {
-        const uint32_t lanes = term == SplitTerm::Colloid                ? 2 * kSplitLanes
-                               : term == SplitTerm::Fp64 && split == 0 ? kSplitLanes / 4 * 7
-                                                                       : kSplitLanes;
-        if (((uint64_t)N << (split + 1)) > lanes)
-            break;
-        ++split;
+        if (term == SplitTerm::Pair && ntypes > 1)
+            return 0;
+        if (term == SplitTerm::PairFp64 || term == SplitTerm::AnisoFp64)
+            {
+            // two lanes where that takes fewer half rounds
+            const uint32_t round = term == SplitTerm::PairFp64 ? kSplitLanes / 2 : kSplitLanes / 4;
+            return (2 * N + round - 1) / round < 2 * ((N + round - 1) / round) ? 1u : 0u;
+            }
         }
+    uint32_t split = 0;
+    while (split < most && ((uint64_t)N << (split + 1)) <= lanes)
+        ++split;
     return split;
     }
 

@@ -886,9 +886,12 @@ static int launch_t(const PairKernelArgs& ka, unsigned block, unsigned slots, hi
     const size_t cap = (TILED && !MIXED) ? kTileLds64 : kTileLds;
     if (shmem > cap)
         return set_error(AZP_ERR_UNSUPPORTED, "too many particle types (%u) for LDS staging", ka.ntypes);
-    kb.split = split_for(ka.N, std::is_same_v<Eval, EvalColloid> ? SplitTerm::Colloid
-                               : MIXED                           ? SplitTerm::Light
-                                                                 : SplitTerm::Fp64);
+    kb.split = split_for(ka.N,
+                         std::is_same_v<Eval, EvalColloid> ? SplitTerm::Colloid
+                         : std::is_same_v<Eval, EvalHertz> ? SplitTerm::Short
+                         : MIXED                           ? SplitTerm::Pair
+                                                           : SplitTerm::PairFp64,
+                         ka.ntypes);
     // the lanes' 32-bit byte offsets into the list reach over a step's rows
     while (kb.split != 0 && ((uint64_t)ka.nlist_pitch << (kb.split + 6)) > 0xffffffffull)
         --kb.split;

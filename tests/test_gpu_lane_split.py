@@ -1,10 +1,10 @@
 """Several lanes per particle (csrc/lane_split.h).
 
-Systems of at most 2^18 / 2^s particles get 2^s lanes each (s <= 4; the FP64
-terms two lanes up to 229,376).  The sizes lie on both sides of lines of that
-rule, with lists shorter than one lane's
-batch, ragged last tiles and columns without entries.  The split depends on N
-alone, so the plain and the tiled list give the same bits at every size; the
+Up to 65,536 particles, systems of at most 2^18 / 2^s get 2^s lanes each
+(s <= 4); above, the pair term decides about two.  The sizes lie on both sides
+of lines of that rule, with lists shorter than one lane's batch, ragged last
+tiles and columns without entries.  The split does not depend on the list's
+layout, so the plain and the tiled list give the same bits at every size; the
 oracle bounds the sums (FP64: a few hundred terms of 2^-53 each, 1e-12; mixed
 form: its FP32 terms, 1e-5).
 """
