@@ -25,6 +25,8 @@
 // 27 batches of 64 candidates, 3,500 in taking 139 entries out of the masks.
 // At 60,000 particles (DPD, density 3) 46 + 37 us against 98, at 4,096 37 + 53
 // against 100.
+#include <type_traits>
+
 #include "cells.h"
 #include "device_common.h"
 #include "group_walk.h"
@@ -33,8 +35,13 @@
 namespace azp
 {
 
-// Candidates of one tile (two bytes of LDS each).
-constexpr uint32_t kTileCand = 6144;
+// Candidates of one tile (two bytes of LDS each).  Tiles of 512 columns reach
+// 6,400 at 50 particles a cell (Yukawa: at about half of the system sizes) and
+// about 7,000 among colloids; they must not fall to 256 columns for that: the
+// FP64 pair kernel's workgroup is then 256 lanes, and one whose neighbors take
+// more than half of the LDS has its CU to itself (225,000 particles, two types:
+// 238 us against 216).
+constexpr uint32_t kTileCand = 9216;
 constexpr uint32_t kUnionCells = 512; // distinct non-empty cells around one tile
 constexpr uint32_t kCellHash = 1024;  // open-addressing table of those cells
 
@@ -263,8 +270,6 @@ template<uint32_t T> __global__ void __launch_bounds__(T, T == 512 ? 4 : 2) k_ti
 
     for (uint32_t k = tid; k < kCellHash; k += T)
         s_key[k] = 0xffffffffu;
-    for (uint32_t k = tid; k < C; k += T)
-        s_mark[k] = 0u;
     if (tid == 0)
         s_n = s_bad = s_direct = 0u;
     __syncthreads();
@@ -425,6 +430,11 @@ template<uint32_t T> __global__ void __launch_bounds__(T, T == 512 ? 4 : 2) k_ti
         }
     if (tid == 0)
         s_off[U] = (uint16_t)Mc;
+    // the marks that the scan reads (places that no cell fills point at the
+    // last one)
+    const uint32_t marks = Mc <= 12u * 512u ? 12u * 512u : C;
+    for (uint32_t k = tid; k < marks; k += T)
+        s_mark[k] = 0u;
     __syncthreads();
 
     // 4. each group's candidates by tile candidate number: a wavefront a
@@ -468,14 +478,46 @@ template<uint32_t T> __global__ void __launch_bounds__(T, T == 512 ? 4 : 2) k_ti
         }
     }
     __syncthreads();
-    // 6. ranks: exclusive scan of the marks; the neighbor set
-    constexpr uint32_t QM = C / T;
-    uint32_t msum = 0;
+    // 6. ranks: exclusive scan of the marks, a run of them per thread; the
+    // neighbor set
+    uint32_t M = 0;
+    auto rank = [&](auto per_thread) {
+        constexpr uint32_t QM = decltype(per_thread)::value;
+        uint32_t msum = 0;
 #pragma unroll
-    for (uint32_t q = 0; q < QM; ++q)
-        msum += s_mark[tid * QM + q];
-    uint32_t M;
-    uint32_t r = tile_scan<T>(msum, s_wave, M);
+        for (uint32_t q = 0; q < QM; ++q)
+            msum += s_mark[tid * QM + q];
+        uint32_t r = tile_scan<T>(msum, s_wave, M);
+        if (M > kTileCap - 1)
+            return;
+        // the union cell of the thread's first candidate, then onwards
+        uint32_t lo = 0, hi = U;
+        while (hi - lo > 1u)
+            {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (s_off[mid] <= tid * QM)
+                lo = mid;
+            else
+                hi = mid;
+            }
+#pragma unroll
+        for (uint32_t q = 0; q < QM; ++q)
+            {
+            const uint32_t m = tid * QM + q;
+            while (lo + 1u < U && s_off[lo + 1u] <= m)
+                ++lo;
+            if (s_mark[m] != 0u)
+                {
+                a.tile_jset[(size_t)t * kTileCap + r] = a.g.members[s_gs[lo] + (m - s_off[lo])];
+                s_mark[m] = (uint16_t)(r << 4); // entries are 16 x rank
+                ++r;
+                }
+            }
+    };
+    if (marks < C)
+        rank(std::integral_constant<uint32_t, 12u * 512u / T>{});
+    else
+        rank(std::integral_constant<uint32_t, C / T>{});
     if (M > kTileCap - 1)
         {
         if (tid == 0)
@@ -484,29 +526,6 @@ template<uint32_t T> __global__ void __launch_bounds__(T, T == 512 ? 4 : 2) k_ti
             a.tile_count[t] = 0u;
             }
         return; // M is the same for every thread
-        }
-    // the union cell of the thread's first candidate, then onwards
-    uint32_t lo = 0, hi = U;
-    while (hi - lo > 1u)
-        {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (s_off[mid] <= tid * QM)
-            lo = mid;
-        else
-            hi = mid;
-        }
-#pragma unroll
-    for (uint32_t q = 0; q < QM; ++q)
-        {
-        const uint32_t m = tid * QM + q;
-        while (lo + 1u < U && s_off[lo + 1u] <= m)
-            ++lo;
-        if (s_mark[m] != 0u)
-            {
-            a.tile_jset[(size_t)t * kTileCap + r] = a.g.members[s_gs[lo] + (m - s_off[lo])];
-            s_mark[m] = (uint16_t)(r << 4); // entries are 16 x rank
-            ++r;
-            }
         }
     if (tid == 0)
         {
