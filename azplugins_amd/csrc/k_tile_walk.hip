@@ -35,13 +35,13 @@
 namespace azp
 {
 
-// Candidates of one tile (two bytes of LDS each).  Tiles of 512 columns reach
-// 6,400 at 50 particles a cell (Yukawa: at about half of the system sizes) and
-// about 7,000 among colloids; they must not fall to 256 columns for that: the
-// FP64 pair kernel's workgroup is then 256 lanes, and one whose neighbors take
-// more than half of the LDS has its CU to itself (225,000 particles, two types:
-// 238 us against 216).
-constexpr uint32_t kTileCand = 9216;
+// Candidates of one tile (two bytes of LDS each).  512-column tiles of 50
+// particles a cell reach 6,600 (Yukawa, at a seventh of the system sizes), and
+// must not fall to 256 columns for that: the FP64 pair kernel's workgroup is
+// then 256 lanes, and one whose neighbors take more than half of the LDS has
+// its CU to itself (225,000 particles, two types: 238 us against 216).  Tiles
+// of colloids (7,000 to 9,500) are left to the plain walk and the hash build.
+constexpr uint32_t kTileCand = 6656;
 constexpr uint32_t kUnionCells = 512; // distinct non-empty cells around one tile
 constexpr uint32_t kCellHash = 1024;  // open-addressing table of those cells
 

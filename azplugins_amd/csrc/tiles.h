@@ -124,11 +124,11 @@ struct TileWalkArgs
     };
 
 // Rank-table entries (two bytes of LDS each) of a tile: with kTileTable two
-// tiles share a CU (80 KiB each with the 28 KB of the compaction's other
+// tiles share a CU (80 KiB each with the 22 KiB of the compaction's other
 // arrays); a build whose tiles need more compacts again with room for them, up
 // to one tile per CU.
-constexpr uint32_t kTileTable = 26624;
-constexpr uint32_t kTileTableMax = 67584;
+constexpr uint32_t kTileTable = 29568;
+constexpr uint32_t kTileTableMax = 69632;
 
 // Most batches of a group the walk makes room for: a 256-column tile of four
 // such groups fills the largest rank tables.

@@ -62,7 +62,7 @@ def test_small_dense_boxes(density, r_cut, N, tile):
 
 @pytest.mark.parametrize("density, r_cut, N", [(0.5, 4.0, 50000), (0.5, 4.0, 100000), (0.5, 4.0, 160000)])
 def test_candidates_of_wide_tiles(density, r_cut, N):
-    """512-column tiles of 6,145 to 9,216 candidates."""
+    """512-column tiles of 6,145 to 6,656 candidates."""
     sysm, _ = _lattice(density, N)
     walk, plain = _list(sysm, r_cut, True), _list(sysm, r_cut, False)
     assert walk.walk_kind() == 1 and walk.get_tiles()[3] == 512
