@@ -10,8 +10,9 @@
 // for one batch stay consecutive.
 //
 // The split depends on the number of particles, the pair term and (the mixed
-// pair form) the number of types alone, so every list layout adds a particle's
-// terms in the same order.
+// pair form) the number of types, not on the list's layout, so every layout adds
+// a particle's terms in the same order (up to pitches of 2^26 / 2^split: see
+// launch_t).
 #pragma once
 
 #include "device_common.h"

@@ -892,8 +892,10 @@ static int launch_t(const PairKernelArgs& ka, unsigned block, unsigned slots, hi
                          : MIXED                           ? SplitTerm::Pair
                                                            : SplitTerm::PairFp64,
                          ka.ntypes);
-    // the lanes' 32-bit byte offsets into the list reach over a step's rows
-    while (kb.split != 0 && ((uint64_t)ka.nlist_pitch << (kb.split + 6)) > 0xffffffffull)
+    // the lanes' 32-bit byte offsets into a column list reach over a step's
+    // rows: a pitch above 2^26 / 2^split gets fewer lanes (the head list's
+    // pitch is not read)
+    while (LAYOUT != kLayoutHead && kb.split != 0 && ((uint64_t)ka.nlist_pitch << (kb.split + 6)) > 0xffffffffull)
         --kb.split;
     // tiled: up to 512 lanes a workgroup, and as many workgroups as the tile's
     // lanes take, each staging the tile's neighbors for its own columns

@@ -123,3 +123,15 @@ def test_aniso_lines(N):
         assert rel_err(r.force, fo) < tol
         assert rel_err(r.torque[:, :3], to[:, :3]) < tol
         assert rel_err(r.virial, vo) < tol
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_head_list_pitch_is_not_read(precision):
+    """The head-list launch gives the same bits whatever nlist_pitch holds."""
+    pos4, Lv, _ = _slab(4097, 1.0, 2)
+    sysm = GpuSystem(pos4, Lv)
+    ref = gpu_pair(CLASSES[1], sysm, 2, PARAMS[1], 2.2, r_buff=0.2, precision=precision, r_on=0.0)
+    for pitch in (0, 1, 0xffffffff):
+        f, v = _head_force(sysm, ref, 1, 2, 2.2, 0.0, "none", precision, pitch)
+        assert np.array_equal(ref.force, f)
+        assert np.array_equal(ref.virial, v)
