@@ -329,12 +329,17 @@ template<bool MIXED> inline size_t tpm_queue_bytes(unsigned block)
     return MIXED ? 0 : (size_t)kTpmQueue * block * sizeof(uint32_t);
     }
 
+// Most dynamic LDS of the TwoPatchMorse kernels: the largest parameter table
+// (64 KiB) and the queue of 512 lanes.
+constexpr size_t kTpmLds = 64 * 1024 + kTpmQueue * 512 * sizeof(uint32_t);
+
 // Lets a kernel use more than 64 KiB of dynamic LDS (gfx950 gives a workgroup
-// 160 KiB; the largest table and the queue of 512 lanes take 96).
+// 160 KiB).  Every call sets the same size, so that no thread lowers it between
+// another's call and its launch.
 inline int tpm_raise_lds(const void* kernel, size_t shmem)
     {
     if (shmem > 64 * 1024)
-        AZP_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem));
+        AZP_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTpmLds));
     return AZP_OK;
     }
 
