@@ -321,11 +321,15 @@ __device__ __forceinline__ uint64_t group_pass(const GroupArgs& a,
     // |FP32 error| <= 16 2^-24 ((|a| + |b|)^2 + r^2): at most a dozen
     // roundings of partial sums no larger than that, and the rounding of the
     // offsets; |a|, |b| <= the window's diagonal.  The direct tests' own error
-    // is far inside 1e-5 r^2.
+    // is far inside 1e-5 r^2.  A difference of two fixed-point coordinates is
+    // off by up to L / 2^32 (doubled here), which a box of 20,000 and more
+    // list radii makes the larger part.
     const float wx = (float)(X.len * G.L[0] / X.n), wy = (float)(Y.len * G.L[1] / Y.n),
                 wz = (float)(Z.len * G.L[2] / Z.n);
     const float diag2 = wx * wx + wy * wy + wz * wz;
-    const float band = 1e-5f * a.thr + (direct ? 0.0f : 9.5367e-7f * (4.0f * diag2 + a.thr));
+    const float off_by = 2.0f * sqrtf(sx * sx + sy * sy + sz * sz);
+    const float band = 1e-5f * a.thr + off_by * (2.0f * a.r_max + off_by)
+                       + (direct ? 0.0f : 9.5367e-7f * (4.0f * diag2 + a.thr));
 
     const float asq = ax * ax + ay * ay + az * az;
     const bool listed = in && (uint32_t)me.fixed.w < a.ntypes;

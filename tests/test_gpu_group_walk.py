@@ -97,3 +97,33 @@ def test_group_walk_list_radii(types):
     rc[0, types - 1] = rc[types - 1, 0] = 0.0
     L = 4.2 * RL
     _check([(L, L, L), (2.1 * RL, 1.5 * L, L), (2.5 * L, L, L)], [500, 200, 900], rc, 6)
+
+
+@pytest.mark.parametrize("types", [1, 11])
+@pytest.mark.parametrize("edge", [2.2, 3.3])
+def test_group_walk_elongated_boxes(edge, types):
+    """Boxes 10,000 to 1,000,000 list radii long hold pairs at the list radius
+    give or take 1e-7 to 1e-3: a fixed-point step is up to 2e-4 list radii."""
+    rng = np.random.default_rng(17 + types)
+    rc = np.full((types, types), RC)
+    if types > 1:
+        rc[1, 1] = 0.7 * RC  # several radii among more than eight types: direct tests
+    boxes, pos4 = [], []
+    for length in (1e4, 1e5, 1e6):
+        box = np.array([edge * RL, edge * RL, length * RL])
+        n = 400
+        a = (rng.random((n, 3)) - 0.5) * box
+        a[:, 2] = (np.arange(n) + 0.5 - n / 2) * box[2] / n
+        d = rng.normal(size=(n, 3)) * [0.3, 0.3, 1.0]
+        d /= np.linalg.norm(d, axis=1)[:, None]
+        far = 1.0 + rng.choice([-1.0, 1.0], n) * 10.0 ** rng.uniform(-7, -3, n)
+        p = np.concatenate([a, a + d * (RL * far)[:, None]])
+        p -= box * np.floor(p / box + 0.5)
+        q = np.zeros((2 * n, 4))
+        q[:, :3] = p
+        q[:, 3] = rng.integers(0, types, 2 * n)
+        boxes.append(tuple(box))
+        pos4.append(q)
+    got = _batch_lists(boxes, pos4, rc)
+    for r, (box, p) in enumerate(zip(boxes, pos4)):
+        assert np.array_equal(got[r], _oracle_pairs(box, p, rc)), f"replica {r}"
