@@ -59,7 +59,7 @@ struct GroupArgs
     const double* r_listsq;
     uint32_t ntypes;
     float thr;    // largest r_list^2
-    float r_max;  // largest r_list
+    double r_max; // largest r_list
     bool direct;  // no matrix tests (several list radii among more types than ONEHOT serves)
     };
 
@@ -229,12 +229,14 @@ __device__ __forceinline__ uint64_t group_pass(const GroupArgs& a,
         return __builtin_amdgcn_readfirstlane((int)(uint32_t)(unsigned long long)(long long)(f * 4294967296.0));
     };
     const int fx0 = middle(0), fy0 = middle(1), fz0 = middle(2);
-    const float ax = (float)fixed_delta(me.fixed.x, fx0) * sx;
-    const float ay = (float)fixed_delta(me.fixed.y, fy0) * sy;
-    const float az = (float)fixed_delta(me.fixed.z, fz0) * sz;
-    const bool far = !(fabsf(ax) + a.r_max < 0.500001f * (float)G.L[0] && fabsf(ay) + a.r_max < 0.500001f * (float)G.L[1]
-                       && fabsf(az) + a.r_max < 0.500001f * (float)G.L[2])
-                     || G.n[0] < 3 || G.n[1] < 3 || G.n[2] < 3;
+    const int dx0 = fixed_delta(me.fixed.x, fx0), dy0 = fixed_delta(me.fixed.y, fy0), dz0 = fixed_delta(me.fixed.z, fz0);
+    const float ax = (float)dx0 * sx, ay = (float)dy0 * sy, az = (float)dz0 * sz;
+    // in whole steps, less the particle's and a candidate's roundings
+    auto beyond = [&](int k, int d) {
+        const double room = 2147483646.0 - a.r_max * G.Linv[k] * 4294967296.0;
+        return !(fabs((double)d) <= room);
+    };
+    const bool far = beyond(0, dx0) || beyond(1, dy0) || beyond(2, dz0) || G.n[0] < 3 || G.n[1] < 3 || G.n[2] < 3;
     const bool direct = a.direct || __ballot(in && far && (uint32_t)me.fixed.w < a.ntypes) != 0ull;
     direct_used = direct_used || direct;
     const GroupAxis X(G.n[0], anchor[0], lo[0], hi[0]);
@@ -328,7 +330,7 @@ __device__ __forceinline__ uint64_t group_pass(const GroupArgs& a,
                 wz = (float)(Z.len * G.L[2] / Z.n);
     const float diag2 = wx * wx + wy * wy + wz * wz;
     const float off_by = 2.0f * sqrtf(sx * sx + sy * sy + sz * sz);
-    const float band = 1e-5f * a.thr + off_by * (2.0f * a.r_max + off_by)
+    const float band = 1e-5f * a.thr + off_by * (2.0f * (float)a.r_max + off_by)
                        + (direct ? 0.0f : 9.5367e-7f * (4.0f * diag2 + a.thr));
 
     const float asq = ax * ax + ay * ay + az * az;

@@ -987,7 +987,7 @@ void enqueue_rebuild(azp_batch* b, hipStream_t s)
     wa.g.cell_fixed = b->cell_fixed.ptr;
     wa.g.r_listsq = b->d_rlistsq.ptr;
     wa.g.ntypes = b->ntypes;
-    wa.g.r_max = (float)b->r_list_max();
+    wa.g.r_max = b->r_list_max();
     wa.g.thr = (float)(b->r_list_max() * b->r_list_max());
     wa.N = N;
     wa.rep_of = b->rep_of.ptr;

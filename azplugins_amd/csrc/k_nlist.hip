@@ -595,7 +595,7 @@ static int nlist_build(azp_nlist* nl, const azp_particles* p, hipStream_t s)
             ta.g.cell_fixed = nl->cell_fixed.ptr;
             ta.g.r_listsq = nl->r_listsq.ptr;
             ta.g.ntypes = nl->ntypes;
-            ta.g.r_max = (float)rmax;
+            ta.g.r_max = rmax;
             ta.g.thr = (float)(rmax * rmax);
             ta.g.direct = false;
             ta.N = N;

@@ -127,3 +127,28 @@ def test_group_walk_elongated_boxes(edge, types):
     got = _batch_lists(boxes, pos4, rc)
     for r, (box, p) in enumerate(zip(boxes, pos4)):
         assert np.array_equal(got[r], _oracle_pairs(box, p, rc)), f"replica {r}"
+
+
+def test_group_walk_reach_of_half_a_box():
+    """Six cells that fit the box to 1e-9: a particle on the far face of its
+    pass's cells and a neighbor at the list radius lie half a box from the
+    pass's middle to within one fixed-point step."""
+    L = 6.0 * RL * (1.0 + 1e-9) * (1.0 + 1e-12)
+    assert int(L / (RL * (1.0 + 1e-9))) == 6
+    rng = np.random.default_rng(1)
+    pos4 = []
+    for axis in range(3):
+        for flip in (1.0, -1.0):
+            # cells 2, 3, 4 and 5 of one row; the middle particle lies in cell 4
+            x = [0.5 * L * (1.0 - 1e-13)]
+            x.append(x[0] + RL * (1.0 - 1e-12) - L)
+            for cell, n in ((2, 10), (3, 10), (4, 30), (5, 9)):
+                x.extend(((cell + rng.uniform(0.1, 0.9, n)) / 6.0 - 0.5) * L)
+            p = np.zeros((len(x), 4))
+            p[:, :3] = L * 0.25 / 6.0
+            p[:, axis] = flip * np.array(x)
+            pos4.append(p)
+    rc = np.array([[RC]])
+    got = _batch_lists([(L, L, L)] * len(pos4), pos4, rc)
+    for r, p in enumerate(pos4):
+        assert np.array_equal(got[r], _oracle_pairs((L, L, L), p, rc)), f"replica {r}"
