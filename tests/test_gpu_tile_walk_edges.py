@@ -1,9 +1,9 @@
 """Edges of the tiled list built from matrix-core group walks.
 
-Three to eight types with unequal radii (the type pairs' radii as a one-hot
-contraction), more than eight (direct tests), boxes from two to nine cells an
-axis (reach of the group's span), and dense clusters that outgrow the first
-rooms for candidate batches and rank tables.  Each list must equal the plain
+Two to eight types with unequal radii (the type pairs' radii as a one-hot
+contraction), nine (left to the plain walk), boxes from two to nine cells an
+axis (reach of the group's span), and clusters in a wide box (whose tiles span
+too many cells: left to the plain walk).  Each list must equal the plain
 walk's, and the plain walk's pairs the oracle's.
 """
 
@@ -29,13 +29,13 @@ def _lists(sysm, nt, rc, tiled, r_buff=0.4):
     return nl
 
 
-def _check(pos4, Lv, nt, rc, fused=True):
+def _check(pos4, Lv, nt, rc, kind=1):
     sysm = GpuSystem(pos4, Lv)
     plain, tiled = _lists(sysm, nt, rc, False), _lists(sysm, nt, rc, True)
     size = tiled.get_tiles()[3]
-    say(f"[edges] N={sysm.N} types={nt} L={Lv[0]:.1f}: tile size {size}")
-    if fused:
-        assert size in (256, 512)
+    say(f"[edges] N={sysm.N} types={nt} L={Lv[0]:.1f}: tile size {size}, walk {tiled.walk_kind()}")
+    assert plain.walk_kind() == 0 and tiled.walk_kind() == kind
+    assert size in (256, 512)
     got = nlist_pairs(tiled, sysm.N)
     assert got == nlist_pairs(plain, sysm.N)
     pairs = oracle.nlist(pos4, Lv, nt, oracle.r_listsq_matrix(rc, 0.4), "cell")
@@ -47,7 +47,7 @@ def test_unequal_radii(nt):
     pos4, rng = jittered_lattice(15, 16.0, 0.2, nt, seed=nt)
     rc = rng.uniform(0.8, 2.6, size=(nt, nt))
     rc = np.maximum(rc, rc.T)
-    _check(pos4, np.full(3, 16.0), nt, rc.ravel())
+    _check(pos4, np.full(3, 16.0), nt, rc.ravel(), 1 if nt <= 8 else 0)
 
 
 @pytest.mark.parametrize("cells", [2, 3, 4, 5, 6, 7, 9])
@@ -67,4 +67,4 @@ def test_dense_clusters(per):
     p -= L * np.floor(p / L + 0.5)
     pos4 = np.zeros((p.shape[0], 4))
     pos4[:, :3] = p
-    _check(pos4, np.full(3, L), 1, [1.2], fused=False)
+    _check(pos4, np.full(3, L), 1, [1.2], kind=0)
