@@ -399,7 +399,6 @@ struct azp_nlist
     DeviceArray<double4> last_pos;
     DeviceArray<uint32_t> cell_of, slot_of, count, start, members, scan_sums;
     DeviceArray<uint32_t> cell_rank; // Morton rank of each cell of the grid below
-    DeviceArray<uint32_t> rank_cell; // its inverse
     int rank_grid[3] = {0, 0, 0};
     DeviceArray<uint32_t> flags; // [1] rebuild, [kFlagStep] the step kernel's check, the others as in tiles.h
     uint32_t* h_flags = nullptr;  // pinned, kHostFlags words ([4], [5] tile build flags)
@@ -496,15 +495,11 @@ static int nlist_build(azp_nlist* nl, const azp_particles* p, hipStream_t s)
 
     if (g.n[0] != nl->rank_grid[0] || g.n[1] != nl->rank_grid[1] || g.n[2] != nl->rank_grid[2])
         {
-        std::vector<uint32_t> rank, inv(ncell);
+        std::vector<uint32_t> rank;
         morton_cell_rank(g, rank);
-        for (size_t k = 0; k < ncell; ++k)
-            inv[rank[k]] = (uint32_t)k;
         AZP_TRY(nl->cell_rank.reserve(ncell));
-        AZP_TRY(nl->rank_cell.reserve(ncell));
         AZP_HIP(hipMemcpyAsync(nl->cell_rank.ptr, rank.data(), ncell * sizeof(uint32_t), hipMemcpyHostToDevice, s));
-        AZP_HIP(hipMemcpyAsync(nl->rank_cell.ptr, inv.data(), ncell * sizeof(uint32_t), hipMemcpyHostToDevice, s));
-        AZP_HIP(hipStreamSynchronize(s)); // the host vectors go out of scope
+        AZP_HIP(hipStreamSynchronize(s)); // the host vector goes out of scope
         for (int k = 0; k < 3; ++k)
             nl->rank_grid[k] = g.n[k];
         nl->span = 0;
