@@ -39,8 +39,8 @@ FP64_BYTES_PER_PARTICLE = 124
 # non-packed VALU issue: 256 CUs x 4 SIMDs x 16 lanes x 2.4 GHz
 VALU_PEAK_LANE_OPS = 256 * 4 * 16 * 2.4e9
 # the headline kernel as rocprofv3 names it: PerturbedLJ, mixed, virial, one
-# type, no xplor, cubic box, tiled list, FP32 partial sums
-HEADLINE_KERNEL = ("void azp::k_pair<azp::EvalPerturbedLJ, true, true, true, false, true, 1, false>"
+# type, no xplor, cubic box, tiled list, FP32 partial sums, one lane a particle
+HEADLINE_KERNEL = ("void azp::k_pair<azp::EvalPerturbedLJ, true, true, true, false, true, 1, false, false>"
                    "(azp::PairKernelArgs)")
 # the sources each counter summary's kernels are compiled from: a summary
 # measured on other sources is not reported
@@ -510,7 +510,8 @@ def bench_dpd(args):
     entries = int(nn.sum())
     # pos 32 + n_neigh 4 + head 8 + force 32 + virial 48 + vel 32 + tag 4 per particle, 4 per list entry
     nbytes = N * 160 + 4 * entries
-    kernel = "void azp::k_dpd_tiled<true>(azp::DPDKernelArgs)" if tiles[3] else "void azp::k_dpd<true, true>(azp::DPDKernelArgs)"
+    kernel = ("void azp::k_dpd_tiled<true, false>(azp::DPDKernelArgs)" if tiles[3]
+              else "void azp::k_dpd<true, true, false>(azp::DPDKernelArgs)")
     res = {"value": pairs / t, "unit": "pair interactions/s", "ms_per_eval": t * 1e3, "N": N,
            "pairs_in_cut": pairs, "nlist_entries": entries, "precision": "fp64",
            "list": "tiled" if tiles[3] else "column", "tile_size": tiles[3], "tile_slots": tiles[4],
@@ -855,6 +856,7 @@ def load_counters(fname, kernel):
         return None
     k = d.get("kernels", {}).get(kernel)
     if k is None:
+        log(f"bench: profiles/{fname} holds no counters of {kernel}")
         return None
     return {"traffic_bytes": k.get("traffic_bytes"), "insts_valu": k.get("SQ_INSTS_VALU"),
             "provenance": f"profiles/{fname}, kernel sources {src}"}
