@@ -148,7 +148,8 @@ template<int ONEHOT> __global__ void __launch_bounds__(64 * kGroupWaves, 4) k_gr
     uint32_t four_low = 0, four_high = 0; // the last of them, the newest in the high bits
     bool room = true, direct = false;
     uint2* cells = a.group_cells + (size_t)group * a.group_cell_cap;
-    uint32_t* used = a.group_used + (size_t)group * a.group_batch_cap * 2u;
+    uint32_t* const group_used = reinterpret_cast<uint32_t*>(a.group_used + (size_t)group * a.group_batch_cap);
+    uint32_t* used = group_used;
     uint16_t* row = a.group_rows + (size_t)me.slot * a.max_neighbors;
     // one entry per lane and step until no lane's ring holds more than `keep`
     // words
@@ -183,7 +184,7 @@ template<int ONEHOT> __global__ void __launch_bounds__(64 * kGroupWaves, 4) k_gr
                 const uint32_t next = k + 1 < n ? s_group[w].first[k + 1] : total;
                 cells[ncell + k] = make_uint2(s_group[w].delta[k] + first, (first + nbatch * 64u) | ((next - first) << 16));
                 }
-        used = a.group_used + ((size_t)group * a.group_batch_cap + nbatch) * 2u;
+        used = group_used + nbatch * 2u;
         from = nbatch * 64u;
         ncell += n;
         nbatch += batches;
@@ -464,7 +465,7 @@ template<uint32_t T> __global__ void __launch_bounds__(T, T == 512 ? 4 : 2) k_ti
     {
     const uint32_t g = min(wave, ng - 1u);
     const uint32_t n = wave < ng ? 2u * s_nb[g] : 0u;
-    const uint32_t* src = a.group_used + (size_t)(g0 + g) * a.group_batch_cap * 2u;
+    const uint32_t* src = reinterpret_cast<const uint32_t*>(a.group_used + (size_t)(g0 + g) * a.group_batch_cap);
     for (uint32_t q0 = 0; q0 < n; q0 += 64u)
         {
         const uint32_t mine = q0 + lane < n ? src[q0 + lane] : 0u;
@@ -659,10 +660,11 @@ static TileWalkArgs tile_args(const TileList& t, const TileWalkArgs& args)
     a.tile_count = t.count.ptr;
     a.tile_jset = t.jset.ptr;
     a.tlist = t.list.ptr;
-    a.group_cells = t.group_cells.ptr;
+    const size_t groups = ((size_t)args.N + 63) / 64;
+    a.group_meta = t.groups.ptr;
+    a.group_used = a.group_meta + groups;
+    a.group_cells = a.group_used + groups * args.group_batch_cap;
     a.group_rows = t.group_rows.ptr;
-    a.group_used = t.group_used.ptr;
-    a.group_meta = t.group_meta.ptr;
     return a;
     }
 
@@ -671,10 +673,8 @@ int tiles_rows(TileList& t, const TileWalkArgs& args, bool uniform, hipStream_t 
     if (args.g.ntypes == 0 || args.g.ntypes > kTileWalkMaxTypes)
         return set_error(AZP_ERR_UNSUPPORTED, "the per-tile walk serves 1 to %u particle types", kTileWalkMaxTypes);
     const size_t groups = ((size_t)args.N + 63) / 64;
-    AZP_TRY(t.group_cells.reserve(groups * args.group_cell_cap));
+    AZP_TRY(t.groups.reserve(groups * (1 + (size_t)args.group_batch_cap + args.group_cell_cap)));
     AZP_TRY(t.group_rows.reserve((size_t)args.N * args.max_neighbors));
-    AZP_TRY(t.group_used.reserve(groups * args.group_batch_cap * 2));
-    AZP_TRY(t.group_meta.reserve(groups));
     const TileWalkArgs a = tile_args(t, args);
     const dim3 grid(grid_for(groups, kGroupWaves)), block(64 * kGroupWaves);
     if (uniform)

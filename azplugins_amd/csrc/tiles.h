@@ -39,11 +39,10 @@ struct TileList
     DeviceArray<uint32_t> nn;        // per-tile walk: list length of column s
     DeviceArray<uint32_t> order_buf; // per-tile walk: particle of column s
     DeviceArray<uint32_t> col;       // per-tile walk: column of particle i
-    // per-tile walk, by group of 64 slots: its cells, how many they are, the
-    // candidates that any of its particles lists, the particles' rows
-    DeviceArray<uint2> group_cells, group_meta;
-    DeviceArray<uint32_t> group_used;
-    DeviceArray<uint16_t> group_rows;
+    // per-tile walk, by group of 64 slots, in one allocation: how many cells
+    // and batches, the candidates that any of its particles lists, its cells
+    DeviceArray<uint2> groups;
+    DeviceArray<uint16_t> group_rows; // the particles' rows
     // Tiles of the per-tile walk: a tile's columns are its cell-list slots
     // reordered by list length (longest first); column s belongs to particle
     // order[s] and has nn[s] entries.  Null for tiles of consecutive
@@ -112,7 +111,7 @@ struct TileWalkArgs
     uint32_t sizes; // kTileSpan512 | kTileSpan256: the tile sizes that this build may use
     // set by tiles_rows / tiles_compact
     uint2* group_cells;    // by group: first slot, first candidate | members << 16 of each cell
-    uint32_t* group_used;  // by group and batch of 64 candidates: two words
+    uint2* group_used;     // by group and batch of 64 candidates
     uint16_t* group_rows;  // by slot: the candidate numbers of its entries
     uint2* group_meta;     // by group: cells, batches (high bit: direct tests)
     uint32_t* tile_nn;     // by column
