@@ -40,8 +40,8 @@ namespace azp
 //   AnisoFp64 rounds of 2^16 lanes (one wavefront a SIMD at a time bound by
 //             FP64 issue): 90,000 80 / 66, 100,000 81 / 85, 140,000 113 / 104,
 //             180,000 115 / 122, 228,000 149 / 139.
-//   Colloid   three divergent branches fill twice as many lanes: 73,000
-//             200 -> 118, 20,000 56 / 51 with 2^18 / 2^19 lanes.
+//   Colloid   three divergent branches fill twice as many lanes: 50,000 87 with
+//             2^18, 80 with 2^19; 73,000 200 -> 116.
 enum class SplitTerm
     {
     Pair,
