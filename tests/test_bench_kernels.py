@@ -1,6 +1,7 @@
 """The kernels that bench.py looks up in the counter summaries exist under
-those names in the library built here."""
+those names in the library built here, and the committed summaries hold them."""
 
+import json
 import os
 import re
 import shutil
@@ -30,3 +31,12 @@ def test_kernel_names_are_in_the_library():
     assert len(names) >= 4
     for name in names:
         assert name in symbols, name
+
+
+def test_summaries_hold_the_kernels():
+    held = set()
+    for fname in bench.KERNEL_SOURCES:
+        with open(os.path.join(ROOT, "profiles", fname)) as fh:
+            held |= set(json.load(fh)["kernels"])
+    for name in _names():
+        assert name in held, name
