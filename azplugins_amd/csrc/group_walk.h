@@ -46,8 +46,26 @@ struct GroupGeom
     int n[3];
     double L[3], Linv[3];
     float scale[3]; // L / 2^32
+    int reach[3];   // group_reach
+    float slip;     // group_slip
     uint32_t cell_base;
     };
+
+// How far a particle may lie from the middle of its pass's cells, in fixed-point
+// steps, for its neighbors to stay within half a box of it: less the particle's
+// and the neighbor's roundings.
+inline int group_reach(double L, double r_max)
+    {
+    return (int)std::max(0.0, std::floor(2147483646.0 - r_max / L * 4294967296.0));
+    }
+
+// Error of r^2 near r_max^2 from the positions' fixed-point steps: a difference
+// of two coordinates is off by up to L / 2^32, doubled here.
+inline float group_slip(const double L[3], double r_max)
+    {
+    const double off = 2.0 * std::sqrt(L[0] * L[0] + L[1] * L[1] + L[2] * L[2]) / 4294967296.0;
+    return (float)(off * (2.0 * r_max + off));
+    }
 
 struct GroupArgs
     {
@@ -59,7 +77,6 @@ struct GroupArgs
     const double* r_listsq;
     uint32_t ntypes;
     float thr;    // largest r_list^2
-    double r_max; // largest r_list
     bool direct;  // no matrix tests (several list radii among more types than ONEHOT serves)
     };
 
@@ -231,12 +248,9 @@ __device__ __forceinline__ uint64_t group_pass(const GroupArgs& a,
     const int fx0 = middle(0), fy0 = middle(1), fz0 = middle(2);
     const int dx0 = fixed_delta(me.fixed.x, fx0), dy0 = fixed_delta(me.fixed.y, fy0), dz0 = fixed_delta(me.fixed.z, fz0);
     const float ax = (float)dx0 * sx, ay = (float)dy0 * sy, az = (float)dz0 * sz;
-    // in whole steps, less the particle's and a candidate's roundings
-    auto beyond = [&](int k, int d) {
-        const double room = 2147483646.0 - a.r_max * G.Linv[k] * 4294967296.0;
-        return !(fabs((double)d) <= room);
-    };
-    const bool far = beyond(0, dx0) || beyond(1, dy0) || beyond(2, dz0) || G.n[0] < 3 || G.n[1] < 3 || G.n[2] < 3;
+    auto beyond = [](int d, int reach) { return (uint32_t)d + (uint32_t)reach > 2u * (uint32_t)reach; };
+    const bool far = beyond(dx0, G.reach[0]) || beyond(dy0, G.reach[1]) || beyond(dz0, G.reach[2]) || G.n[0] < 3
+                     || G.n[1] < 3 || G.n[2] < 3;
     const bool direct = a.direct || __ballot(in && far && (uint32_t)me.fixed.w < a.ntypes) != 0ull;
     direct_used = direct_used || direct;
     const GroupAxis X(G.n[0], anchor[0], lo[0], hi[0]);
@@ -323,15 +337,12 @@ __device__ __forceinline__ uint64_t group_pass(const GroupArgs& a,
     // |FP32 error| <= 16 2^-24 ((|a| + |b|)^2 + r^2): at most a dozen
     // roundings of partial sums no larger than that, and the rounding of the
     // offsets; |a|, |b| <= the window's diagonal.  The direct tests' own error
-    // is far inside 1e-5 r^2.  A difference of two fixed-point coordinates is
-    // off by up to L / 2^32 (doubled here), which a box of 20,000 and more
-    // list radii makes the larger part.
+    // is far inside 1e-5 r^2.  The fixed-point steps' part is the larger one in
+    // a box of 20,000 and more list radii.
     const float wx = (float)(X.len * G.L[0] / X.n), wy = (float)(Y.len * G.L[1] / Y.n),
                 wz = (float)(Z.len * G.L[2] / Z.n);
     const float diag2 = wx * wx + wy * wy + wz * wz;
-    const float off_by = 2.0f * sqrtf(sx * sx + sy * sy + sz * sz);
-    const float band = 1e-5f * a.thr + off_by * (2.0f * (float)a.r_max + off_by)
-                       + (direct ? 0.0f : 9.5367e-7f * (4.0f * diag2 + a.thr));
+    const float band = 1e-5f * a.thr + G.slip + (direct ? 0.0f : 9.5367e-7f * (4.0f * diag2 + a.thr));
 
     const float asq = ax * ax + ay * ay + az * az;
     const bool listed = in && (uint32_t)me.fixed.w < a.ntypes;

@@ -40,6 +40,8 @@ struct RepInfo
     double L[3];
     double Linv[3];
     float fx_scale[3];
+    float slip;         // group_slip
+    int reach[3];       // group_reach
     int n[3];           // cell grid
     uint32_t cell_base; // first global cell
     uint32_t first;     // first particle
@@ -315,7 +317,9 @@ template<int ONEHOT> __global__ void __launch_bounds__(64 * kWalkWaves, 3) k_b_w
             G.L[k] = R.L[k];
             G.Linv[k] = R.Linv[k];
             G.scale[k] = R.fx_scale[k];
+            G.reach[k] = R.reach[k];
             }
+        G.slip = R.slip;
         G.cell_base = R.cell_base;
         todo &= ~group_pass<ONEHOT, true>(a.g, G, s_group[w], me, todo, al, rep == r0, direct, begin, emit);
         }
@@ -867,8 +871,10 @@ int batch_upload_tables(azp_batch* b, hipStream_t s)
             ri.L[k] = L[k];
             ri.Linv[k] = 1.0 / L[k];
             ri.fx_scale[k] = (float)(L[k] / 4294967296.0);
+            ri.reach[k] = group_reach(L[k], rmax);
             ri.n[k] = g.n[k];
             }
+        ri.slip = group_slip(L, rmax);
         ri.cell_base = cells;
         ri.first = b->offsets[r];
         ri.count = n_r;
@@ -987,7 +993,6 @@ void enqueue_rebuild(azp_batch* b, hipStream_t s)
     wa.g.cell_fixed = b->cell_fixed.ptr;
     wa.g.r_listsq = b->d_rlistsq.ptr;
     wa.g.ntypes = b->ntypes;
-    wa.g.r_max = b->r_list_max();
     wa.g.thr = (float)(b->r_list_max() * b->r_list_max());
     wa.N = N;
     wa.rep_of = b->rep_of.ptr;

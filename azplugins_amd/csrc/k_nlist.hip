@@ -590,13 +590,16 @@ static int nlist_build(azp_nlist* nl, const azp_particles* p, hipStream_t s)
             ta.g.cell_fixed = nl->cell_fixed.ptr;
             ta.g.r_listsq = nl->r_listsq.ptr;
             ta.g.ntypes = nl->ntypes;
-            ta.g.r_max = rmax;
             ta.g.thr = (float)(rmax * rmax);
             ta.g.direct = false;
             ta.N = N;
             ta.box = box;
             for (int k = 0; k < 3; ++k)
+                {
                 ta.fx_scale[k] = (float)(box.L[k] / 4294967296.0);
+                ta.reach[k] = group_reach(L[k], rmax);
+                }
+            ta.slip = group_slip(L, rmax);
             ta.grid = g;
             ta.cell_of = nl->cell_of.ptr;
             ta.n_neigh = nl->n_neigh.ptr;

@@ -113,9 +113,9 @@ template<int ONEHOT> __global__ void __launch_bounds__(64 * kGroupWaves, 4) k_gr
     __shared__ uint16_t s_first[kGroupWaves][kRowBuffer * 64];
     const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     const uint32_t group = xcd_logical_block() * kGroupWaves + w;
-    // the whole wavefront leaves (no barrier below spans wavefronts)
-    if (group * 64u >= a.N || (a.flags[kTileFlagSpan] & a.sizes) == a.sizes)
-        return;
+    if (group * 64u >= a.N)
+        return; // the whole wavefront (no barrier below spans wavefronts)
+    const uint32_t span = a.flags[kTileFlagSpan];
     GroupColumn me;
     me.slot = group * 64u + lane;
     me.valid = me.slot < a.N;
@@ -129,12 +129,16 @@ template<int ONEHOT> __global__ void __launch_bounds__(64 * kGroupWaves, 4) k_gr
         G.L[k] = a.box.L[k];
         G.Linv[k] = a.box.Linv[k];
         G.scale[k] = a.fx_scale[k];
+        G.reach[k] = a.reach[k];
         }
+    G.slip = a.slip;
     G.cell_base = 0u;
     me.c[0] = (int)(me.cell % (uint32_t)G.n[0]);
     me.c[1] = (int)((me.cell / (uint32_t)G.n[0]) % (uint32_t)G.n[1]);
     me.c[2] = (int)(me.cell / ((uint32_t)G.n[0] * (uint32_t)G.n[1]));
     me.fixed = a.g.cell_fixed[me.valid ? me.slot : 0u];
+    if ((span & a.sizes) == a.sizes)
+        return; // no tile size fits (tested here, behind the loads above)
     if (me.valid && (uint32_t)me.fixed.w >= a.g.ntypes)
         {
         const double4 p = a.g.pos[me.i];
@@ -261,8 +265,7 @@ template<uint32_t T> __global__ void __launch_bounds__(T, T == 512 ? 4 : 2) k_ti
     uint16_t* s_val = reinterpret_cast<uint16_t*>(s_hash + kCellHash);
     uint16_t* s_table = reinterpret_cast<uint16_t*>(s_ucell);
 
-    if (a.flags[kTileFlagSpan] & (T == 512u ? kTileSpan512 : kTileSpan256))
-        return; // a tile of this size spans too many cells: the host sees the flag
+    const uint32_t span = a.flags[kTileFlagSpan];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t t = xcd_logical_block();
     const uint32_t slot = t * T + tid;
@@ -270,8 +273,12 @@ template<uint32_t T> __global__ void __launch_bounds__(T, T == 512 ? 4 : 2) k_ti
     const uint32_t g0 = t * G, ng = min(G, (a.N + 63u) / 64u - g0);
     const uint32_t i = active ? a.g.members[slot] : 0u;
 
+    // most tiles' candidates; the places after them are cleared where needed
+    constexpr uint32_t kMarks = 12u * 512u;
     for (uint32_t k = tid; k < kCellHash; k += T)
         s_key[k] = 0xffffffffu;
+    for (uint32_t k = tid; k < kMarks; k += T)
+        s_mark[k] = 0u;
     if (tid == 0)
         s_n = s_bad = s_direct = 0u;
     __syncthreads();
@@ -283,6 +290,8 @@ template<uint32_t T> __global__ void __launch_bounds__(T, T == 512 ? 4 : 2) k_ti
         if (m.y & 0x80000000u)
             s_direct = 1u;
         }
+    if (span & (T == 512u ? kTileSpan512 : kTileSpan256))
+        return; // a tile of this size spans too many cells: the host sees the flag
     __syncthreads();
     if (tid == 0)
         {
@@ -432,11 +441,9 @@ template<uint32_t T> __global__ void __launch_bounds__(T, T == 512 ? 4 : 2) k_ti
         }
     if (tid == 0)
         s_off[U] = (uint16_t)Mc;
-    // the marks that the scan reads (places that no cell fills point at the
-    // last one)
-    const uint32_t marks = Mc <= 12u * 512u ? 12u * 512u : C;
-    for (uint32_t k = tid; k < marks; k += T)
-        s_mark[k] = 0u;
+    if (Mc > kMarks)
+        for (uint32_t k = kMarks + tid; k < C; k += T)
+            s_mark[k] = 0u;
     __syncthreads();
 
     // 4. each group's candidates by tile candidate number: a wavefront a
@@ -516,8 +523,8 @@ template<uint32_t T> __global__ void __launch_bounds__(T, T == 512 ? 4 : 2) k_ti
                 }
             }
     };
-    if (marks < C)
-        rank(std::integral_constant<uint32_t, 12u * 512u / T>{});
+    if (Mc <= kMarks)
+        rank(std::integral_constant<uint32_t, kMarks / T>{});
     else
         rank(std::integral_constant<uint32_t, C / T>{});
     if (M > kTileCap - 1)

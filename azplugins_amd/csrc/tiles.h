@@ -101,6 +101,8 @@ struct TileWalkArgs
     uint32_t N;
     DevBox box;
     float fx_scale[3]; // L / 2^32 per axis
+    int reach[3];      // group_reach per axis
+    float slip;        // group_slip
     CellGrid grid;
     const uint32_t* cell_of; // geometric cell of each particle
     uint32_t* n_neigh;       // by particle
