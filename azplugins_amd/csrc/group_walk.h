@@ -349,7 +349,8 @@ __device__ __forceinline__ uint64_t group_pass(const GroupArgs& a,
     // a result is |a - b|^2 - r^2 - band: negative for every pair that may be
     // listed, and above -2 band (in the integer order of negative floats:
     // below `near_bits`) where FP32 does not decide
-    const float c0 = !listed ? 1e30f : (ONEHOT == 0 ? asq - a.thr : asq) - band;
+    // (the direct tests' differences are the pair's own: no |a|^2)
+    const float c0 = !listed ? 1e30f : (direct ? -a.thr : (ONEHOT == 0 ? asq - a.thr : asq)) - band;
     const int near_bits = __float_as_int(-2.0f * band);
     // matrix operands of columns 0..31 (lanes' values of half 0) and 32..63
     float bxy[2], bzw[2], cc[2];
@@ -492,26 +493,41 @@ __device__ __forceinline__ uint64_t group_pass(const GroupArgs& a,
                 }
             else
                 {
-                for (uint64_t m = served; m != 0ull; m &= m - 1ull)
-                    {
-                    const int q = __builtin_ctzll(m);
-                    const uint32_t tq = (uint32_t)lane_value(me.fixed.w, q);
-                    const float x = (float)fixed_delta(c.x, lane_value(me.fixed.x, q)) * sx;
-                    const float y = (float)fixed_delta(c.y, lane_value(me.fixed.y, q)) * sy;
-                    const float z = (float)fixed_delta(c.z, lane_value(me.fixed.z, q)) * sz;
-                    const bool both = real && tq < a.ntypes;
-                    float rl = a.thr;
-                    if (ONEHOT > 0 || a.direct)
-                        rl = both ? (float)a.r_listsq[tq * a.ntypes + (uint32_t)c.w] : 0.0f;
-                    const float d = (both && rl > 0.0f) ? x * x + y * y + z * z - rl - band : 1e30f;
-                    const uint64_t hit = __ballot(d < 0.0f), maybe = __ballot(__float_as_int(d) < near_bits);
-                    if (lane == (uint32_t)q)
+                // the candidates one after the other, each against every
+                // lane's own column: 17 instructions, and 30 for a column after
+                // the other against all lanes' candidates (922 particles in two
+                // cells an axis: 100 us a walk, and 182)
+                const uint64_t ok = __ballot(real);
+                int least = 0;
+                auto half = [&](int first, float extra) {
+                    uint32_t m = 0;
+#pragma unroll 8
+                    for (int q = first + 31; q >= first; --q)
                         {
-                        low = (uint32_t)hit;
-                        high = (uint32_t)(hit >> 32);
-                        near_low = (uint32_t)maybe;
-                        near_high = (uint32_t)(maybe >> 32);
+                        float shift = c0 + extra;
+                        if (ONEHOT > 0 || a.direct)
+                            {
+                            const uint32_t tq = (uint32_t)lane_value(c.w, q);
+                            const double rl = (listed && tq < a.ntypes)
+                                                  ? a.r_listsq[(uint32_t)me.fixed.w * a.ntypes + tq]
+                                                  : 0.0;
+                            shift = rl > 0.0 ? extra - (float)rl - band : 1e30f;
+                            }
+                        const float x = (float)fixed_delta(lane_value(c.x, q), me.fixed.x) * sx;
+                        const float y = (float)fixed_delta(lane_value(c.y, q), me.fixed.y) * sy;
+                        const float z = (float)fixed_delta(lane_value(c.z, q), me.fixed.z) * sz;
+                        const float d = __builtin_fmaf(x, x, __builtin_fmaf(y, y, __builtin_fmaf(z, z, shift)));
+                        m = __builtin_amdgcn_alignbit(m, __float_as_uint(d), 31);
+                        least = min(least, __float_as_int(d));
                         }
+                    return m & (uint32_t)(ok >> first);
+                };
+                low = half(0, 0.0f);
+                high = half(32, 0.0f);
+                if (__ballot(least < near_bits) != 0ull)
+                    {
+                    near_low = low & ~half(0, 2.0f * band);
+                    near_high = high & ~half(32, 2.0f * band);
                     }
                 }
             if (__ballot((near_low | near_high) != 0u) != 0ull)
