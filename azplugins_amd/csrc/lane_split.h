@@ -27,9 +27,11 @@ namespace azp
 //   Pair      the mixed form of one type: PerturbedLJ 90,000 31.2 / 29.4.  With
 //             several types the table reads make it issue-bound: PerturbedLJ
 //             90,000 48.2 / 53.8, Yukawa 67 / 72.
-//   Short     Hertz, lists of about ten entries: four lanes hold them all, and
-//             the chip is full at 2^17 lanes (FP64 900 particles 9.1, two lanes
-//             8.3, four 8.3, sixteen 12.1; mixed 130,000 9.2 / 10.2).
+//   Short     Hertz, lists of about ten entries, which two lanes (mixed) or four
+//             (FP64) make short enough, and the chip is full at 2^17 lanes:
+//             mixed 900 particles 6.1, two 5.8, four 6.3, sixteen 7.4; 16,000
+//             two 6.3, four 6.9; 130,000 9.2 / 10.2.  FP64 900 particles 9.1,
+//             two 8.3, four 8.3, sixteen 12.1; 16,000 two 10.4, four 8.8.
 //   PairFp64  one 512-lane workgroup a CU (LDS, registers), so the chip runs
 //             rounds of 2^17 lanes, and two lanes gain where the rounds round
 //             down: 160,000 PerturbedLJ 103 / 91, Yukawa 165 / 145; 195,000
@@ -46,6 +48,7 @@ enum class SplitTerm
     {
     Pair,
     Short,
+    ShortFp64,
     PairFp64,
     Dpd,
     Aniso,
@@ -58,10 +61,8 @@ constexpr uint32_t kSplitMax = 4;
 // log2 of the lanes per particle.
 inline uint32_t split_for(uint32_t N, SplitTerm term, uint32_t ntypes)
     {
-    const uint32_t lanes = term == SplitTerm::Colloid ? 2 * kSplitLanes
-                           : term == SplitTerm::Short ? kSplitLanes / 2
-                                                      : kSplitLanes;
-    const uint32_t most = term == SplitTerm::Short ? 2u : kSplitMax;
+    const uint32_t most = term == SplitTerm::Short ? 1u : term == SplitTerm::ShortFp64 ? 2u : kSplitMax;
+    const uint32_t lanes = term == SplitTerm::Colloid ? 2 * kSplitLanes : most < kSplitMax ? kSplitLanes / 2 : kSplitLanes;
     if (N > kSplitLanes / 4 && N <= kSplitLanes)
         {
         if (term == SplitTerm::Pair && ntypes > 1)

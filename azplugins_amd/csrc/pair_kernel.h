@@ -888,7 +888,7 @@ static int launch_t(const PairKernelArgs& ka, unsigned block, unsigned slots, hi
         return set_error(AZP_ERR_UNSUPPORTED, "too many particle types (%u) for LDS staging", ka.ntypes);
     kb.split = split_for(ka.N,
                          std::is_same_v<Eval, EvalColloid> ? SplitTerm::Colloid
-                         : std::is_same_v<Eval, EvalHertz> ? SplitTerm::Short
+                         : std::is_same_v<Eval, EvalHertz> ? (MIXED ? SplitTerm::Short : SplitTerm::ShortFp64)
                          : MIXED                           ? SplitTerm::Pair
                                                            : SplitTerm::PairFp64,
                          ka.ntypes);
